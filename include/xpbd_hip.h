@@ -317,7 +317,8 @@ int xpbd_batch_step(xpbd_batch* b, int32_t nsteps);
  * cluster kernel and the quad kernel at 64/128/256 threads per workgroup, each
  * in its full and its LDS-lean form (vertex 3's weights summed in the quad and
  * vertex bases read across lanes: more instructions, more waves per CU), each
- * with the deltas interleaved and split (XPBD_QUAD_SPLIT);
+ * with the deltas interleaved and split (XPBD_QUAD_SPLIT), and the
+ * fused-colour launches (XPBD_QUAD_TILE);
  * the patch Jacobi kernel with and without the fused one-launch iteration;
  * cluster and patch kernels each with and without the XCD-contiguous
  * workgroup mapping) as replays of a captured graph of the handle's
@@ -328,7 +329,8 @@ int xpbd_batch_step(xpbd_batch* b, int32_t nsteps);
 int xpbd_autotune(xpbd_batch* b, const char* cache_path);
 /* The kernel variant in use (XPBD_VARIANT_*); block: for CLUSTER_QUAD the
  * workgroup size (negative for the LDS-lean form; magnitude XPBD_QUAD_SPLIT +
- * size when the iterations keep the vertex deltas in their own array), for
+ * size when the iterations keep the vertex deltas in their own array;
+ * XPBD_QUAD_TILE for the fused-colour launches), for
  * PATCH 1 when the fused one-launch iteration is in use
  * (deterministic mode without attachments), else 0; xcd: whether the
  * XCD-contiguous workgroup mapping is on (block and xcd may be NULL). */
@@ -339,6 +341,12 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
  * vertices share 32-byte write sectors (same results).  Handles with
  * attachments keep the interleaved layout. */
 #define XPBD_QUAD_SPLIT 1000
+/* The quad block value of the fused-colour launches, the untuned default where
+ * the mesh's size suits them: several consecutive colours share one launch, in
+ * which a workgroup runs them on a spatial tile of the mesh (same element order;
+ * the same results up to FP32 rounding within an element).  Handles with
+ * attachments run the 256-thread quad shape instead. */
+#define XPBD_QUAD_TILE 4000
 /* Batch handles are also plain handles: xpbd_step, xpbd_destroy, ... apply. */
 
 /* ---- host-side mesh utilities (no GPU needed) ------------------------------ */

@@ -4,6 +4,7 @@
 //
 // Gauss-Seidel handles built with clusters can switch between the one-thread
 // cluster kernel and the quad kernel at 64, 128 or 256 threads per workgroup
+// and to the fused-colour launches (gs_tiles.h)
 // without rebuilding anything (same clusters, colours and order, so the same
 // results up to FP32 summation order within an element).  Patch Jacobi handles
 // time the fused one-launch iteration against the patch + shared-vertex +
@@ -69,6 +70,7 @@ void write_cache(const char* path, const std::string& key, const Candidate& c, d
 bool valid(const xpbd_handle* h, const Candidate& c)
 {
     if (c.variant == XPBD_VARIANT_CLUSTER) return h->nclusters > 0;
+    if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile) return !h->tiles.launches.empty();
     if (c.variant == XPBD_VARIANT_CLUSTER_QUAD) return h->nclusters > 0 && quad_block_supported(c.block);
     if (c.variant == XPBD_VARIANT_PATCH) return h->variant == XPBD_VARIANT_PATCH && (c.block == 0 || h->fused_ok);
     return c.variant == h->variant;
@@ -97,12 +99,14 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     if (!h) return XPBD_E_INVALID_ARG;
     const std::string key = shape_key(h);
     Candidate c{};
+    (void)ensure_gs_tiles(h);   // without a plan the other shapes are there
     if (read_cache(cache_path, key, &c) && valid(h, c)) {
         apply(h, c);
         return XPBD_OK;
     }
     std::vector<Candidate> cand;
     if (h->params.solver == XPBD_SOLVER_GS_COLORED && h->nclusters > 0) {
+        if (!h->tiles.launches.empty() && h->natt == 0) cand.push_back({ XPBD_VARIANT_CLUSTER_QUAD, kQuadTile, 1 });
         for (int x = 1; x >= 0; x--)
             for (const Candidate& b : { Candidate{ XPBD_VARIANT_CLUSTER, 0, x }, Candidate{ XPBD_VARIANT_CLUSTER_QUAD, 64, x },
                                         Candidate{ XPBD_VARIANT_CLUSTER_QUAD, 128, x },

@@ -51,6 +51,14 @@ static int dalloc(xpbd_handle* h, T** p, size_t n)
     return XPBD_OK;
 }
 
+int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes)
+{
+    char* q = nullptr;
+    int rc = dalloc(h, &q, bytes);
+    *p = q;
+    return rc;
+}
+
 static void release_graphs(xpbd_handle* h)
 {
     for (int i = 0; i < 2; i++) {
@@ -666,6 +674,11 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         xpbd_destroy(h);
         return r;
     }
+    // untuned default of Gauss-Seidel: fused-colour launches where a plan fits
+    if (P->variant == XPBD_VARIANT_AUTO && cluster) {
+        if (ensure_gs_tiles(h) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
+        h->err.clear();
+    }
     *out = h;
     return XPBD_OK;
 }
@@ -791,6 +804,53 @@ int enqueue_contacts_jacobi(xpbd_handle* h, bool first)
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "contacts_jacobi launch");
 }
 
+// The iterations by fused-colour launches (gs_tiles.h).  A launch reads its
+// group's slots and writes the next group's; a closed plan's tiles depend on
+// nothing outside them and update in place, all iterations in one launch when
+// no contacts come between them.
+static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
+{
+    hipStream_t s = h->stream;
+    const bool con = contacts_enabled(h);
+    const GsTilePlan& P = h->tiles;
+    const size_t ng = P.launches.size();
+    const bool swap = ng == 1 && !P.closed;
+    int cur = 0;   // which of the first group's two arrays, where it has two
+    hipError_t e = launch_gs_tile_load(s, h->d_pos, P.slot_vert, P.nslots, P.launches[0].nslots, P.launches[0].d[0],
+                                       P.base);
+    if (e != hipSuccess) return hip_err(h, e, "gs_tile_load launch");
+    for (int it = 0, inner; it < iters; it += inner) {
+        const bool import = it == 0 && !reset_lambda;
+        inner = P.closed && !con && !import ? iters - it : 1;
+        if (timed) timed_begin(h);
+        for (size_t g = 0; g < ng; g++) {
+            const GsTileLaunch& L = P.launches[g];
+            GsTileArgs A = L.args;
+            A.din = L.d[swap ? cur : 0];
+            A.dout = swap ? L.d[1 - cur] : P.launches[(g + 1) % ng].d[0];
+            A.niter = inner;
+            A.lam_zero = it == 0 && reset_lambda;
+            A.lam_out = it + inner == iters;
+            e = launch_gs_tile(s, A, P.shape, L.ntiles, L.threads, L.smem, import);
+            if (e != hipSuccess) return hip_err(h, e, "gs_tile launch");
+            if (swap) cur = 1 - cur;
+        }
+        if (timed) {
+            timed_end(h);
+            h->timed_iterations += inner;
+        }
+        if (con) {
+            const ContactSlots slots{ P.launches[0].d[cur], P.copy_off, P.copy };
+            e = launch_contacts_gs(s, h->d_faces, h->d_fci_off, h->nfcolors, h->ninst, h->d_cpos, h->d_clist, h->d_rest,
+                                   h->d_pos, h->d_lo, h->d_cp, h->d_cn, h->d_cb, h->d_clam, it == 0 && reset_lambda,
+                                   nullptr, nullptr, &slots);
+            if (e != hipSuccess) return hip_err(h, e, "contacts_gs launch");
+        }
+    }
+    e = launch_gs_tile_store(s, h->d_pos, P.owner, h->nv, P.launches[0].d[cur]);
+    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "gs_tile_store launch");
+}
+
 // Enqueue the solver iterations of one step (no predict / finish).  With
 // reset_lambda (the reference solve, XPBDSolver.hpp:66-77) the first iteration
 // starts every multiplier at zero; without it every multiplier (element,
@@ -856,8 +916,12 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
     // for their own array before the loop and return after it, and the bases,
     // which the loop only reads, are copied into one (the attachment pass reads
     // the records, so handles with attachments stay interleaved).
+    const bool tiled = h->variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block == kQuadTile && h->natt == 0 &&
+                       iters > 0 && !h->tiles.launches.empty();
+    if (tiled) return enqueue_tiled_iterations(h, iters, timed, reset_lambda);
+    const int quad_block = h->quad_block == kQuadTile ? 256 : h->quad_block;
     float4* dsep = h->params.solver == XPBD_SOLVER_GS_COLORED && h->variant == XPBD_VARIANT_CLUSTER_QUAD &&
-                           quad_split(h->quad_block) && h->natt == 0 && iters > 0
+                           quad_split(quad_block) && h->natt == 0 && iters > 0
                        ? h->d_dsep
                        : nullptr;
     if (dsep) {
@@ -875,7 +939,7 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
                                           h->color_off[c + 1], first, h->xcd_map);
                 else if (h->variant == XPBD_VARIANT_CLUSTER_QUAD)
                     e = launch_gs_cluster_quad(s, ta, h->d_cverts, h->d_cstart, h->d_tloc, h->d_pos,
-                                               h->color_off[c], h->color_off[c + 1], first, h->quad_block,
+                                               h->color_off[c], h->color_off[c + 1], first, quad_block,
                                                h->xcd_map, h->cluster_max_tets, dsep, dsep ? dsep + h->nv : nullptr);
                 else
                     e = launch_gs_color(s, ta, h->d_pos, h->color_off[c], h->color_off[c + 1], first);

@@ -7,12 +7,33 @@
 #include <utility>
 #include <vector>
 
+#include "gs_tile_kernels.h"
 #include "kernels.h"
 #include "mesh_tools.h"
 #include "xpbd_hip.h"
 
 namespace xpbd {
 struct Learned;
+
+// The fused-colour launches of one Gauss-Seidel iteration (gs_tiles.h).
+struct GsTileLaunch {
+    GsTileArgs args{};
+    int ntiles = 0, threads = 0, nslots = 0;
+    size_t smem = 0;
+    float4* d[2] = { nullptr, nullptr };   // in-step motion by slot; the second only where a group follows itself
+};
+struct GsTilePlan {
+    bool built = false;      // tried; launches is empty where no plan fits
+    bool closed = false;     // one launch without copies: its tiles can run all iterations
+    GsTileShape shape;
+    std::vector<GsTileLaunch> launches;
+    int nslots = 0;                      // of all launches
+    const int32_t* slot_vert = nullptr;  // slot -> vertex, launch by launch
+    float4* base = nullptr;              // by slot
+    const int32_t* owner = nullptr;      // vertex -> the owner's slot of the first group
+    const int32_t* copy_off = nullptr;   // vertex -> its slots of the first group
+    const int32_t* copy = nullptr;
+};
 }
 
 struct xpbd_handle {
@@ -40,6 +61,7 @@ struct xpbd_handle {
     std::string tuned;                         // last autotuner choice, "" if none
     std::vector<int32_t> cl_start;             // cluster variant: tet range of each cluster (solver order)
     int nclusters = 0;
+    xpbd::GsTilePlan tiles;                    // cluster variants: fused-colour launches
     xpbd::Patches patches;                     // patch variant (host copy)
     std::vector<int32_t> fperm;                // solver face position -> caller's face index
     std::vector<int32_t> fcol_off;
@@ -163,6 +185,10 @@ int enqueue_local_collision(xpbd_handle* h);
 int enqueue_contacts_jacobi(xpbd_handle* h, bool first);
 bool detect_this_step(const xpbd_handle* h);
 int run_steps(xpbd_handle* h, int32_t nsteps);
+int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes);
+// The fused-colour plan of a Gauss-Seidel handle with clusters (built once;
+// not under capture).  XPBD_OK also where no plan fits the mesh.
+int ensure_gs_tiles(xpbd_handle* h);
 void timed_begin(xpbd_handle* h);
 void timed_end(xpbd_handle* h);
 int collect_timing(xpbd_handle* h);

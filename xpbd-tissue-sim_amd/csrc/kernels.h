@@ -71,6 +71,7 @@ hipError_t launch_gs_cluster(hipStream_t s, const TetArrays& ta, const int4* cve
 // while an iteration loop runs in the split layout, else null (both in the
 // interleaved vertex records).
 constexpr int kQuadSplit = XPBD_QUAD_SPLIT;
+constexpr int kQuadTile = XPBD_QUAD_TILE;
 hipError_t launch_gs_cluster_quad(hipStream_t s, const TetArrays& ta, const int4* cverts, const int* cstart,
                                   const uint32_t* tloc, float4* pos, int cbeg, int cend, bool first, int block,
                                   bool xcd, int max_tets, float4* dsep = nullptr, const float4* dbase = nullptr);
@@ -198,10 +199,18 @@ hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int
 // Gauss-Seidel contacts: one workgroup per instance (instances share no
 // vertex), colour by colour; fci_off[c * (ninst + 1) + i] is the face position
 // where instance i's faces of colour c start.
+// The in-step motions lie in the vertex records, in arrays of their own (dsep,
+// dbase), or, with slots, in every slot that a fused-colour launch reads them from.
+struct ContactSlots {
+    float4* d;
+    const int* off;    // vertex -> its range in slot
+    const int* slot;
+};
 hipError_t launch_contacts_gs(hipStream_t s, const int4* faces, const int* fci_off, int ncol, int ninst,
                               const int* cpos, const int* clist, const double* rest, float4* pos, const float4* lo,
                               const double* cp, const double* cn, const double* cb, double* clam, bool first,
-                              float4* dsep = nullptr, const float4* dbase = nullptr);
+                              float4* dsep = nullptr, const float4* dbase = nullptr,
+                              const ContactSlots* slots = nullptr);
 hipError_t launch_contacts_jacobi(hipStream_t s, const int4* faces, int nf, const int* cpos, const int* clist,
                                   const double* rest, const float4* pos, const float4* lo, float* acc,
                                   const double* cp, const double* cn, const double* cb, double* clam, bool first);

@@ -12,6 +12,7 @@
 
 #include "kernels.h"
 #include "mesh_tools.h"
+#include "quad_ops.h"
 #include "xpbd_math.h"
 
 namespace xpbd {
@@ -41,20 +42,6 @@ __device__ __forceinline__ void gather4(const float4* __restrict__ pos, const in
         g.d[3 * i + 1] = d.y;
         g.d[3 * i + 2] = d.z;
     }
-}
-
-// Workgroups are dispatched round-robin over the 8 XCDs (workgroup b runs on
-// XCD b % 8), and each XCD has its own L2.  With remap set, workgroup b takes
-// the work item that gives every XCD one contiguous eighth of the G items:
-// neighbouring clusters or patches (adjacent in solver order) then share an L2,
-// and since every colour's clusters follow the same spatial order, a vertex
-// written in one colour launch is read in the next by the same XCD.
-constexpr int kXcds = 8;
-__device__ __forceinline__ int xcd_item(int b, int G, bool remap)
-{
-    if (!remap) return b;
-    const int q = G / kXcds, r = G % kXcds, x = b % kXcds;
-    return x * q + min(x, r) + b / kXcds;
 }
 
 __device__ __forceinline__ void load_tet(const TetArrays& ta, int e, float* q, float2& at, float& g)
@@ -302,30 +289,6 @@ __global__ __launch_bounds__(kClusterBlock) void k_gs_cluster(TetArrays ta, cons
 // lanes per colour are the point: a colour holds only ~1/8 of the clusters.
 // ---------------------------------------------------------------------------
 
-__device__ __forceinline__ float dpp_xor1(float x)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, true));
-}
-__device__ __forceinline__ float dpp_xor2(float x)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, true));
-}
-// Sum of a * b over the four lanes of a quad, (x + swap1) + swap2, the same
-// bits in all four lanes.  The product is rounded in every lane first:
-// contracted into an FMA, each lane would add its own unrounded product to its
-// partners' rounded ones, and the lanes would no longer hold the same sum.
-__device__ __forceinline__ float quad_sum_of_product(float a, float b)
-{
-#pragma clang fp contract(off)
-    const float x = a * b;
-    const float y = x + dpp_xor1(x);
-    return y + dpp_xor2(y);
-}
-__device__ __forceinline__ float quad_lane3(float x)
-{
-    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xFF, 0xF, 0xF, true));
-}
-
 // BLOCK threads per workgroup = BLOCK / 4 clusters; the launch shape is a tuning choice.
 // MT bounds the elements of a cluster: 8 in general, 6 where every cluster is
 // one hexahedral cell, which leaves a wave's element planes a quarter smaller
@@ -353,16 +316,6 @@ struct QuadLds {
 
 // The unrolled step loop covers every element of a cluster.
 static_assert(kClusterTets == 8 && kClusterVerts == 8, "cluster shape of build_clusters");
-
-// Where the in-step motion (delta) of vertex v lies: after its base in the
-// interleaved vertex record, or, while a Gauss-Seidel iteration loop runs in
-// the split layout, in its own array (dsep), where the deltas of neighbouring
-// vertices share 32-byte write sectors.
-template <bool SPLIT>
-__device__ __forceinline__ float4* delta_at(float4* pos, float4* dsep, int v)
-{
-    return SPLIT ? dsep + v : pos + 2 * (size_t)v + 1;
-}
 
 // One chunk of BLOCK / 4 consecutive clusters starting at cluster cb (clusters
 // below cend), projected by one workgroup and written back.  Each wave owns 16
@@ -1485,59 +1438,71 @@ __device__ __forceinline__ bool contact_dx(const double* const x[3], const float
 
 // One contact of the Gauss-Seidel pass: project it from the current positions
 // and apply its correction to the face's three vertices.
-template <bool SPLIT>
+// Where a contact finds and leaves the in-step motion of its vertices.
+enum { kMotionRecords = 0, kMotionSplit = 1, kMotionSlots = 2 };
+struct MotionPlace {
+    int first, more, end;   // index of the motion; further slots [more, end) of ContactSlots.slot
+};
+template <int MODE>
+__device__ __forceinline__ MotionPlace motion_place(const ContactSlots& sl, int v)
+{
+    if constexpr (MODE == kMotionSlots) {
+        const int o = sl.off[v];
+        return { sl.slot[o], o + 1, sl.off[v + 1] };
+    }
+    return { MODE == kMotionSplit ? v : 2 * v + 1, 0, 0 };
+}
+template <int MODE>
+__device__ __forceinline__ float4* motion_array(float4* pos, float4* dsep, const ContactSlots& sl)
+{
+    return MODE == kMotionSlots ? sl.d : MODE == kMotionSplit ? dsep : pos;
+}
+__device__ __forceinline__ void motion_write(float4* d, const ContactSlots& sl, const MotionPlace& p, const float4 x)
+{
+    d[p.first] = x;
+    for (int k = p.more; k < p.end; k++) d[sl.slot[k]] = x;
+}
+
+template <int MODE>
 __device__ __forceinline__ void contact_gs_one(bool first, int j, const int4* __restrict__ faces,
                                                const double* __restrict__ rest, float4* __restrict__ pos,
                                                float4* __restrict__ dsep, const float4* __restrict__ dbase,
                                                const float4* __restrict__ lo, const double* __restrict__ cp,
                                                const double* __restrict__ cn, const double* __restrict__ cb,
-                                               double* __restrict__ clam)
+                                               double* __restrict__ clam, const ContactSlots& slots)
 {
     const int4 f = faces[j];
-    double x0[3], x1[3], x2[3];
-    if constexpr (SPLIT) {
-        // world_pos with the delta read from the split array, in the same order
-        const int vv[3] = { f.x, f.y, f.z };
-        double* xx[3] = { x0, x1, x2 };
-#pragma unroll
-        for (int m = 0; m < 3; m++) {
-            const float4 b = dbase[vv[m]];
-            const float4 l = lo[vv[m]];
-            double u[3] = { (double)b.x + (double)l.x, (double)b.y + (double)l.y, (double)b.z + (double)l.z };
-            const float4 d = dsep[vv[m]];
-            u[0] += (double)d.x;
-            u[1] += (double)d.y;
-            u[2] += (double)d.z;
-#pragma unroll
-            for (int k = 0; k < 3; k++) xx[m][k] = rest[3 * (size_t)vv[m] + k] + u[k];
-        }
-    } else {
-        world_pos(rest, pos, lo, f.x, true, x0);
-        world_pos(rest, pos, lo, f.y, true, x1);
-        world_pos(rest, pos, lo, f.z, true, x2);
-    }
-    const double* xs[3] = { x0, x1, x2 };
+    const int vid[3] = { f.x, f.y, f.z };
+    float4* const md = motion_array<MODE>(pos, dsep, slots);
+    MotionPlace mp[3];
+    float4 d[3];
+    double x[3][3];
     float w[3];
-    if constexpr (SPLIT) {
-        w[0] = dbase[f.x].w;
-        w[1] = dbase[f.y].w;
-        w[2] = dbase[f.z].w;
-    } else {
-        w[0] = pos[2 * (size_t)f.x].w;
-        w[1] = pos[2 * (size_t)f.y].w;
-        w[2] = pos[2 * (size_t)f.z].w;
+#pragma unroll
+    for (int m = 0; m < 3; m++) {
+        // world_pos, in the same order, wherever the motion lies
+        mp[m] = motion_place<MODE>(slots, vid[m]);
+        const float4 b = MODE == kMotionSplit ? dbase[vid[m]] : pos[2 * (size_t)vid[m]];
+        const float4 l = lo[vid[m]];
+        d[m] = md[mp[m].first];
+        double u[3] = { (double)b.x + (double)l.x, (double)b.y + (double)l.y, (double)b.z + (double)l.z };
+        u[0] += (double)d[m].x;
+        u[1] += (double)d[m].y;
+        u[2] += (double)d[m].z;
+#pragma unroll
+        for (int k = 0; k < 3; k++) x[m][k] = rest[3 * (size_t)vid[m] + k] + u[k];
+        w[m] = b.w;
     }
+    const double* xs[3] = { x[0], x[1], x[2] };
     double lam = first ? 0.0 : clam[j];
     double dx[9];
     if (contact_dx(xs, w, cp + 3 * (size_t)j, cn + 3 * (size_t)j, cb + 3 * (size_t)j, &lam, dx)) {
-        const int vid[3] = { f.x, f.y, f.z };
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            float4 d = *delta_at<SPLIT>(pos, dsep, vid[i]);
-            d.x = (float)((double)d.x + dx[3 * i]);
-            d.y = (float)((double)d.y + dx[3 * i + 1]);
-            d.z = (float)((double)d.z + dx[3 * i + 2]);
-            *delta_at<SPLIT>(pos, dsep, vid[i]) = d;
+            d[i].x = (float)((double)d[i].x + dx[3 * i]);
+            d[i].y = (float)((double)d[i].y + dx[3 * i + 1]);
+            d[i].z = (float)((double)d[i].z + dx[3 * i + 2]);
+            motion_write(md, slots, mp[i], d[i]);
         }
     }
     clam[j] = lam;
@@ -1553,7 +1518,7 @@ __device__ __forceinline__ void contact_gs_one(bool first, int j, const int4* __
 // masses, contact point, normal, barycentrics, multiplier) is loaded once, so a
 // colour costs one round trip for the in-step motion of its vertices.  Contacts
 // past the first kBlock of an instance are loaded as they are projected.
-template <bool FIRST, bool SPLIT>
+template <bool FIRST, int MODE>
 __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__ faces,
                                                        const int* __restrict__ fci_off, int ncol, int ninst,
                                                        const int* __restrict__ cpos, const int* __restrict__ clist,
@@ -1561,8 +1526,10 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__
                                                        float4* __restrict__ dsep, const float4* __restrict__ dbase,
                                                        const float4* __restrict__ lo,
                                                        const double* __restrict__ cp, const double* __restrict__ cn,
-                                                       const double* __restrict__ cb, double* __restrict__ clam)
+                                                       const double* __restrict__ cb, double* __restrict__ clam,
+                                                       ContactSlots slots)
 {
+    float4* const md = motion_array<MODE>(pos, dsep, slots);
     __shared__ int rng[2 * kBlock];  // per colour of the chunk: the instance's range in clist
     __shared__ int loc[kBlock + 1];  // per colour: number of the instance's first contact of that colour
     const int tid = threadIdx.x, inst = blockIdx.x;
@@ -1585,7 +1552,7 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__
         __syncthreads();
         // this thread's contact: its colour (loc is non-decreasing) and fixed data
         int mc = -1, j = 0;
-        int vid[3] = { 0, 0, 0 };
+        MotionPlace mp[3];
         double xr[3][3], sbl[3][3], ccp[3], ccn[3], ccb[3], lam = 0.0;
         float w[3] = { 0.f, 0.f, 0.f };
         if (tid < loc[nc]) {
@@ -1598,12 +1565,11 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__
             mc = lo_c;
             j = clist[rng[2 * mc] + (tid - loc[mc])];
             const int4 f = faces[j];
-            vid[0] = f.x;
-            vid[1] = f.y;
-            vid[2] = f.z;
+            const int vid[3] = { f.x, f.y, f.z };
 #pragma unroll
             for (int m = 0; m < 3; m++) {
-                const float4 bv = SPLIT ? dbase[vid[m]] : pos[2 * (size_t)vid[m]];
+                mp[m] = motion_place<MODE>(slots, vid[m]);
+                const float4 bv = MODE == kMotionSplit ? dbase[vid[m]] : pos[2 * (size_t)vid[m]];
                 const float4 l = lo[vid[m]];
                 sbl[m][0] = (double)bv.x + (double)l.x;
                 sbl[m][1] = (double)bv.y + (double)l.y;
@@ -1629,7 +1595,7 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__
                 double x[3][3];
 #pragma unroll
                 for (int m = 0; m < 3; m++) {
-                    d[m] = *delta_at<SPLIT>(pos, dsep, vid[m]);
+                    d[m] = md[mp[m].first];
                     const double u[3] = { sbl[m][0] + (double)d[m].x, sbl[m][1] + (double)d[m].y,
                                           sbl[m][2] + (double)d[m].z };
 #pragma unroll
@@ -1644,14 +1610,14 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(const int4* __restrict__
                         dn.x = (float)((double)dn.x + dx[3 * m]);
                         dn.y = (float)((double)dn.y + dx[3 * m + 1]);
                         dn.z = (float)((double)dn.z + dx[3 * m + 2]);
-                        *delta_at<SPLIT>(pos, dsep, vid[m]) = dn;
+                        motion_write(md, slots, mp[m], dn);
                     }
                 }
             }
             for (int q = loc[c] + tid; q < loc[c + 1]; q += kBlock)
                 if (q >= kBlock)
-                    contact_gs_one<SPLIT>(FIRST, clist[cs + (q - loc[c])], faces, rest, pos, dsep, dbase, lo, cp, cn,
-                                          cb, clam);
+                    contact_gs_one<MODE>(FIRST, clist[cs + (q - loc[c])], faces, rest, pos, dsep, dbase, lo, cp, cn,
+                                         cb, clam, slots);
             __syncthreads();
         }
         if (mc >= 0) clam[j] = lam;
@@ -2622,23 +2588,23 @@ hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int
 hipError_t launch_contacts_gs(hipStream_t s, const int4* faces, const int* fci_off, int ncol, int ninst,
                               const int* cpos, const int* clist, const double* rest, float4* pos, const float4* lo,
                               const double* cp, const double* cn, const double* cb, double* clam, bool first,
-                              float4* dsep, const float4* dbase)
+                              float4* dsep, const float4* dbase, const ContactSlots* slots)
 {
     if (ninst <= 0 || ncol <= 0) return hipSuccess;
-    const dim3 g(ninst), b(kBlock);
-    const bool split = dsep && dbase;
-    if (first && split)
-        hipLaunchKernelGGL((k_contacts_gs<true, true>), g, b, 0, s, faces, fci_off, ncol, ninst, cpos, clist, rest, pos,
-                           dsep, dbase, lo, cp, cn, cb, clam);
-    else if (first)
-        hipLaunchKernelGGL((k_contacts_gs<true, false>), g, b, 0, s, faces, fci_off, ncol, ninst, cpos, clist, rest,
-                           pos, nullptr, nullptr, lo, cp, cn, cb, clam);
-    else if (split)
-        hipLaunchKernelGGL((k_contacts_gs<false, true>), g, b, 0, s, faces, fci_off, ncol, ninst, cpos, clist, rest,
-                           pos, dsep, dbase, lo, cp, cn, cb, clam);
-    else
-        hipLaunchKernelGGL((k_contacts_gs<false, false>), g, b, 0, s, faces, fci_off, ncol, ninst, cpos, clist, rest,
-                           pos, nullptr, nullptr, lo, cp, cn, cb, clam);
+    const ContactSlots sl = slots ? *slots : ContactSlots{ nullptr, nullptr, nullptr };
+#define XPBD_CONTACTS_LAUNCH(F, M)                                                                                    \
+    hipLaunchKernelGGL((k_contacts_gs<F, M>), dim3(ninst), dim3(kBlock), 0, s, faces, fci_off, ncol, ninst, cpos, clist, \
+                       rest, pos, dsep, dbase, lo, cp, cn, cb, clam, sl)
+    const int mode = slots ? kMotionSlots : dsep && dbase ? kMotionSplit : kMotionRecords;
+    switch (2 * mode + (first ? 1 : 0)) {
+    case 0: XPBD_CONTACTS_LAUNCH(false, kMotionRecords); break;
+    case 1: XPBD_CONTACTS_LAUNCH(true, kMotionRecords); break;
+    case 2: XPBD_CONTACTS_LAUNCH(false, kMotionSplit); break;
+    case 3: XPBD_CONTACTS_LAUNCH(true, kMotionSplit); break;
+    case 4: XPBD_CONTACTS_LAUNCH(false, kMotionSlots); break;
+    default: XPBD_CONTACTS_LAUNCH(true, kMotionSlots); break;
+    }
+#undef XPBD_CONTACTS_LAUNCH
     return hipGetLastError();
 }
 
