@@ -1051,11 +1051,8 @@ int enqueue_local_collision(xpbd_handle* h)
 int enqueue_detect(xpbd_handle* h)
 {
     hipError_t e = launch_detect(h->stream, h->d_faces, h->nf, h->d_rest, h->d_pos, h->d_lo, h->d_sdf, h->d_step,
-                                 h->params.dt, h->d_flag, h->d_cp, h->d_cn, h->d_cb);
-    if (e != hipSuccess) return hip_err(h, e, "detect launch");
-    e = launch_compact(h->stream, h->d_flag, h->nf, h->d_cpos, h->d_clist, h->d_bsum);
-    if (e != hipSuccess) return hip_err(h, e, "compact launch");
-    return XPBD_OK;
+                                 h->params.dt, h->d_flag, h->d_cpos, h->d_clist, h->d_bsum, h->d_cp, h->d_cn, h->d_cb);
+    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "detect launch");
 }
 
 int enqueue_predict(xpbd_handle* h)

@@ -189,11 +189,12 @@ hipError_t launch_element_forces(hipStream_t s, const TetArrays& ta, const Prima
 hipError_t launch_consistent_shift(hipStream_t s, float4* pos, const float4* pred, const int* vt_off,
                                    const double* ef, int nv);
 
-// Contacts.  faces: (a, b, c, instance) in colour-sorted order.
+// Contacts.  faces: (a, b, c, instance) in colour-sorted order.  Detection, then
+// the ordered compaction of its hits; bsum is scratch of compact_blocks(nf) ints.
 hipError_t launch_detect(hipStream_t s, const int4* faces, int nf, const double* rest, const float4* pos,
                          const float4* lo, const SdfDev* sdf, const unsigned long long* step, double dt, int* flag,
-                         double* cp, double* cn, double* cb);
-// Ordered compaction of hit flags; bsum is scratch of compact_blocks(nf) ints.
+                         int* cpos, int* clist, int* bsum, double* cp, double* cn, double* cb);
+// The compaction alone, of flags from elsewhere.
 int compact_blocks(int nf);
 hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int* clist, int* bsum);
 // Gauss-Seidel contacts: one workgroup per instance (instances share no

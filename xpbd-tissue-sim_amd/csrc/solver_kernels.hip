@@ -915,6 +915,11 @@ __global__ __launch_bounds__(kBlock) void k_fill_zero(uint32_t* __restrict__ p, 
 // arithmetic, so that detection from the same state takes the same branches
 // (Frank-Wolfe's vertex choice compares dot products that can tie exactly).
 #pragma clang fp contract(off)
+}  // namespace
+}  // namespace xpbd
+#include "sdf_descent.h"   // not above: it has the same pragma, which holds from there on
+namespace xpbd {
+namespace {
 // ---------------------------------------------------------------------------
 // FP64 residual / energy (XPBDSolver.hpp:327-391, XPBDMeshObject.cpp:537-549).
 // The FP32 state is promoted and the constraint maths evaluated in double.
@@ -1163,85 +1168,9 @@ __global__ __launch_bounds__(kBlock) void k_sum_squares(const double* __restrict
 }
 
 // ---------------------------------------------------------------------------
-// Signed distance fields and contact detection in FP64:
-// SphereSDF.cpp:16-26, BoxSDF.cpp:19-84, GeometryUtils.cpp:6-24,92-102,
-// CollisionScene.cpp:171-214 (face loop) and 253-283 (Frank-Wolfe).
+// Contact detection in FP64 (signed distances and the search on a face:
+// sdf_descent.h): CollisionScene.cpp:171-214 (face loop).
 // ---------------------------------------------------------------------------
-struct Pose {
-    int kind;
-    double p[3], q[4], prm[3];
-};
-
-__device__ __forceinline__ void qrot(const double* v, const double* q, double* o)
-{
-    const double uv = q[0] * v[0] + q[1] * v[1] + q[2] * v[2];
-    const double cx = q[1] * v[2] - q[2] * v[1];
-    const double cy = q[2] * v[0] - q[0] * v[2];
-    const double cz = q[0] * v[1] - q[1] * v[0];
-    const double s = 2 * q[3] * q[3] - 1;
-    o[0] = 2 * uv * q[0] + s * v[0] + 2 * q[3] * cx;
-    o[1] = 2 * uv * q[1] + s * v[1] + 2 * q[3] * cy;
-    o[2] = 2 * uv * q[2] + s * v[2] + 2 * q[3] * cz;
-}
-
-__device__ __forceinline__ void to_body(const Pose& P, const double* x, double* xb)
-{
-    const double n2 = P.q[0] * P.q[0] + P.q[1] * P.q[1] + P.q[2] * P.q[2] + P.q[3] * P.q[3];
-    const double qi[4] = { -P.q[0] / n2, -P.q[1] / n2, -P.q[2] / n2, P.q[3] / n2 };
-    const double rel[3] = { x[0] - P.p[0], x[1] - P.p[1], x[2] - P.p[2] };
-    qrot(rel, qi, xb);
-}
-
-__device__ double sdf_eval(const Pose& P, const double* x)
-{
-    if (P.kind == 1) {
-        const double d0 = x[0] - P.p[0], d1 = x[1] - P.p[1], d2 = x[2] - P.p[2];
-        return sqrt(d0 * d0 + d1 * d1 + d2 * d2) - P.prm[0];
-    }
-    double xb[3];
-    to_body(P, x, xb);
-    double q[3], qc[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        q[k] = fabs(xb[k]) - 0.5 * P.prm[k];
-        qc[k] = q[k] > 0.0 ? q[k] : 0.0;
-    }
-    const double mq = fmax(q[0], fmax(q[1], q[2]));
-    return sqrt(qc[0] * qc[0] + qc[1] * qc[1] + qc[2] * qc[2]) + (mq < 0.0 ? mq : 0.0);
-}
-
-__device__ void sdf_grad(const Pose& P, const double* x, double* g)
-{
-    if (P.kind == 1) {
-        const double d[3] = { x[0] - P.p[0], x[1] - P.p[1], x[2] - P.p[2] };
-        const double n = sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2]);
-#pragma unroll
-        for (int k = 0; k < 3; k++) g[k] = n > 0 ? d[k] / n : d[k];
-        return;
-    }
-    double xb[3];
-    to_body(P, x, xb);
-    double q[3], qc[3], sg[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        q[k] = fabs(xb[k]) - P.prm[k] / 2.0;
-        qc[k] = q[k] > 0.0 ? q[k] : 0.0;
-        sg[k] = xb[k] > 0 ? 1.0 : -1.0;
-    }
-    const double mq = fmax(q[0], fmax(q[1], q[2]));
-    const double md = mq < 0.0 ? mq : 0.0;
-    double go[3] = { sg[0] * qc[0], sg[1] * qc[1], sg[2] * qc[2] };
-    const double n = sqrt(go[0] * go[0] + go[1] * go[1] + go[2] * go[2]);
-    if (n > 0) {
-#pragma unroll
-        for (int k = 0; k < 3; k++) go[k] /= n;
-    }
-    double gb[3];
-#pragma unroll
-    for (int k = 0; k < 3; k++) gb[k] = go[k] + sg[k] * (q[k] == md ? 1.0 : 0.0);
-    qrot(gb, P.q, g);
-}
-
 // world position rest + base + low part (+ in-step motion during a solve)
 __device__ __forceinline__ void world_pos(const double* rest, const float4* pos, const float4* lo, int v,
                                           bool with_delta, double* x)
@@ -1253,162 +1182,164 @@ __device__ __forceinline__ void world_pos(const double* rest, const float4* pos,
     x[2] = rest[3 * (size_t)v + 2] + u[2];
 }
 
+__device__ __forceinline__ bool detect_face(const SdfDev& S, double t, const double* p1, const double* p2,
+                                            const double* p3, double* cp, double* cn, double* cb)
+{
+    if (S.kind == 0) return false;
+    Pose pose;
+    pose.kind = S.kind;
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        pose.p[k] = S.pos[k] + S.vel[k] * t;
+        pose.prm[k] = S.prm[k];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k++) pose.q[k] = S.quat[k];
+    const PosedSdf P(pose);
+    double e12 = 0, e13 = 0, e23 = 0, cen[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        e12 += (p2[k] - p1[k]) * (p2[k] - p1[k]);
+        e13 += (p3[k] - p1[k]) * (p3[k] - p1[k]);
+        e23 += (p3[k] - p2[k]) * (p3[k] - p2[k]);
+        cen[k] = (p1[k] + p2[k] + p3[k]) / 3;
+    }
+    const double me = fmax(e12, fmax(e13, e23));
+    const double cd = sdf_eval(P, cen);
+    if (cd * cd > me) return false;
+    // from the closest vertex
+    const double d1 = sdf_eval(P, p1), d2 = sdf_eval(P, p2), d3 = sdf_eval(P, p3);
+    const int st = (d1 <= d2 && d1 <= d3) ? 0 : ((d2 <= d1 && d2 <= d3) ? 1 : 2);
+    double x[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) x[k] = st == 0 ? p1[k] : st == 1 ? p2[k] : p3[k];
+    if (P.kind == 1) face_descent<false, true>(P, p1, p2, p3, x);
+    else face_descent<true, true>(P, p1, p2, p3, x);
+    const double dist = sdf_eval(P, x);
+    if (!(dist <= 1e-4)) return false;
+    double v0[3], v1[3], v2[3];
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        v0[k] = p2[k] - p1[k];
+        v1[k] = p3[k] - p1[k];
+        v2[k] = x[k] - p1[k];
+    }
+    const double d00 = v0[0] * v0[0] + v0[1] * v0[1] + v0[2] * v0[2];
+    const double d01 = v0[0] * v1[0] + v0[1] * v1[1] + v0[2] * v1[2];
+    const double d11 = v1[0] * v1[0] + v1[1] * v1[1] + v1[2] * v1[2];
+    const double d20 = v2[0] * v0[0] + v2[1] * v0[1] + v2[2] * v0[2];
+    const double d21 = v2[0] * v1[0] + v2[1] * v1[1] + v2[2] * v1[2];
+    const double den = d00 * d11 - d01 * d01;
+    const double bv = (d11 * d20 - d01 * d21) / den;
+    const double bw = (d00 * d21 - d01 * d20) / den;
+    double g[3];
+    sdf_grad(P, x, g);
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        cp[k] = x[k] - g[k] * dist;
+        cn[k] = g[k];
+    }
+    cb[0] = 1 - bv - bw;
+    cb[1] = bv;
+    cb[2] = bw;
+    return true;
+}
+
+// Hits of a workgroup's faces before this thread's, and in hits of all of them.
+constexpr int kWaves = kBlock / 64;
+__device__ __forceinline__ int hits_before(bool hit, int* ws, int& hits)
+{
+    const unsigned long long m = __ballot(hit);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) ws[wv] = __popcll(m);
+    __syncthreads();
+    int before = __popcll(m & ((1ull << lane) - 1ull));
+    hits = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) {
+        if (w < wv) before += ws[w];
+        hits += ws[w];
+    }
+    return before;
+}
+
+// One thread a face.  Few waves get past the distance test, so the kernel takes as
+// long as one wave's chain: 32 search steps of some 55 instructions (sphere) or 110
+// (box), each some 9 cycles after the one it needs.  With the search's quick vertex
+// choice, and all loads of a level in flight together: 12x12x12 cells and a box 36
+// -> 24 us, a tissue block and a sphere 26 -> 15.5, 48 objects and boxes 71 -> 45.
 __global__ __launch_bounds__(kBlock) void k_detect(const int4* __restrict__ faces, int nf,
                                                   const double* __restrict__ rest,
                                                   const float4* __restrict__ pos, const float4* __restrict__ lo,
                                                   const SdfDev* __restrict__ sdf,
                                                   const unsigned long long* __restrict__ step, double dt,
-                                                  int* __restrict__ flag, double* __restrict__ cp,
-                                                  double* __restrict__ cn, double* __restrict__ cb)
+                                                  int* __restrict__ flag, int* __restrict__ bsum,
+                                                  double* __restrict__ cp, double* __restrict__ cn,
+                                                  double* __restrict__ cb)
 {
+    __shared__ int ws[kWaves];
     const int j = blockIdx.x * kBlock + threadIdx.x;
-    if (j >= nf) return;
-    const int4 f = faces[j];
-    const SdfDev S = sdf[f.w];
-    int hit = 0;
-    if (S.kind != 0) {
-        Pose P;
-        P.kind = S.kind;
-        const double t = (double)step[0] * dt;
+    // face, then collider and vertices, all loads of each before their first use
+    int4 f = faces[min(j, nf - 1)];
+    double t = (double)step[0] * dt;
+    asm volatile("" : "+v"(f.x), "+v"(f.y), "+v"(f.z), "+v"(f.w));
+    SdfDev S = sdf[f.w];
+    double p1[3], p2[3], p3[3];
+    world_pos(rest, pos, lo, f.x, false, p1);
+    world_pos(rest, pos, lo, f.y, false, p2);
+    world_pos(rest, pos, lo, f.z, false, p3);
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            P.p[k] = S.pos[k] + S.vel[k] * t;
-            P.prm[k] = S.prm[k];
-        }
-#pragma unroll
-        for (int k = 0; k < 4; k++) P.q[k] = S.quat[k];
-        double p1[3], p2[3], p3[3];
-        world_pos(rest, pos, lo, f.x, false, p1);
-        world_pos(rest, pos, lo, f.y, false, p2);
-        world_pos(rest, pos, lo, f.z, false, p3);
-        double e12 = 0, e13 = 0, e23 = 0, cen[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) {
-            e12 += (p2[k] - p1[k]) * (p2[k] - p1[k]);
-            e13 += (p3[k] - p1[k]) * (p3[k] - p1[k]);
-            e23 += (p3[k] - p2[k]) * (p3[k] - p2[k]);
-            cen[k] = (p1[k] + p2[k] + p3[k]) / 3;
-        }
-        const double me = fmax(e12, fmax(e13, e23));
-        const double cd = sdf_eval(P, cen);
-        if (!(cd * cd > me)) {
-            // Frank-Wolfe, 32 steps of size 2/(i+3), started at the closest vertex
-            const double d1 = sdf_eval(P, p1), d2 = sdf_eval(P, p2), d3 = sdf_eval(P, p3);
-            double x[3];
-            const double* st = (d1 <= d2 && d1 <= d3) ? p1 : ((d2 <= d1 && d2 <= d3) ? p2 : p3);
-#pragma unroll
-            for (int k = 0; k < 3; k++) x[k] = st[k];
-            for (int it = 0; it < 32; it++) {
-                const double al = 2.0 / (it + 3);
-                double g[3];
-                sdf_grad(P, x, g);
-                const double s1 = p1[0] * g[0] + p1[1] * g[1] + p1[2] * g[2];
-                const double s2 = p2[0] * g[0] + p2[1] * g[1] + p2[2] * g[2];
-                const double s3 = p3[0] * g[0] + p3[1] * g[1] + p3[2] * g[2];
-                const double* sv = (s1 < s2 && s1 < s3) ? p1 : ((s2 < s1 && s2 < s3) ? p2 : p3);
-#pragma unroll
-                for (int k = 0; k < 3; k++) x[k] = x[k] + al * (sv[k] - x[k]);
-            }
-            const double dist = sdf_eval(P, x);
-            if (dist <= 1e-4) {
-                double v0[3], v1[3], v2[3];
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    v0[k] = p2[k] - p1[k];
-                    v1[k] = p3[k] - p1[k];
-                    v2[k] = x[k] - p1[k];
-                }
-                const double d00 = v0[0] * v0[0] + v0[1] * v0[1] + v0[2] * v0[2];
-                const double d01 = v0[0] * v1[0] + v0[1] * v1[1] + v0[2] * v1[2];
-                const double d11 = v1[0] * v1[0] + v1[1] * v1[1] + v1[2] * v1[2];
-                const double d20 = v2[0] * v0[0] + v2[1] * v0[1] + v2[2] * v0[2];
-                const double d21 = v2[0] * v1[0] + v2[1] * v1[1] + v2[2] * v1[2];
-                const double den = d00 * d11 - d01 * d01;
-                const double bv = (d11 * d20 - d01 * d21) / den;
-                const double bw = (d00 * d21 - d01 * d20) / den;
-                double g[3];
-                sdf_grad(P, x, g);
-#pragma unroll
-                for (int k = 0; k < 3; k++) {
-                    cp[3 * (size_t)j + k] = x[k] - g[k] * dist;
-                    cn[3 * (size_t)j + k] = g[k];
-                }
-                cb[3 * (size_t)j] = 1 - bv - bw;
-                cb[3 * (size_t)j + 1] = bv;
-                cb[3 * (size_t)j + 2] = bw;
-                hit = 1;
-            }
-        }
+    for (int k = 0; k < 3; k++) {
+        asm volatile("" : "+v"(p1[k]), "+v"(p2[k]), "+v"(p3[k]));
+        asm volatile("" : "+v"(S.pos[k]), "+v"(S.vel[k]), "+v"(S.prm[k]), "+v"(S.quat[k]));
     }
-    flag[j] = hit;
+    asm volatile("" : "+v"(S.kind), "+v"(S.quat[3]), "+v"(t));
+    bool hit = false;
+    if (j < nf) {
+        hit = detect_face(S, t, p1, p2, p3, cp + 3 * (size_t)j, cn + 3 * (size_t)j, cb + 3 * (size_t)j);
+        flag[j] = hit ? 1 : 0;
+    }
+    int hits;
+    hits_before(hit, ws, hits);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = hits;
 }
-
-// Ordered compaction of the hit flags in three small kernels:
-//   count   per 256-face block, hits counted with wave ballots
-//   scan    one workgroup turns the block counts into block offsets
-//   scatter each hit's position = block offset + hits before it in the block
-// Result: cpos[j] = number of hits before face slot j, cpos[nf] = total,
-// clist[cpos[j]] = j for every hit (face order preserved).
-constexpr int kScan = 1024;
-constexpr int kWaves = kBlock / 64;
 
 __global__ __launch_bounds__(kBlock) void k_count_hits(const int* __restrict__ flag, int nf, int* __restrict__ bsum)
 {
     __shared__ int ws[kWaves];
     const int j = blockIdx.x * kBlock + threadIdx.x;
-    const unsigned long long m = __ballot(j < nf && flag[j] != 0);
-    if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = __popcll(m);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int w = 0; w < kWaves; w++) t += ws[w];
-        bsum[blockIdx.x] = t;
-    }
+    int hits;
+    hits_before(j < nf && flag[j] != 0, ws, hits);
+    if (threadIdx.x == 0) bsum[blockIdx.x] = hits;
 }
 
-__global__ __launch_bounds__(kScan) void k_scan_blocks(int* __restrict__ bsum, int nb, int* __restrict__ cpos, int nf)
-{
-    __shared__ int sh[kScan];
-    const int chunk = (nb + kScan - 1) / kScan;
-    const int b = threadIdx.x * chunk;
-    const int e = min(nb, b + chunk);
-    int cnt = 0;
-    for (int j = b; j < e; j++) cnt += bsum[j];
-    sh[threadIdx.x] = cnt;
-    __syncthreads();
-    for (int off = 1; off < kScan; off <<= 1) {  // Hillis-Steele inclusive scan
-        const int v = (int)threadIdx.x >= off ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
-        sh[threadIdx.x] += v;
-        __syncthreads();
-    }
-    int run = sh[threadIdx.x] - cnt;
-    for (int j = b; j < e; j++) {
-        const int v = bsum[j];
-        bsum[j] = run;
-        run += v;
-    }
-    if (threadIdx.x == kScan - 1) cpos[nf] = sh[kScan - 1];
-}
-
+// Ordered compaction of the hit flags, from the hits of each 256 faces:
+// cpos[j] = number of hits before face slot j, cpos[nf] = total,
+// clist[cpos[j]] = j for every hit (face order preserved).  Every workgroup adds
+// up the counts before its own, some loads a thread (a million faces: 16),
+// instead of a launch of its own for that.
 __global__ __launch_bounds__(kBlock) void k_scatter_hits(const int* __restrict__ flag, int nf,
-                                                        const int* __restrict__ boff, int* __restrict__ cpos,
+                                                        const int* __restrict__ bsum, int* __restrict__ cpos,
                                                         int* __restrict__ clist)
 {
-    __shared__ int ws[kWaves];
+    __shared__ int ws[kWaves], wb[kWaves];
     const int j = blockIdx.x * kBlock + threadIdx.x;
+    int sum = 0;
+    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) sum += bsum[b];
     const bool f = j < nf && flag[j] != 0;
-    const unsigned long long m = __ballot(f);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) ws[wv] = __popcll(m);
-    __syncthreads();
-    int base = boff[blockIdx.x];
-    for (int w = 0; w < wv; w++) base += ws[w];
-    const int p = base + __popcll(m & ((1ull << lane) - 1ull));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    if ((threadIdx.x & 63) == 0) wb[threadIdx.x >> 6] = sum;
+    int hits;
+    int p = hits_before(f, ws, hits), base = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; w++) base += wb[w];
+    p += base;
     if (j < nf) {
         cpos[j] = p;
         if (f) clist[p] = j;
     }
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) cpos[nf] = base + hits;
 }
 
 // Static contact projection in FP64 (alpha = 0, inequality):
@@ -2566,11 +2497,13 @@ hipError_t launch_primary_residual(hipStream_t s, const TetArrays& ta, const Pri
 
 hipError_t launch_detect(hipStream_t s, const int4* faces, int nf, const double* rest, const float4* pos,
                          const float4* lo, const SdfDev* sdf, const unsigned long long* step, double dt, int* flag,
-                         double* cp, double* cn, double* cb)
+                         int* cpos, int* clist, int* bsum, double* cp, double* cn, double* cb)
 {
     if (nf <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_detect, dim3(nblk(nf, kBlock)), dim3(kBlock), 0, s, faces, nf, rest, pos, lo, sdf, step, dt,
-                       flag, cp, cn, cb);
+    const dim3 g(nblk(nf, kBlock));
+    hipLaunchKernelGGL(k_detect, g, dim3(kBlock), 0, s, faces, nf, rest, pos, lo, sdf, step, dt, flag, bsum, cp, cn,
+                       cb);
+    hipLaunchKernelGGL(k_scatter_hits, g, dim3(kBlock), 0, s, flag, nf, bsum, cpos, clist);
     return hipGetLastError();
 }
 
@@ -2580,7 +2513,6 @@ hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int
 {
     const int nb = compact_blocks(nf);
     hipLaunchKernelGGL(k_count_hits, dim3(nb), dim3(kBlock), 0, s, flag, nf, bsum);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(kScan), 0, s, bsum, nb, cpos, nf);
     hipLaunchKernelGGL(k_scatter_hits, dim3(nb), dim3(kBlock), 0, s, flag, nf, bsum, cpos, clist);
     return hipGetLastError();
 }
