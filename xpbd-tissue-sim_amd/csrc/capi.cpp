@@ -478,6 +478,22 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
     rc |= dalloc(h, &h->d_cn, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_cb, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_clam, nf);
+    // Gauss-Seidel contacts: room for what a solve's first contact pass leaves to
+    // the later ones (without it each gathers for itself)
+    if (rc == XPBD_OK && P->solver == XPBD_SOLVER_GS_COLORED && nf > 0) {
+        std::vector<int32_t> count(h->ninst, 0);
+        for (int f = 0; f < nf; f++) count[faces[4 * (size_t)f + 3]]++;
+        ContactWork& W = h->contact_work;
+        W.cap = std::min(compact_block(), *std::max_element(count.begin(), count.end()));
+        const size_t room = (size_t)h->ninst * W.cap, kept = h->allocs.size();
+        if (dalloc(h, &W.head, (size_t)h->ninst) || dalloc(h, &W.where, 3 * room) || dalloc(h, &W.contact, room) ||
+            dalloc(h, &W.fixed, kContactDoubles * room)) {
+            for (; h->allocs.size() > kept; h->allocs.pop_back()) (void)hipFree(h->allocs.back());
+            W = ContactWork{};
+            (void)hipGetLastError();
+            h->err.clear();
+        }
+    }
     // deterministic patch Jacobi: contact corrections per face slot, gathered per
     // vertex over (face slot * 3 + corner) in ascending face slot
     std::vector<int32_t> vf_off, vf;
@@ -843,7 +859,7 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
             const ContactSlots slots{ P.launches[0].d[cur], P.copy_off, P.copy };
             e = launch_contacts_gs(s, h->d_faces, h->d_fci_off, h->nfcolors, h->ninst, h->d_cpos, h->d_clist, h->d_rest,
                                    h->d_pos, h->d_lo, h->d_cp, h->d_cn, h->d_cb, h->d_clam, it == 0 && reset_lambda,
-                                   nullptr, nullptr, &slots);
+                                   nullptr, nullptr, &slots, &h->contact_work, it > 0 && h->contact_work.cap > 0);
             if (e != hipSuccess) return hip_err(h, e, "contacts_gs launch");
         }
     }
@@ -949,7 +965,8 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
             if (con) {
                 e = launch_contacts_gs(s, h->d_faces, h->d_fci_off, h->nfcolors, h->ninst, h->d_cpos, h->d_clist, h->d_rest,
                                        h->d_pos, h->d_lo, h->d_cp, h->d_cn, h->d_cb, h->d_clam, first, dsep,
-                                       dsep ? dsep + h->nv : nullptr);
+                                       dsep ? dsep + h->nv : nullptr, nullptr, &h->contact_work,
+                                       it > 0 && h->contact_work.cap > 0);
                 if (e != hipSuccess) return hip_err(h, e, "contacts_gs launch");
             }
             // attachments follow the collision projectors (type-list order, XPBDTypedefs.hpp:56)

@@ -70,6 +70,7 @@ struct xpbd_handle {
     // are one run: fci_off[c * (ninst + 1) + i] is where instance i's faces of
     // colour c start (i = ninst: the colour's end)
     std::vector<int32_t> fci_off;
+    xpbd::ContactWork contact_work;   // Gauss-Seidel; cap 0: none
     std::vector<xpbd::SdfDev> sdf_host;
     bool sdf_active = false;
     bool contacts_given = false;  // a contact set from xpbd_set_contacts is in use

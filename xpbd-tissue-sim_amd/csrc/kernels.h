@@ -196,6 +196,7 @@ hipError_t launch_detect(hipStream_t s, const int4* faces, int nf, const double*
                          int* cpos, int* clist, int* bsum, double* cp, double* cn, double* cb);
 // The compaction alone, of flags from elsewhere.
 int compact_blocks(int nf);
+int compact_block();   // faces of a block, threads of a contact workgroup
 hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int* clist, int* bsum);
 // Gauss-Seidel contacts: one workgroup per instance (instances share no
 // vertex), colour by colour; fci_off[c * (ninst + 1) + i] is the face position
@@ -207,11 +208,22 @@ struct ContactSlots {
     const int* off;    // vertex -> its range in slot
     const int* slot;
 };
+// With work a pass leaves what it gathered there, and with reuse, for the later
+// passes of the same solve, on the same motions' places, it starts from that.
+constexpr int kContactDoubles = 37;
+struct ContactWork {
+    int cap = 0;               // contacts of an instance that there is room for, at most compact_block()
+    int4* head = nullptr;      // per instance
+    int4* where = nullptr;     // 3 cap an instance
+    int4* contact = nullptr;   // cap an instance
+    double* fixed = nullptr;   // kContactDoubles * cap an instance
+};
 hipError_t launch_contacts_gs(hipStream_t s, const int4* faces, const int* fci_off, int ncol, int ninst,
                               const int* cpos, const int* clist, const double* rest, float4* pos, const float4* lo,
                               const double* cp, const double* cn, const double* cb, double* clam, bool first,
                               float4* dsep = nullptr, const float4* dbase = nullptr,
-                              const ContactSlots* slots = nullptr);
+                              const ContactSlots* slots = nullptr, const ContactWork* work = nullptr,
+                              bool reuse = false);
 hipError_t launch_contacts_jacobi(hipStream_t s, const int4* faces, int nf, const int* cpos, const int* clist,
                                   const double* rest, const float4* pos, const float4* lo, float* acc,
                                   const double* cp, const double* cn, const double* cb, double* clam, bool first);
