@@ -453,6 +453,7 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         rc |= dalloc(h, &h->d_inc, Pt.inc.size());
         rc |= dalloc(h, &h->d_partial, 2 * (size_t)Pt.nslots);
         rc |= dalloc(h, &h->d_shared, Pt.shared.size());
+        rc |= dalloc(h, &h->d_vshare, nv);
         rc |= dalloc(h, &h->d_soff, Pt.soff.size());
         rc |= dalloc(h, &h->d_pshare, Pt.pverts.size());
         rc |= dalloc(h, &h->d_sbuf, 2 * Pt.shared.size());
@@ -648,6 +649,9 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         if (!Pt.shared.empty()) {
             UP(h->d_shared, Pt.shared.data(), sizeof(int32_t) * Pt.shared.size());
         }
+        std::vector<int32_t> vshare(nv, -1);
+        for (size_t j = 0; j < Pt.shared.size(); j++) vshare[Pt.shared[j]] = (int32_t)j;
+        UP(h->d_vshare, vshare.data(), sizeof(int32_t) * vshare.size());
         UP(h->d_soff, Pt.soff.data(), sizeof(int32_t) * Pt.soff.size());
         UP(h->d_pshare, Pt.pshare.data(), sizeof(int32_t) * Pt.pshare.size());
         if (h->fused_ok) {
@@ -820,11 +824,54 @@ int enqueue_contacts_jacobi(xpbd_handle* h, bool first)
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "contacts_jacobi launch");
 }
 
+static Prediction prediction(const xpbd_handle* h)
+{
+    const double dt = h->params.dt;
+    return { h->d_vel, h->params.first_order ? h->d_dz1 : nullptr, (float)dt, (float)(-h->params.g * dt * dt) };
+}
+
+static HitLists hit_lists(const xpbd_handle* h)
+{
+    HitLists H;
+    H.flag = h->d_flag;
+    H.nf = h->nf;
+    H.bsum = h->d_bsum;
+    H.cpos = h->d_cpos;
+    H.clist = h->d_clist;
+    return H;
+}
+
+// What else of a step the iterations' own first and last launches do, where the
+// step lets them (step_ends): each launch of its own costs some 4 us.
+struct StepEnds {
+    bool predict = false;   // the motions start as the prediction
+    bool hits = false;      // with predict: lists of the detection's hits
+    bool finish = false;    // velocities, bases, the step counter
+};
+
+static bool runs_tiled(const xpbd_handle* h, int iters)
+{
+    return h->variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block == kQuadTile && h->natt == 0 && iters > 0 &&
+           !h->tiles.launches.empty();
+}
+
+static bool runs_fused_jacobi(const xpbd_handle* h)
+{
+    return h->variant == XPBD_VARIANT_PATCH && h->patch_fused && h->fused_ok && h->params.deterministic != 0 &&
+           h->natt == 0;
+}
+
+static int enqueue_finish(xpbd_handle* h, const MotionSource& from)
+{
+    hipError_t e = launch_finish(h->stream, h->d_pos, h->d_lo, h->d_vel, h->nv, (float)h->params.dt, h->d_step, from);
+    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "finish launch");
+}
+
 // The iterations by fused-colour launches (gs_tiles.h).  A launch reads its
 // group's slots and writes the next group's; a closed plan's tiles depend on
 // nothing outside them and update in place, all iterations in one launch when
 // no contacts come between them.
-static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
+static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda, const StepEnds& ends)
 {
     hipStream_t s = h->stream;
     const bool con = contacts_enabled(h);
@@ -832,8 +879,10 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
     const size_t ng = P.launches.size();
     const bool swap = ng == 1 && !P.closed;
     int cur = 0;   // which of the first group's two arrays, where it has two
+    const Prediction predict = prediction(h);
+    const HitLists hits = hit_lists(h);
     hipError_t e = launch_gs_tile_load(s, h->d_pos, P.slot_vert, P.nslots, P.launches[0].nslots, P.launches[0].d[0],
-                                       P.base);
+                                       P.base, ends.predict ? &predict : nullptr, ends.hits ? &hits : nullptr);
     if (e != hipSuccess) return hip_err(h, e, "gs_tile_load launch");
     for (int it = 0, inner; it < iters; it += inner) {
         const bool import = it == 0 && !reset_lambda;
@@ -863,6 +912,12 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
             if (e != hipSuccess) return hip_err(h, e, "contacts_gs launch");
         }
     }
+    if (ends.finish) {
+        MotionSource from;
+        from.owner = P.owner;
+        from.d = P.launches[0].d[cur];
+        return enqueue_finish(h, from);
+    }
     e = launch_gs_tile_store(s, h->d_pos, P.owner, h->nv, P.launches[0].d[cur]);
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "gs_tile_store launch");
 }
@@ -871,14 +926,13 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
 // reset_lambda (the reference solve, XPBDSolver.hpp:66-77) the first iteration
 // starts every multiplier at zero; without it every multiplier (element,
 // contact, attachment) keeps the value the caller left (a warm start).
-int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
+static int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda, const StepEnds& ends)
 {
     hipStream_t s = h->stream;
     TetArrays ta = tet_arrays(h);
     const bool con = contacts_enabled(h);
     hipError_t e = hipSuccess;
-    if (h->variant == XPBD_VARIANT_PATCH && h->patch_fused && h->fused_ok && h->params.deterministic != 0 &&
-        h->natt == 0) {
+    if (runs_fused_jacobi(h)) {
         // fused patch Jacobi: one launch per iteration, the shared vertices' last
         // sums after the loop
         const Patches& Pt = h->patches;
@@ -920,10 +974,20 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
                 h->timed_iterations++;
             }
         }
+        // after iteration n-1: values before it in half n % 2, its partials in half (n-1) % 2
+        const float4 *prd = h->d_partial + ((iters - 1) & 1) * nsl, *brd = h->d_sbuf + (iters & 1) * nsh;
+        if (ends.finish) {
+            MotionSource from;
+            if (iters > 0) {
+                from.vshare = h->d_vshare;
+                from.soff = h->d_soff;
+                from.prd = prd;
+                from.brd = brd;
+            }
+            return enqueue_finish(h, from);
+        }
         if (iters > 0) {
-            // after iteration n-1: values before it in half n % 2, its partials in half (n-1) % 2
-            e = launch_jacobi_fused_final(s, h->d_shared, h->d_soff, h->d_partial + ((iters - 1) & 1) * nsl,
-                                          h->d_sbuf + (iters & 1) * nsh, h->d_pos, (int)nsh);
+            e = launch_jacobi_fused_final(s, h->d_shared, h->d_soff, prd, brd, h->d_pos, (int)nsh);
             if (e != hipSuccess) return hip_err(h, e, "jacobi_fused_final launch");
         }
         return XPBD_OK;
@@ -932,9 +996,7 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
     // for their own array before the loop and return after it, and the bases,
     // which the loop only reads, are copied into one (the attachment pass reads
     // the records, so handles with attachments stay interleaved).
-    const bool tiled = h->variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block == kQuadTile && h->natt == 0 &&
-                       iters > 0 && !h->tiles.launches.empty();
-    if (tiled) return enqueue_tiled_iterations(h, iters, timed, reset_lambda);
+    if (runs_tiled(h, iters)) return enqueue_tiled_iterations(h, iters, timed, reset_lambda, ends);
     const int quad_block = h->quad_block == kQuadTile ? 256 : h->quad_block;
     float4* dsep = h->params.solver == XPBD_SOLVER_GS_COLORED && h->variant == XPBD_VARIANT_CLUSTER_QUAD &&
                            quad_split(quad_block) && h->natt == 0 && iters > 0
@@ -1023,10 +1085,15 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
 // contacts) with the multipliers kept.  Gauss-Seidel visits the elements in the
 // global solve's order, an element's repeats back to back; Jacobi sums every
 // projection of a pass from the same positions.  Attachments are not part of it.
+static bool local_collision(const xpbd_handle* h)
+{
+    return h->params.local_collision_iters > 0 && h->d_mult && contacts_enabled(h);
+}
+
 int enqueue_local_collision(xpbd_handle* h)
 {
     const int n = h->params.local_collision_iters;
-    if (n <= 0 || !h->d_mult || !contacts_enabled(h)) return XPBD_OK;
+    if (!local_collision(h)) return XPBD_OK;
     hipStream_t s = h->stream;
     const TetArrays ta = tet_arrays(h);
     hipError_t e = launch_fill_zero(s, h->d_mult, sizeof(int32_t) * (size_t)h->nt);
@@ -1065,36 +1132,60 @@ int enqueue_local_collision(xpbd_handle* h)
     return XPBD_OK;
 }
 
-int enqueue_detect(xpbd_handle* h)
+static int enqueue_flags(xpbd_handle* h)
 {
-    hipError_t e = launch_detect(h->stream, h->d_faces, h->nf, h->d_rest, h->d_pos, h->d_lo, h->d_sdf, h->d_step,
-                                 h->params.dt, h->d_flag, h->d_cpos, h->d_clist, h->d_bsum, h->d_cp, h->d_cn, h->d_cb);
+    hipError_t e = launch_detect(h->stream, h->d_faces, h->d_rest, h->d_pos, h->d_lo, h->d_sdf, h->d_step, h->params.dt,
+                                 h->d_flag, hit_lists(h), h->d_cp, h->d_cn, h->d_cb);
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "detect launch");
 }
 
-int enqueue_predict(xpbd_handle* h)
+int enqueue_detect(xpbd_handle* h)
 {
-    const double dt = h->params.dt;
-    hipError_t e = h->params.first_order
-                       ? launch_predict_first_order(h->stream, h->d_pos, h->d_dz1, h->nv)
-                       : launch_predict(h->stream, h->d_pos, h->d_vel, h->nv, (float)dt, (float)(-h->params.g * dt * dt));
+    int rc = enqueue_flags(h);
+    if (rc || h->nf <= 0) return rc;
+    hipError_t e = launch_compact(h->stream, hit_lists(h), false);
+    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "compact launch");
+}
+
+static int enqueue_predict(xpbd_handle* h, bool hits)
+{
+    const HitLists H = hit_lists(h);
+    hipError_t e = launch_predict(h->stream, h->d_pos, h->nv, prediction(h), hits ? &H : nullptr);
     if (e == hipSuccess && h->primary_residual) e = launch_keep_prediction(h->stream, h->d_pos, h->d_pred, h->nv);
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "predict launch");
 }
 
-int enqueue_finish(xpbd_handle* h)
+int enqueue_predict(xpbd_handle* h) { return enqueue_predict(h, false); }
+
+int enqueue_finish(xpbd_handle* h) { return enqueue_finish(h, MotionSource{}); }
+
+int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
 {
-    hipError_t e = launch_finish(h->stream, h->d_pos, h->d_lo, h->d_vel, h->nv, (float)h->params.dt, h->d_step);
-    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "finish launch");
+    return enqueue_iterations(h, iters, timed, reset_lambda, StepEnds{});
+}
+
+// What the iterations' launches may do besides: the prediction where nothing else
+// reads it, the velocity update where nothing comes between.
+static StepEnds step_ends(const xpbd_handle* h, bool detect)
+{
+    const bool tiled = runs_tiled(h, h->params.iters);
+    StepEnds ends;
+    ends.predict = tiled && !h->primary_residual;
+    ends.hits = ends.predict && detect;
+    ends.finish = (tiled || runs_fused_jacobi(h)) && !records_residuals(h) && !local_collision(h);
+    return ends;
 }
 
 // Whole step: [detect] predict iterations finish
 static int enqueue_step(xpbd_handle* h, bool detect, bool timed)
 {
     int rc;
-    if (detect && contacts_enabled(h) && (rc = enqueue_detect(h))) return rc;
-    if ((rc = enqueue_predict(h))) return rc;
-    if ((rc = enqueue_iterations(h, h->params.iters, timed))) return rc;
+    const bool det = detect && contacts_enabled(h) && h->nf > 0;
+    const StepEnds ends = step_ends(h, det);
+    if (det && (rc = enqueue_flags(h))) return rc;
+    if (!ends.predict && (rc = enqueue_predict(h, det))) return rc;
+    if ((rc = enqueue_iterations(h, h->params.iters, timed, true, ends))) return rc;
+    if (ends.finish) return XPBD_OK;
     if (records_residuals(h) && (rc = enqueue_step_residual(h))) return rc;
     if ((rc = enqueue_local_collision(h))) return rc;
     return enqueue_finish(h);
@@ -1726,7 +1817,7 @@ extern "C" int xpbd_set_contacts(xpbd_handle* h, int32_t n, const int32_t* faces
         if (e == hipSuccess) e = hipMemcpyAsync(h->d_cn, cn.data(), sizeof(double) * 3 * nf, hipMemcpyHostToDevice, h->stream);
         if (e == hipSuccess) e = hipMemcpyAsync(h->d_cb, cb.data(), sizeof(double) * 3 * nf, hipMemcpyHostToDevice, h->stream);
         if (e == hipSuccess) e = launch_fill_zero(h->stream, h->d_clam, sizeof(double) * nf);
-        if (e == hipSuccess) e = launch_compact(h->stream, h->d_flag, nf, h->d_cpos, h->d_clist, h->d_bsum);
+        if (e == hipSuccess) e = launch_compact(h->stream, hit_lists(h), true);
         if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
         if (e != hipSuccess) return hip_err(h, e, "set_contacts");
     }

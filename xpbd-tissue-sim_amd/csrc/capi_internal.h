@@ -98,6 +98,7 @@ struct xpbd_handle {
     int32_t* d_inc_off = nullptr;
     uint16_t* d_inc = nullptr;
     float4* d_partial = nullptr;     // 2 x nslots: partial sums, by iteration parity in the fused variant
+    int32_t* d_vshare = nullptr;   // vertex -> its place among the shared ones, or -1
     int32_t* d_shared = nullptr;
     int32_t* d_soff = nullptr;
     // fused patch Jacobi (one launch per iteration, see FusedPatchArgs)

@@ -64,7 +64,7 @@ hipError_t launch_gs_tile(hipStream_t s, const GsTileArgs& A, const GsTileShape&
 hipError_t launch_gs_tile_fill(hipStream_t s, const GsTileFill& A, const GsTileShape& S);
 // bases of the vertex records into n slots, in-step motions into the first nd; motions back
 hipError_t launch_gs_tile_load(hipStream_t s, const float4* pos, const int* slot_vert, int n, int nd, float4* d,
-                               float4* base);
+                               float4* base, const Prediction* predict = nullptr, const HitLists* hits = nullptr);
 hipError_t launch_gs_tile_store(hipStream_t s, float4* pos, const int* owner, int nv, const float4* d);
 
 }  // namespace xpbd

@@ -14,6 +14,7 @@
 
 #include "gs_tile_kernels.h"
 #include "quad_ops.h"
+#include "step_ops.h"
 #include "xpbd_math.h"
 
 namespace xpbd {
@@ -591,17 +592,27 @@ __global__ __launch_bounds__(256) void k_gs_tile_lane_fill(GsTileFill A)
 
 // The step's motions and bases out of the vertex records into all groups' slots
 // (the motions into the first group's, whose slots come first), and the motions
-// back from the owners' slots.
+// back from the owners' slots.  PREDICT: the motions are the step's prediction,
+// formed here, and the launch makes the lists of a detection's hits too.
+template <bool PREDICT>
 __global__ __launch_bounds__(256) void k_gs_tile_load(const float4* __restrict__ pos, const int* __restrict__ slot_vert,
-                                                     int n, int nd, float4* __restrict__ d, float4* __restrict__ base)
+                                                     int n, int nd, float4* __restrict__ d, float4* __restrict__ base,
+                                                     Prediction P, HitLists H, int nload)
 {
+    if constexpr (PREDICT) {
+        __shared__ int ws[2 * kStepWaves];
+        if ((int)blockIdx.x >= nload) {
+            scatter_hits(H, blockIdx.x - nload, gridDim.x - nload, ws);
+            return;
+        }
+    }
     const int s = blockIdx.x * 256 + threadIdx.x;
     if (s >= n) return;
     const int v = slot_vert[s];
     float4 b = make_float4(0.f, 0.f, 0.f, 0.f), x = b;
     if (v >= 0) {
         b = pos[2 * (size_t)v];
-        if (s < nd) x = pos[2 * (size_t)v + 1];
+        if (s < nd) x = PREDICT ? predicted(P, v) : pos[2 * (size_t)v + 1];
     }
     base[s] = b;
     if (s < nd) d[s] = x;
@@ -677,10 +688,17 @@ hipError_t launch_gs_tile_fill(hipStream_t s, const GsTileFill& A, const GsTileS
 }
 
 hipError_t launch_gs_tile_load(hipStream_t s, const float4* pos, const int* slot_vert, int n, int nd, float4* d,
-                               float4* base)
+                               float4* base, const Prediction* predict, const HitLists* hits)
 {
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_gs_tile_load, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, pos, slot_vert, n, nd, d, base);
+    const int nl = (n + 255) / 256, nh = hits && hits->nf > 0 ? compact_blocks(hits->nf) : 0;
+    if (nl + nh <= 0) return hipSuccess;
+    if (hits && !predict) return hipErrorInvalidValue;
+    if (predict)
+        hipLaunchKernelGGL(k_gs_tile_load<true>, dim3(nl + nh), dim3(256), 0, s, pos, slot_vert, n, nd, d, base, *predict,
+                           hits ? *hits : HitLists{}, nl);
+    else
+        hipLaunchKernelGGL(k_gs_tile_load<false>, dim3(nl), dim3(256), 0, s, pos, slot_vert, n, nd, d, base, Prediction{},
+                           HitLists{}, nl);
     return hipGetLastError();
 }
 

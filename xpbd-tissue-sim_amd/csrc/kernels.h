@@ -32,11 +32,37 @@ struct TetArrays {
 // Vertex records: pos[2i] = (base displacement xyz, inverse mass),
 // pos[2i+1] = (in-step motion xyz, 0); lo[i] = low-order part of the base;
 // vel[i] = (velocity xyz, pinned flag).
-hipError_t launch_predict(hipStream_t s, float4* pos, const float4* vel, int nv, float dt, float dz);
-// first-order inertial move: delta = (0, 0, dz1[i])
-hipError_t launch_predict_first_order(hipStream_t s, float4* pos, const float* dz1, int nv);
+struct Prediction {   // inertial move: (dt vel.xy, dt vel.z + dz), or, first order, (0, 0, dz1[i])
+    const float4* vel;
+    const float* dz1;   // null: second order
+    float dt, dz;
+};
+// Hit flags of the face slots and the lists made of them; bsum: hits of each
+// compact_block() faces.
+struct HitLists {
+    const int* flag = nullptr;
+    int nf = 0;            // 0: none
+    int* bsum = nullptr;   // compact_blocks(nf)
+    int* cpos = nullptr;   // nf + 1
+    int* clist = nullptr;  // nf
+};
+int compact_block();    // faces of a block; also the threads of a contact workgroup
+int compact_blocks(int nf);
+// With hits, the same launch also makes the lists of a detection's flags.
+hipError_t launch_predict(hipStream_t s, float4* pos, int nv, const Prediction& P, const HitLists* hits = nullptr);
+// Where the step's motions are found, if not in the vertex records: in fused-colour
+// slots (d by owner), or, for the vertices that patches share (vshare >= 0), as a
+// last iteration's value before it plus its partial sums.
+struct MotionSource {
+    const int* owner = nullptr;
+    const float4* d = nullptr;
+    const int* vshare = nullptr;
+    const int* soff = nullptr;
+    const float4* prd = nullptr;
+    const float4* brd = nullptr;
+};
 hipError_t launch_finish(hipStream_t s, float4* pos, float4* lo, float4* vel, int nv, float dt,
-                         unsigned long long* step_counter);
+                         unsigned long long* step_counter, const MotionSource& from = MotionSource{});
 // Deterministic Jacobi: contacts into per-face slots, then a per-vertex gather in
 // face-slot order; local passes into per-element slots, then a per-vertex gather
 // in solver-position order.
@@ -189,15 +215,13 @@ hipError_t launch_element_forces(hipStream_t s, const TetArrays& ta, const Prima
 hipError_t launch_consistent_shift(hipStream_t s, float4* pos, const float4* pred, const int* vt_off,
                                    const double* ef, int nv);
 
-// Contacts.  faces: (a, b, c, instance) in colour-sorted order.  Detection, then
-// the ordered compaction of its hits; bsum is scratch of compact_blocks(nf) ints.
-hipError_t launch_detect(hipStream_t s, const int4* faces, int nf, const double* rest, const float4* pos,
-                         const float4* lo, const SdfDev* sdf, const unsigned long long* step, double dt, int* flag,
-                         int* cpos, int* clist, int* bsum, double* cp, double* cn, double* cb);
-// The compaction alone, of flags from elsewhere.
-int compact_blocks(int nf);
-int compact_block();   // faces of a block, threads of a contact workgroup
-hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int* clist, int* bsum);
+// Contacts.  faces: (a, b, c, instance) in colour-sorted order.  Detection leaves
+// flags and block counts; launch_compact (with count, of flags from elsewhere) or
+// launch_predict makes the lists.
+hipError_t launch_detect(hipStream_t s, const int4* faces, const double* rest, const float4* pos, const float4* lo,
+                         const SdfDev* sdf, const unsigned long long* step, double dt, int* flag, const HitLists& hits,
+                         double* cp, double* cn, double* cb);
+hipError_t launch_compact(hipStream_t s, const HitLists& hits, bool count);
 // Gauss-Seidel contacts: one workgroup per instance (instances share no
 // vertex), colour by colour; fci_off[c * (ninst + 1) + i] is the face position
 // where instance i's faces of colour c start.

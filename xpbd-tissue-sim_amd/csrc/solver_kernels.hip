@@ -13,6 +13,7 @@
 #include "kernels.h"
 #include "mesh_tools.h"
 #include "quad_ops.h"
+#include "step_ops.h"
 #include "xpbd_math.h"
 
 namespace xpbd {
@@ -57,23 +58,16 @@ __device__ __forceinline__ void load_tet(const TetArrays& ta, int e, float* q, f
 // The step's motion starts as delta = dt v + (0, 0, -g dt^2); the base is the
 // position at the start of the step, so x_prev needs no copy.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void k_predict(float4* __restrict__ pos, const float4* __restrict__ vel,
-                                                   int nv, float dt, float dz)
+__global__ __launch_bounds__(kBlock) void k_predict(float4* __restrict__ pos, int nv, Prediction P, HitLists H,
+                                                   int npredict)
 {
+    __shared__ int ws[2 * kStepWaves];
+    if ((int)blockIdx.x >= npredict) {
+        scatter_hits(H, blockIdx.x - npredict, gridDim.x - npredict, ws);
+        return;
+    }
     const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nv) return;
-    const float4 v = vel[i];
-    pos[2 * (size_t)i + 1] = make_float4(dt * v.x, dt * v.y, dt * v.z + dz, 0.f);
-}
-
-// first-order inertial move (XPBDMeshObject.cpp:450-457): z -= g m_i dt / B_i,
-// no velocity term
-__global__ __launch_bounds__(kBlock) void k_predict_first_order(float4* __restrict__ pos,
-                                                               const float* __restrict__ dz1, int nv)
-{
-    const int i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= nv) return;
-    pos[2 * (size_t)i + 1] = make_float4(0.f, 0.f, dz1[i], 0.f);
+    if (i < nv) pos[2 * (size_t)i + 1] = predicted(P, i);
 }
 
 // ---------------------------------------------------------------------------
@@ -88,15 +82,39 @@ __device__ __forceinline__ void two_sum(float a, float b, float& s, float& e)
     e = (a - (s - bb)) + (b - bb);
 }
 
+// A vertex that patches share, after the last fused patch Jacobi iteration.
+__device__ __forceinline__ float4 shared_motion(const int* __restrict__ soff, const float4* __restrict__ prd,
+                                                const float4* __restrict__ brd, int j)
+{
+    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
+    for (int k = soff[j]; k < soff[j + 1]; k++) {
+        const float4 v = prd[k];
+        a0 += v.x;
+        a1 += v.y;
+        a2 += v.z;
+    }
+    float4 d = brd[j];
+    d.x += a0;
+    d.y += a1;
+    d.z += a2;
+    return d;
+}
+
+// The motion comes from wherever the iterations left it, so that no launch has to
+// bring it back to the records first.
 __global__ __launch_bounds__(kBlock) void k_finish(float4* __restrict__ pos, float4* __restrict__ lo,
                                                   float4* __restrict__ vel, int nv, float dt,
-                                                  unsigned long long* __restrict__ step)
+                                                  unsigned long long* __restrict__ step, MotionSource from)
 {
     const int i = blockIdx.x * kBlock + threadIdx.x;
     if (i == 0) step[0] = step[0] + 1ull;
     if (i >= nv) return;
     float4 b = pos[2 * (size_t)i];
-    float4 d = pos[2 * (size_t)i + 1];
+    float4 d = from.owner ? from.d[from.owner[i]] : pos[2 * (size_t)i + 1];
+    if (from.vshare) {
+        const int j = from.vshare[i];
+        if (j >= 0) d = shared_motion(from.soff, from.prd, from.brd, j);
+    }
     float4 l = lo[i];
     float4 v = vel[i];
     if (v.w != 0.0f) d = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1245,23 +1263,8 @@ __device__ __forceinline__ bool detect_face(const SdfDev& S, double t, const dou
     return true;
 }
 
-// Hits of a workgroup's faces before this thread's, and in hits of all of them.
-constexpr int kWaves = kBlock / 64;
-__device__ __forceinline__ int hits_before(bool hit, int* ws, int& hits)
-{
-    const unsigned long long m = __ballot(hit);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) ws[wv] = __popcll(m);
-    __syncthreads();
-    int before = __popcll(m & ((1ull << lane) - 1ull));
-    hits = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) {
-        if (w < wv) before += ws[w];
-        hits += ws[w];
-    }
-    return before;
-}
+constexpr int kWaves = kStepWaves;
+static_assert(kBlock == kStepBlock, "hits are counted by workgroup");
 
 // One thread a face.  Few waves get past the distance test, so the kernel takes as
 // long as one wave's chain: 32 search steps of some 55 instructions (sphere) or 110
@@ -1313,33 +1316,10 @@ __global__ __launch_bounds__(kBlock) void k_count_hits(const int* __restrict__ f
     if (threadIdx.x == 0) bsum[blockIdx.x] = hits;
 }
 
-// Ordered compaction of the hit flags, from the hits of each 256 faces:
-// cpos[j] = number of hits before face slot j, cpos[nf] = total,
-// clist[cpos[j]] = j for every hit (face order preserved).  Every workgroup adds
-// up the counts before its own, some loads a thread (a million faces: 16),
-// instead of a launch of its own for that.
-__global__ __launch_bounds__(kBlock) void k_scatter_hits(const int* __restrict__ flag, int nf,
-                                                        const int* __restrict__ bsum, int* __restrict__ cpos,
-                                                        int* __restrict__ clist)
+__global__ __launch_bounds__(kBlock) void k_scatter_hits(HitLists H)
 {
-    __shared__ int ws[kWaves], wb[kWaves];
-    const int j = blockIdx.x * kBlock + threadIdx.x;
-    int sum = 0;
-    for (int b = threadIdx.x; b < (int)blockIdx.x; b += kBlock) sum += bsum[b];
-    const bool f = j < nf && flag[j] != 0;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
-    if ((threadIdx.x & 63) == 0) wb[threadIdx.x >> 6] = sum;
-    int hits;
-    int p = hits_before(f, ws, hits), base = 0;
-#pragma unroll
-    for (int w = 0; w < kWaves; w++) base += wb[w];
-    p += base;
-    if (j < nf) {
-        cpos[j] = p;
-        if (f) clist[p] = j;
-    }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) cpos[nf] = base + hits;
+    __shared__ int ws[2 * kStepWaves];
+    scatter_hits(H, blockIdx.x, gridDim.x, ws);
 }
 
 // Static contact projection in FP64 (alpha = 0, inequality):
@@ -2058,18 +2038,7 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_fused_final(const int* __rest
 {
     const int j = blockIdx.x * kBlock + threadIdx.x;
     if (j >= ns) return;
-    float a0 = 0.f, a1 = 0.f, a2 = 0.f;
-    for (int k = soff[j]; k < soff[j + 1]; k++) {
-        const float4 v = prd[k];
-        a0 += v.x;
-        a1 += v.y;
-        a2 += v.z;
-    }
-    float4 d = brd[j];
-    d.x += a0;
-    d.y += a1;
-    d.z += a2;
-    pos[2 * (size_t)shared[j] + 1] = d;
+    pos[2 * (size_t)shared[j] + 1] = shared_motion(soff, prd, brd, j);
 }
 
 // Attachments (AttachmentConstraint.hpp:31-71 with ConstraintProjector.hpp:111-172,
@@ -2370,24 +2339,20 @@ hipError_t launch_jacobi_local(hipStream_t s, const TetArrays& ta, const int* mu
     return hipGetLastError();
 }
 
-hipError_t launch_predict(hipStream_t s, float4* pos, const float4* vel, int nv, float dt, float dz)
+hipError_t launch_predict(hipStream_t s, float4* pos, int nv, const Prediction& P, const HitLists* hits)
 {
-    if (nv <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_predict, dim3(nblk(nv, kBlock)), dim3(kBlock), 0, s, pos, vel, nv, dt, dz);
-    return hipGetLastError();
-}
-
-hipError_t launch_predict_first_order(hipStream_t s, float4* pos, const float* dz1, int nv)
-{
-    hipLaunchKernelGGL(k_predict_first_order, dim3(nblk(nv, kBlock)), dim3(kBlock), 0, s, pos, dz1, nv);
+    const HitLists H = hits ? *hits : HitLists{};
+    const int np = (int)nblk(nv, kBlock), nh = H.nf > 0 ? compact_blocks(H.nf) : 0;
+    if (np + nh <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_predict, dim3(np + nh), dim3(kBlock), 0, s, pos, nv, P, H, np);
     return hipGetLastError();
 }
 
 hipError_t launch_finish(hipStream_t s, float4* pos, float4* lo, float4* vel, int nv, float dt,
-                         unsigned long long* step_counter)
+                         unsigned long long* step_counter, const MotionSource& from)
 {
     hipLaunchKernelGGL(k_finish, dim3(nblk(nv > 0 ? nv : 1, kBlock)), dim3(kBlock), 0, s, pos, lo, vel, nv, dt,
-                       step_counter);
+                       step_counter, from);
     return hipGetLastError();
 }
 
@@ -2716,15 +2681,13 @@ hipError_t launch_primary_residual(hipStream_t s, const TetArrays& ta, const Pri
     return hipGetLastError();
 }
 
-hipError_t launch_detect(hipStream_t s, const int4* faces, int nf, const double* rest, const float4* pos,
-                         const float4* lo, const SdfDev* sdf, const unsigned long long* step, double dt, int* flag,
-                         int* cpos, int* clist, int* bsum, double* cp, double* cn, double* cb)
+hipError_t launch_detect(hipStream_t s, const int4* faces, const double* rest, const float4* pos, const float4* lo,
+                         const SdfDev* sdf, const unsigned long long* step, double dt, int* flag, const HitLists& hits,
+                         double* cp, double* cn, double* cb)
 {
-    if (nf <= 0) return hipSuccess;
-    const dim3 g(nblk(nf, kBlock));
-    hipLaunchKernelGGL(k_detect, g, dim3(kBlock), 0, s, faces, nf, rest, pos, lo, sdf, step, dt, flag, bsum, cp, cn,
-                       cb);
-    hipLaunchKernelGGL(k_scatter_hits, g, dim3(kBlock), 0, s, flag, nf, bsum, cpos, clist);
+    if (hits.nf <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_detect, dim3(nblk(hits.nf, kBlock)), dim3(kBlock), 0, s, faces, hits.nf, rest, pos, lo, sdf,
+                       step, dt, flag, hits.bsum, cp, cn, cb);
     return hipGetLastError();
 }
 
@@ -2732,11 +2695,11 @@ int compact_block() { return kBlock; }
 
 int compact_blocks(int nf) { return (int)nblk(nf > 0 ? nf : 1, kBlock); }
 
-hipError_t launch_compact(hipStream_t s, const int* flag, int nf, int* cpos, int* clist, int* bsum)
+hipError_t launch_compact(hipStream_t s, const HitLists& hits, bool count)
 {
-    const int nb = compact_blocks(nf);
-    hipLaunchKernelGGL(k_count_hits, dim3(nb), dim3(kBlock), 0, s, flag, nf, bsum);
-    hipLaunchKernelGGL(k_scatter_hits, dim3(nb), dim3(kBlock), 0, s, flag, nf, bsum, cpos, clist);
+    const dim3 g(compact_blocks(hits.nf));
+    if (count) hipLaunchKernelGGL(k_count_hits, g, dim3(kBlock), 0, s, hits.flag, hits.nf, hits.bsum);
+    hipLaunchKernelGGL(k_scatter_hits, g, dim3(kBlock), 0, s, hits);
     return hipGetLastError();
 }
 
