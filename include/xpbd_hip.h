@@ -331,7 +331,8 @@ int xpbd_autotune(xpbd_batch* b, const char* cache_path);
  * workgroup size (negative for the LDS-lean form; magnitude XPBD_QUAD_SPLIT +
  * size when the iterations keep the vertex deltas in their own array;
  * XPBD_QUAD_TILE for the fused-colour launches), for
- * PATCH 1 when the fused one-launch iteration is in use
+ * PATCH XPBD_PATCH_TILE for the vertex-tile launches, 1 when the fused one-launch
+ * iteration is in use
  * (deterministic mode without attachments), else 0; xcd: whether the
  * XCD-contiguous workgroup mapping is on (block and xcd may be NULL). */
 int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* xcd);
@@ -347,6 +348,13 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
  * the same results up to FP32 rounding within an element).  Handles with
  * attachments run the 256-thread quad shape instead. */
 #define XPBD_QUAD_TILE 4000
+/* The patch block value of the vertex-tile Jacobi launches, the untuned default
+ * where the mesh's size suits them: a workgroup owns a set of vertices and
+ * projects every element around them, so that one launch is an iteration and a
+ * vertex's corrections are summed in one place, in solver order (the sums of the
+ * other patch launches in another grouping).  Deterministic mode without
+ * attachments; otherwise such a handle runs the other patch launches. */
+#define XPBD_PATCH_TILE 2
 /* Batch handles are also plain handles: xpbd_step, xpbd_destroy, ... apply. */
 
 /* ---- host-side mesh utilities (no GPU needed) ------------------------------ */

@@ -72,17 +72,22 @@ bool valid(const xpbd_handle* h, const Candidate& c)
     if (c.variant == XPBD_VARIANT_CLUSTER) return h->nclusters > 0;
     if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile) return !h->tiles.launches.empty();
     if (c.variant == XPBD_VARIANT_CLUSTER_QUAD) return h->nclusters > 0 && quad_block_supported(c.block);
-    if (c.variant == XPBD_VARIANT_PATCH) return h->variant == XPBD_VARIANT_PATCH && (c.block == 0 || h->fused_ok);
+    if (c.variant == XPBD_VARIANT_PATCH) return h->variant == XPBD_VARIANT_PATCH &&
+               (c.block == XPBD_PATCH_TILE ? h->jtiles.ready : c.block == 0 || h->fused_ok);
     return c.variant == h->variant;
 }
 
 void apply(xpbd_handle* h, const Candidate& c)
 {
     if (h->variant != c.variant || (c.variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block != c.block) ||
-        (c.variant == XPBD_VARIANT_PATCH && h->patch_fused != (c.block == 1)) || h->xcd_map != (c.xcd != 0)) {
+        (c.variant == XPBD_VARIANT_PATCH &&
+         (h->patch_fused != (c.block == 1) || h->patch_tile != (c.block == XPBD_PATCH_TILE))) || h->xcd_map != (c.xcd != 0)) {
         h->variant = c.variant;
         if (c.variant == XPBD_VARIANT_CLUSTER_QUAD) h->quad_block = c.block;
-        if (c.variant == XPBD_VARIANT_PATCH) h->patch_fused = c.block == 1;
+        if (c.variant == XPBD_VARIANT_PATCH) {
+            h->patch_fused = c.block == 1;
+            h->patch_tile = c.block == XPBD_PATCH_TILE;
+        }
         h->xcd_map = c.xcd != 0;
         invalidate_graphs(h);
     }
@@ -100,6 +105,7 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     const std::string key = shape_key(h);
     Candidate c{};
     (void)ensure_gs_tiles(h);   // without a plan the other shapes are there
+    (void)ensure_jacobi_tiles(h);
     if (read_cache(cache_path, key, &c) && valid(h, c)) {
         apply(h, c);
         return XPBD_OK;
@@ -120,7 +126,9 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
                     cand.push_back({ b.variant, b.block < 0 ? b.block - kQuadSplit : b.block + kQuadSplit, x });
             }
     } else if (h->variant == XPBD_VARIANT_PATCH) {
-        // block 1: the fused one-launch iteration (when the layout allows it)
+        // the vertex-tile launches; block 1: the fused one-launch iteration (when the layout allows it)
+        if (h->jtiles.ready && h->natt == 0)
+            for (int x = 1; x >= 0; x--) cand.push_back({ h->variant, XPBD_PATCH_TILE, x });
         for (int f = h->fused_ok ? 1 : 0; f >= 0; f--)
             for (int x = 1; x >= 0; x--) cand.push_back({ h->variant, f, x });
     } else {
@@ -144,7 +152,7 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     if (e == hipSuccess) e = hipMemcpyAsync(save_lam, h->d_lam, lam_bytes, hipMemcpyDeviceToDevice, s);
     int rc = e == hipSuccess ? XPBD_OK : hip_err(h, e, "autotune set-up");
     const int saved_variant = h->variant, saved_block = h->quad_block;
-    const bool saved_xcd = h->xcd_map, saved_fused = h->patch_fused;
+    const bool saved_xcd = h->xcd_map, saved_fused = h->patch_fused, saved_tile = h->patch_tile;
     double best_ms = 1e300;
     Candidate best = cand[0];
     const int iters = h->params.iters > 0 ? h->params.iters : 1;
@@ -152,7 +160,10 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
         if (rc) break;
         h->variant = cd.variant;
         if (cd.variant == XPBD_VARIANT_CLUSTER_QUAD) h->quad_block = cd.block;
-        if (cd.variant == XPBD_VARIANT_PATCH) h->patch_fused = cd.block == 1;
+        if (cd.variant == XPBD_VARIANT_PATCH) {
+            h->patch_fused = cd.block == 1;
+            h->patch_tile = cd.block == XPBD_PATCH_TILE;
+        }
         h->xcd_map = cd.xcd != 0;
         double ms_best = 1e300;
         // the candidate's iterations are captured into a graph and the replays are
@@ -209,6 +220,7 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     h->quad_block = saved_block;
     h->xcd_map = saved_xcd;
     h->patch_fused = saved_fused;
+    h->patch_tile = saved_tile;
     if (rc) return rc;
     apply(h, best);
     write_cache(cache_path, key, best, best_ms / iters);
@@ -221,7 +233,7 @@ extern "C" int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block
     *variant = h->variant;
     if (block)
         *block = h->variant == XPBD_VARIANT_CLUSTER_QUAD ? h->quad_block
-               : h->variant == XPBD_VARIANT_PATCH    ? (h->patch_fused && h->fused_ok ? 1 : 0)
+               : h->variant == XPBD_VARIANT_PATCH    ? (h->patch_tile && h->jtiles.ready ? XPBD_PATCH_TILE : h->patch_fused && h->fused_ok ? 1 : 0)
                                                      : 0;
     if (xcd) *xcd = h->xcd_map ? 1 : 0;
     return XPBD_OK;

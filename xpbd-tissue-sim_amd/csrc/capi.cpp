@@ -699,6 +699,11 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         if (ensure_gs_tiles(h) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
         h->err.clear();
     }
+    // and of Jacobi: vertex-tile launches
+    if (P->variant == XPBD_VARIANT_AUTO && h->variant == XPBD_VARIANT_PATCH) {
+        h->patch_tile = ensure_jacobi_tiles(h) == XPBD_OK && h->jtiles.ready;
+        h->err.clear();
+    }
     *out = h;
     return XPBD_OK;
 }
@@ -861,6 +866,12 @@ static bool runs_fused_jacobi(const xpbd_handle* h)
            h->natt == 0;
 }
 
+static bool runs_tiled_jacobi(const xpbd_handle* h, int iters)
+{
+    return h->variant == XPBD_VARIANT_PATCH && h->patch_tile && h->jtiles.ready && h->params.deterministic != 0 &&
+           h->natt == 0 && iters > 0;
+}
+
 static int enqueue_finish(xpbd_handle* h, const MotionSource& from)
 {
     hipError_t e = launch_finish(h->stream, h->d_pos, h->d_lo, h->d_vel, h->nv, (float)h->params.dt, h->d_step, from);
@@ -922,6 +933,48 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "gs_tile_store launch");
 }
 
+// The Jacobi iterations by vertex-tile launches (jacobi_tiles.h): from one array of
+// slots to the other, or, where no tile reads another's vertices, all in one launch.
+static int enqueue_tiled_jacobi(xpbd_handle* h, int iters, bool timed, bool reset_lambda, const StepEnds& ends)
+{
+    hipStream_t s = h->stream;
+    const JacobiTilePlan& P = h->jtiles;
+    const Prediction predict = prediction(h);
+    const HitLists hits = hit_lists(h);
+    const bool con = contacts_enabled(h);
+    hipError_t e = launch_gs_tile_load(s, h->d_pos, P.args.vert, P.nslots, P.nslots, P.d[0], P.base,
+                                       ends.predict ? &predict : nullptr, ends.hits ? &hits : nullptr);
+    if (e != hipSuccess) return hip_err(h, e, "gs_tile_load launch");
+    int cur = 0;
+    for (int it = 0, inner; it < iters; it += inner) {
+        inner = P.closed ? iters : 1;
+        JacobiTileArgs A = P.args;
+        A.din = P.d[cur];
+        A.dout = P.d[1 - cur];
+        A.niter = inner;
+        A.xcd = h->xcd_map ? 1 : 0;
+        A.lam_zero = it == 0 && reset_lambda;
+        A.import = it == 0 && !reset_lambda;
+        A.lam_out = it + inner == iters;
+        if (timed) timed_begin(h);
+        e = launch_jacobi_tile(s, A, P.threads, con);
+        if (e != hipSuccess) return hip_err(h, e, "jacobi_tile launch");
+        if (timed) {
+            timed_end(h);
+            h->timed_iterations += inner;
+        }
+        cur = 1 - cur;
+    }
+    if (ends.finish) {
+        MotionSource from;
+        from.owner = P.owner;
+        from.d = P.d[cur];
+        return enqueue_finish(h, from);
+    }
+    e = launch_gs_tile_store(s, h->d_pos, P.owner, h->nv, P.d[cur]);
+    return e == hipSuccess ? XPBD_OK : hip_err(h, e, "gs_tile_store launch");
+}
+
 // Enqueue the solver iterations of one step (no predict / finish).  With
 // reset_lambda (the reference solve, XPBDSolver.hpp:66-77) the first iteration
 // starts every multiplier at zero; without it every multiplier (element,
@@ -932,6 +985,7 @@ static int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_
     TetArrays ta = tet_arrays(h);
     const bool con = contacts_enabled(h);
     hipError_t e = hipSuccess;
+    if (runs_tiled_jacobi(h, iters)) return enqueue_tiled_jacobi(h, iters, timed, reset_lambda, ends);
     if (runs_fused_jacobi(h)) {
         // fused patch Jacobi: one launch per iteration, the shared vertices' last
         // sums after the loop
@@ -1168,7 +1222,7 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda)
 // reads it, the velocity update where nothing comes between.
 static StepEnds step_ends(const xpbd_handle* h, bool detect)
 {
-    const bool tiled = runs_tiled(h, h->params.iters);
+    const bool tiled = runs_tiled(h, h->params.iters) || runs_tiled_jacobi(h, h->params.iters);
     StepEnds ends;
     ends.predict = tiled && !h->primary_residual;
     ends.hits = ends.predict && detect;

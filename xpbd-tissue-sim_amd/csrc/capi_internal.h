@@ -8,6 +8,7 @@
 #include <vector>
 
 #include "gs_tile_kernels.h"
+#include "jacobi_tile_kernels.h"
 #include "kernels.h"
 #include "mesh_tools.h"
 #include "xpbd_hip.h"
@@ -22,6 +23,16 @@ struct GsTileLaunch {
     size_t smem = 0;
     float4* d[2] = { nullptr, nullptr };   // in-step motion by slot; the second only where a group follows itself
 };
+struct JacobiTilePlan {
+    bool built = false, ready = false;   // tried; there is one
+    bool closed = false;                 // its tiles can run all iterations in one launch
+    xpbd::JacobiTileArgs args{};
+    float4* d[2] = {};                   // motions by slot, in turn
+    float4* base = nullptr;
+    const int32_t* owner = nullptr;      // vertex -> its owner's slot
+    int nslots = 0, threads = 0;
+};
+
 struct GsTilePlan {
     bool built = false;      // tried; launches is empty where no plan fits
     bool closed = false;     // one launch without copies: its tiles can run all iterations
@@ -104,6 +115,8 @@ struct xpbd_handle {
     // fused patch Jacobi (one launch per iteration, see FusedPatchArgs)
     bool fused_ok = false;           // the patch layout and the faces allow it
     bool patch_fused = false;        // in use (autotuned)
+    bool patch_tile = false;         // vertex-tile launches in use
+    xpbd::JacobiTilePlan jtiles;
     int2* d_pshare = nullptr;
     int32_t* d_pf_off = nullptr;
     int4* d_pf = nullptr;
@@ -191,6 +204,7 @@ int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes);
 // The fused-colour plan of a Gauss-Seidel handle with clusters (built once;
 // not under capture).  XPBD_OK also where no plan fits the mesh.
 int ensure_gs_tiles(xpbd_handle* h);
+int ensure_jacobi_tiles(xpbd_handle* h);
 void timed_begin(xpbd_handle* h);
 void timed_end(xpbd_handle* h);
 int collect_timing(xpbd_handle* h);

@@ -1,0 +1,147 @@
+// Builds a handle's vertex-tile Jacobi plan: how many tiles, and the device data.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <exception>
+#include <thread>
+
+#include "capi_internal.h"
+#include "jacobi_tile_kernels.h"
+#include "jacobi_tiles.h"
+
+using namespace xpbd;
+
+namespace {
+
+constexpr size_t kLds = 160 * 1024;   // of a workgroup, gfx950
+
+template <typename T>
+int room(xpbd_handle* h, T** dst, size_t n)
+{
+    void* p = nullptr;
+    int rc = dalloc_bytes(h, &p, sizeof(T) * n);
+    *dst = static_cast<T*>(p);
+    return rc;
+}
+
+template <typename D, typename T>
+int put(xpbd_handle* h, const D** dst, const std::vector<T>& v)
+{
+    char* p = nullptr;
+    int rc = room(h, &p, sizeof(T) * v.size());
+    if (rc) return rc;
+    if (!v.empty()) {
+        hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
+        if (e != hipSuccess) return hip_err(h, e, "Jacobi tile lists");
+    }
+    *dst = reinterpret_cast<const D*>(p);
+    return XPBD_OK;
+}
+
+// Tiles of a plan, 0 for a tile an instance, -1 for no plan.  us a step of 10 iterations against the
+// patch launches:
+// - an instance a tile, all iterations in a launch, while an instance's elements are
+//   one a thread: 4^3 cells 33 against 62 (22 tiles of few vertices: 57), 5^3 37
+//   against 65; 6^3 is more, 57 against 52 by tiles.
+// - else a tile a compute unit, which is all that fit side by side: 12^3 56 against
+//   76, 24^3 68 against 102, 40^3 143 against 166, beam 200x20x20 168 against 195.
+//   Of fewer than 12 vertices a tile is mostly border (12^3 with 9: 59).
+// A tile's corrections have to fit in LDS, up to some 400 vertices.  With more tiles
+// than units the border's extra elements and the second round take what is gained
+// (50^3: 246 against 246, 56^3 306 against 297): no plan.
+int tile_count(const xpbd_handle* h, int units)
+{
+    int64_t most = 0;   // elements of an instance
+    for (int i = 0; i < h->ninst; i++) most = std::max(most, h->t_off[i + 1] - h->t_off[i]);
+    if (most <= 1024) return 0;
+    const int own = std::max(12, (h->nv + units - 1) / units);
+    if (own > 420) return -1;
+    return (h->nv + own - 1) / own;
+}
+
+int make_tiles(xpbd_handle* h)
+{
+    JacobiTilePlan& P = h->jtiles;
+    if (h->variant != XPBD_VARIANT_PATCH || h->params.deterministic == 0 || h->nt <= 0) return XPBD_OK;
+    int units = 0;
+    hipError_t e = hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, h->device);
+    if (e != hipSuccess || units <= 0) return hip_err(h, e, "device attribute");
+    const int parts = tile_count(h, units);
+    if (parts < 0) return XPBD_OK;
+    std::vector<int32_t> tets(4 * (size_t)h->nt), faces(4 * (size_t)h->nf);
+    e = hipMemcpy(tets.data(), h->d_tet, sizeof(int32_t) * tets.size(), hipMemcpyDeviceToHost);
+    if (e == hipSuccess && h->nf > 0)
+        e = hipMemcpy(faces.data(), h->d_faces, sizeof(int32_t) * faces.size(), hipMemcpyDeviceToHost);
+    if (e != hipSuccess) return hip_err(h, e, "element table");
+    const JacobiMesh M{ h->nv, h->nt, h->nf, tets.data(), faces.data(), h->v_off, h->rest };
+    const int threads = h->nt < 20000 ? 1 : 8;
+    JacobiTiles J;
+    if (!build_jacobi_tiles(M, parts, threads, J) || jacobi_tile_smem(J.verts, J.slots) > kLds)
+        return XPBD_OK;
+    JacobiTileArgs A{};
+    const size_t n = J.home.size(), slots = J.vert.size();
+    float4* stream = nullptr;
+    float4* base = nullptr;
+    int rc = put(h, &A.head, J.head);
+    if (!rc) rc = put(h, &A.local, J.local);
+    if (!rc) rc = put(h, &A.home, J.home);
+    if (!rc) rc = put(h, &A.face, J.face);
+    if (!rc) rc = put(h, &A.group, J.group);
+    if (!rc) rc = put(h, &A.degree, J.degree);
+    if (!rc) rc = put(h, &A.out, J.out);
+    if (!rc) rc = put(h, &A.vert, J.vert);
+    if (!rc) rc = put(h, &P.owner, J.owner);
+    if (!rc) rc = room(h, &stream, 3 * n);
+    if (!rc) rc = room(h, &A.lam, n);
+    if (!rc) rc = room(h, &base, slots);
+    for (int i = 0; i < 2 && !rc; i++) rc = room(h, &P.d[i], slots);
+    if (rc) return rc;
+    e = launch_fill_zero(h->stream, A.lam, sizeof(float2) * n);
+    for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_fill_zero(h->stream, P.d[i], sizeof(float4) * slots);
+    if (e == hipSuccess) e = launch_jacobi_tile_fill(h->stream, tet_arrays(h), A.home, (int)n, stream);
+    if (e == hipSuccess) e = jacobi_tile_prepare();
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+    if (e != hipSuccess) return hip_err(h, e, "Jacobi tile set-up");
+    A.stream = stream;
+    A.base = base;
+    A.dlam = h->d_lam;
+    A.n = (int)n;
+    A.verts = J.verts;
+    A.slots = J.slots;
+    A.ntiles = J.ntiles;
+    A.flag = h->d_flag;
+    A.rest = h->d_rest;
+    A.lo = h->d_lo;
+    A.cp = h->d_cp;
+    A.cn = h->d_cn;
+    A.cb = h->d_cb;
+    A.clam = h->d_clam;
+    P.args = A;
+    P.base = base;
+    P.closed = J.closed;
+    P.nslots = (int)slots;
+    P.threads = std::min(1024, std::max(64, (J.tets + 63) / 64 * 64));
+    P.ready = true;
+    return XPBD_OK;
+}
+
+}  // namespace
+
+int xpbd::ensure_jacobi_tiles(xpbd_handle* h)
+{
+    if (h->jtiles.built) return XPBD_OK;
+    const size_t kept = h->allocs.size();
+    int rc;
+    try {
+        rc = make_tiles(h);
+    } catch (const std::exception&) {   // host memory
+        rc = set_err(h, XPBD_E_NOMEM, "Jacobi tile plan");
+    }
+    if (rc) {   // the handle goes on with its other launch shapes
+        for (; h->allocs.size() > kept; h->allocs.pop_back()) (void)hipFree(h->allocs.back());
+        h->jtiles = JacobiTilePlan{};
+        (void)hipGetLastError();
+    }
+    h->jtiles.built = true;
+    return rc;
+}
