@@ -24,6 +24,7 @@ thread_local std::string g_create_error;
 // largest patch count for which a patch Jacobi handle starts on the fused
 // one-launch iteration before any autotuning
 constexpr int kFusedDefaultMaxPatches = 256;
+constexpr size_t kReadPiece = 480 * 1024;   // bytes of a state that are packed while the last ones are copied
 }
 
 namespace xpbd {
@@ -479,6 +480,17 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
     rc |= dalloc(h, &h->d_cn, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_cb, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_clam, nf);
+    // state readers: two pieces of pinned memory
+    if (rc == XPBD_OK) {
+        h->read_bytes = std::min<size_t>(kReadPiece, 3 * sizeof(double) * (size_t)nv);
+        hipError_t re = hipHostMalloc(reinterpret_cast<void**>(&h->h_read), 2 * h->read_bytes, hipHostMallocDefault);
+        for (hipEvent_t& ev : h->read_done)
+            if (re == hipSuccess) re = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (re != hipSuccess) {
+            (void)hipGetLastError();
+            rc = XPBD_E_NOMEM;
+        }
+    }
     // Gauss-Seidel contacts: room for what a solve's first contact pass leaves to
     // the later ones (without it each gathers for itself)
     if (rc == XPBD_OK && P->solver == XPBD_SOLVER_GS_COLORED && nf > 0) {
@@ -729,6 +741,9 @@ extern "C" int xpbd_destroy(xpbd_handle* h)
         if (ev.second) (void)hipEventDestroy(ev.second);
     }
     for (void* p : h->allocs) (void)hipFree(p);
+    if (h->h_read) (void)hipHostFree(h->h_read);
+    for (hipEvent_t ev : h->read_done)
+        if (ev) (void)hipEventDestroy(ev);
     destroy_learned(h);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -1361,18 +1376,40 @@ int download_f4(xpbd_handle* h, std::vector<float4>& hu, const float4* src, size
 }
 }  // namespace xpbd
 
-// position = rest + base + low part + in-step motion (zero between steps)
-static int positions_range(xpbd_handle* h, int64_t v0, int64_t v1, double* out)
+// position = rest + base + low part + in-step motion (zero between steps), or the
+// velocity, of vertices [v0, v1).  The kernel packs a caller's 12 or 24 bytes a vertex
+// (the records hold 48) straight into pinned host memory, and the host copies them
+// on, piece by piece while the next piece is packed.  us for positions in FP64 and
+// velocities, by copies of the records before: 4^3 cells 47 and 24, now 14 each; 28^3
+// 128 and 42, now 36 each; beam of 88,641 vertices 492 and 150, now 94 and 89.  Packed
+// into device memory and copied from there: 14, 49 and 151 each.
+static int read_state(xpbd_handle* h, bool velocities, int64_t v0, int64_t v1, bool f32, void* out)
 {
-    std::vector<float4> hp, hl;
-    int rc = download_f4(h, hp, h->d_pos, 2 * (size_t)h->nv);
-    if (!rc) rc = download_f4(h, hl, h->d_lo, h->nv);
-    if (rc) return rc;
-    for (int64_t i = v0; i < v1; i++) {
-        const float4 b = hp[2 * i], d = hp[2 * i + 1], l = hl[i];
-        out[3 * (i - v0) + 0] = h->rest[3 * i + 0] + ((double)b.x + (double)l.x + (double)d.x);
-        out[3 * (i - v0) + 1] = h->rest[3 * i + 1] + ((double)b.y + (double)l.y + (double)d.y);
-        out[3 * (i - v0) + 2] = h->rest[3 * i + 2] + ((double)b.z + (double)l.z + (double)d.z);
+    const size_t per = 3 * (f32 ? sizeof(float) : sizeof(double));
+    const int64_t piece = (int64_t)(h->read_bytes / per);
+    std::lock_guard<std::mutex> lock(h->read_mutex);
+    char *dst = static_cast<char*>(out), *prev = nullptr;
+    size_t waiting = 0;   // bytes of the piece before, on their way into prev
+    hipError_t e = hipSuccess;
+    for (int64_t v = v0, c = 0; e == hipSuccess && (v < v1 || waiting); v += piece, c++) {
+        char* const buf = h->h_read + (c & 1) * h->read_bytes;
+        const int64_t n = std::min(piece, v1 - v);
+        if (n > 0) {
+            e = launch_read_state(h->stream, velocities ? nullptr : h->d_rest, h->d_pos, h->d_lo, h->d_vel, (int)v, (int)n,
+                                  f32, buf);
+            if (e == hipSuccess) e = hipEventRecord(h->read_done[c & 1], h->stream);
+        }
+        if (e == hipSuccess && waiting) {
+            e = hipEventSynchronize(h->read_done[1 - (c & 1)]);
+            if (e == hipSuccess) std::memcpy(dst, prev, waiting);
+            dst += waiting;
+        }
+        waiting = n > 0 ? per * (size_t)n : 0;
+        prev = buf;
+    }
+    if (e != hipSuccess) {
+        (void)hipStreamSynchronize(h->stream);
+        return hip_err(h, e, "state read");
     }
     return XPBD_OK;
 }
@@ -1380,24 +1417,20 @@ static int positions_range(xpbd_handle* h, int64_t v0, int64_t v1, double* out)
 extern "C" int xpbd_get_positions(xpbd_handle* h, double* out)
 {
     if (!h || !out) return h ? set_err(h, XPBD_E_INVALID_ARG, "out is NULL") : XPBD_E_INVALID_ARG;
-    return positions_range(h, 0, h->nv, out);
+    return read_state(h, false, 0, h->nv, false, out);
 }
 
 extern "C" int xpbd_get_positions_f32(xpbd_handle* h, float* out)
 {
     if (!h || !out) return h ? set_err(h, XPBD_E_INVALID_ARG, "out is NULL") : XPBD_E_INVALID_ARG;
-    std::vector<double> tmp(3 * (size_t)h->nv);
-    int rc = positions_range(h, 0, h->nv, tmp.data());
-    if (rc) return rc;
-    for (size_t i = 0; i < tmp.size(); i++) out[i] = (float)tmp[i];
-    return XPBD_OK;
+    return read_state(h, false, 0, h->nv, true, out);
 }
 
 extern "C" int xpbd_batch_get_positions(xpbd_batch* b, int32_t instance, double* out)
 {
     if (!b || !out) return b ? set_err(b, XPBD_E_INVALID_ARG, "out is NULL") : XPBD_E_INVALID_ARG;
     if (instance < 0 || instance >= b->ninst) return set_err(b, XPBD_E_INVALID_ARG, "instance out of range");
-    return positions_range(b, b->v_off[instance], b->v_off[instance + 1], out);
+    return read_state(b, false, b->v_off[instance], b->v_off[instance + 1], false, out);
 }
 
 extern "C" int xpbd_batch_step(xpbd_batch* b, int32_t nsteps)
@@ -1415,15 +1448,7 @@ extern "C" int xpbd_batch_num_instances(xpbd_batch* b, int32_t* out)
 extern "C" int xpbd_get_velocities(xpbd_handle* h, double* out)
 {
     if (!h || !out) return h ? set_err(h, XPBD_E_INVALID_ARG, "out is NULL") : XPBD_E_INVALID_ARG;
-    std::vector<float4> hv;
-    int rc = download_f4(h, hv, h->d_vel, h->nv);
-    if (rc) return rc;
-    for (int i = 0; i < h->nv; i++) {
-        out[3 * (size_t)i] = hv[i].x;
-        out[3 * (size_t)i + 1] = hv[i].y;
-        out[3 * (size_t)i + 2] = hv[i].z;
-    }
-    return XPBD_OK;
+    return read_state(h, true, 0, h->nv, false, out);
 }
 
 extern "C" int xpbd_set_state(xpbd_handle* h, const double* x, const double* v)

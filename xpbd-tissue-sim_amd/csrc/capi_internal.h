@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -81,6 +82,12 @@ struct xpbd_handle {
     // are one run: fci_off[c * (ninst + 1) + i] is where instance i's faces of
     // colour c start (i = ninst: the colour's end)
     std::vector<int32_t> fci_off;
+    // what the state's readers are given, in two pieces of pinned memory; for one
+    // reader at a time
+    std::mutex read_mutex;
+    char* h_read = nullptr;
+    size_t read_bytes = 0;   // of a piece
+    hipEvent_t read_done[2] = {};
     xpbd::ContactWork contact_work;   // Gauss-Seidel; cap 0: none
     std::vector<xpbd::SdfDev> sdf_host;
     bool sdf_active = false;

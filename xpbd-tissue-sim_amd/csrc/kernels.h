@@ -63,6 +63,10 @@ struct MotionSource {
 };
 hipError_t launch_finish(hipStream_t s, float4* pos, float4* lo, float4* vel, int nv, float dt,
                          unsigned long long* step_counter, const MotionSource& from = MotionSource{});
+// 3 n numbers a caller reads: positions of vertices v0.., or with rest null their
+// velocities, in FP64 or rounded to FP32.
+hipError_t launch_read_state(hipStream_t s, const double* rest, const float4* pos, const float4* lo, const float4* vel,
+                             int v0, int n, bool f32, void* out);
 // Deterministic Jacobi: contacts into per-face slots, then a per-vertex gather in
 // face-slot order; local passes into per-element slots, then a per-vertex gather
 // in solver-position order.

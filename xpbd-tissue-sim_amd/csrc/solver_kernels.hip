@@ -2259,6 +2259,25 @@ __global__ __launch_bounds__(kBlock) void k_jacobi_local(TetArrays ta, const int
 
 inline unsigned nblk(long long n, int b) { return (unsigned)((n + b - 1) / b); }
 
+// Positions (rest + ((base + low) + in-step motion), in FP64, rounded once for T =
+// float) or, without rest, velocities of vertices v0.., packed as the caller gets them.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_read_state(const double* __restrict__ rest, const float4* __restrict__ pos,
+                                                      const float4* __restrict__ lo, const float4* __restrict__ vel,
+                                                      int v0, int n, T* __restrict__ out)
+{
+    const int i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= 3 * n) return;
+    const int v = v0 + i / 3, k = i % 3;
+    auto comp = [&](const float4& x) { return k == 0 ? x.x : k == 1 ? x.y : x.z; };
+    if (!rest) {
+        out[i] = (T)comp(vel[v]);
+        return;
+    }
+    const float b = comp(pos[2 * (size_t)v]), d = comp(pos[2 * (size_t)v + 1]), l = comp(lo[v]);
+    out[i] = (T)(rest[3 * (size_t)v + k] + ((double)b + (double)l + (double)d));
+}
+
 }  // namespace
 
 hipError_t launch_attach_gs(hipStream_t s, const int* av, const double* ap, double* alam, const double* rest,
@@ -2329,6 +2348,19 @@ hipError_t launch_finish(hipStream_t s, float4* pos, float4* lo, float4* vel, in
 {
     hipLaunchKernelGGL(k_finish, dim3(nblk(nv > 0 ? nv : 1, kBlock)), dim3(kBlock), 0, s, pos, lo, vel, nv, dt,
                        step_counter, from);
+    return hipGetLastError();
+}
+
+hipError_t launch_read_state(hipStream_t s, const double* rest, const float4* pos, const float4* lo, const float4* vel,
+                             int v0, int n, bool f32, void* out)
+{
+    if (n <= 0) return hipSuccess;
+    const dim3 g(nblk(3ll * n, kBlock));
+    if (f32)
+        hipLaunchKernelGGL(k_read_state<float>, g, dim3(kBlock), 0, s, rest, pos, lo, vel, v0, n, static_cast<float*>(out));
+    else
+        hipLaunchKernelGGL(k_read_state<double>, g, dim3(kBlock), 0, s, rest, pos, lo, vel, v0, n,
+                           static_cast<double*>(out));
     return hipGetLastError();
 }
 
