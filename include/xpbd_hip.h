@@ -351,9 +351,9 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
 /* The patch block value of the vertex-tile Jacobi launches, the untuned default
  * where the mesh's size suits them: a workgroup owns a set of vertices and
  * projects every element around them, so that one launch is an iteration and a
- * vertex's corrections are summed in one place, in solver order (the sums of the
- * other patch launches in another grouping).  Deterministic mode without
- * attachments; otherwise such a handle runs the other patch launches. */
+ * vertex's corrections are summed in one place (in the groups of the other patch
+ * launches: the same results).  Deterministic mode without attachments; otherwise
+ * such a handle runs the other patch launches. */
 #define XPBD_PATCH_TILE 2
 /* Batch handles are also plain handles: xpbd_step, xpbd_destroy, ... apply. */
 

@@ -1,7 +1,8 @@
 // Runs the vertex-tile Jacobi plan of a mesh on the CPU and compares it with the
 // plain iteration.  Elements and faces give each of their vertices a hash of all
 // their vertices' values, summed as integers.
-//   jacobi_tiles_check NX NY NZ INSTANCES PARTS
+// Each is added once, contacts by patch (LATE 0) or at the end.
+//   jacobi_tiles_check NX NY NZ INSTANCES PARTS LATE
 #include <algorithm>
 #include <cstdint>
 #include <cstdio>
@@ -29,10 +30,12 @@ static uint64_t part(uint64_t kind, int item, const uint64_t* v, int n, int k)
 
 int main(int argc, char** argv)
 {
-    if (argc != 6) return 2;
+    if (argc != 7) return 2;
+    const int patch = 16;
+    const bool late = atoi(argv[6]) != 0;
     const int nx = atoi(argv[1]), ny = atoi(argv[2]), nz = atoi(argv[3]), ninst = atoi(argv[4]), parts = atoi(argv[5]);
     std::vector<double> x;
-    std::vector<int32_t> t, faces;
+    std::vector<int32_t> t, faces, face_patch;
     std::vector<int64_t> v_off(1, 0);
     for (int i = 0; i < ninst; i++) {   // instances of different sizes, all at the origin
         std::vector<double> xi;
@@ -43,13 +46,16 @@ int main(int argc, char** argv)
         for (int32_t v : ti) t.push_back(v + v0);
         x.insert(x.end(), xi.begin(), xi.end());
         v_off.push_back((int64_t)x.size() / 3);
-        for (size_t k = 0; k + 4 <= ti.size(); k += 12)   // any triangles will do
+        const int e0 = (int)(t.size() - ti.size()) / 4;
+        for (size_t k = 0; k + 4 <= ti.size(); k += 12) {   // any triangles will do
             for (int32_t v : { ti[k] + v0, ti[k + 1] + v0, ti[k + 2] + v0, i }) faces.push_back(v);
+            if (!late) face_patch.push_back((e0 + (int)k / 4) / patch);
+        }
     }
     x.insert(x.end(), { 9.0, 9.0, 9.0 });   // a vertex of no element
     v_off.back()++;
     const int nv = (int)(x.size() / 3), nt = (int)(t.size() / 4), nf = (int)(faces.size() / 4);
-    const JacobiMesh M{ nv, nt, nf, t.data(), faces.data(), v_off, x };
+    const JacobiMesh M{ nv, nt, nf, t.data(), faces.data(), patch, face_patch, v_off, x };
     JacobiTiles J;
     if (!build_jacobi_tiles(M, parts, 4, J)) return puts("no plan"), 1;
     std::vector<uint64_t> ref(nv), sum(nv);
@@ -102,11 +108,27 @@ int main(int argc, char** argv)
                 if (it == 0) kept_face[a[0] >> 1] += a[0] & 1;
             }
             for (int o = 0; o < h[JacobiTiles::OWN]; o++) {
-                const int deg = J.degree[h[JacobiTiles::V0] + o];
+                const uint32_t* q = &J.sums[JacobiTiles::kSums * (size_t)(h[JacobiTiles::V0] + o)];
+                const uint64_t end = q[0] | (uint64_t)q[1] << 32, con = q[2] | (uint64_t)q[3] << 32;
                 const int32_t* gr = &J.group[2 * (size_t)(h[JacobiTiles::G0] + o / 64)];
-                uint64_t s = 0;
-                for (int e = 0; e < (deg & 0xffff); e++) s += red[gr[0] + 64 * e + o % 64];
-                for (int e = 0; e < deg >> 16; e++) s += red[gr[1] + 64 * e + o % 64];
+                uint64_t s = 0, part = 0;
+                uint32_t f = 0;
+                auto contacts = [&] {
+                    for (bool more = true; more; f++) {
+                        s += red[gr[1] + 64 * f + o % 64];
+                        more = !(q[5] >> f & 1);
+                    }
+                };
+                for (uint32_t e = 0; e < (q[4] & 0xffff); e++) {
+                    part += red[gr[0] + 64 * e + o % 64];
+                    if (con >> e & 1) contacts();
+                    if (end >> e & 1) {
+                        s += part;
+                        part = 0;
+                    }
+                }
+                if (late && q[4] >> 16) contacts();
+                bad += part != 0 || f != q[4] >> 16;
                 own[o] = mix(l[o] + s);
             }
             for (int k = h[JacobiTiles::O0]; k < h[JacobiTiles::O0] + h[JacobiTiles::NO]; k++)

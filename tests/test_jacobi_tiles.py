@@ -22,8 +22,9 @@ def check(tmp_path_factory):
 # nx ny nz, instances, tiles (0: one an instance)
 @pytest.mark.parametrize("case", ["1 1 1 1 1", "1 1 1 1 9", "6 5 7 1 0", "9 9 9 1 16", "12 12 12 1 256", "40 3 5 1 9",
                                   "4 6 3 5 6", "4 6 3 5 0", "4 6 3 5 60", "20 17 19 1 64", "3 3 3 1 1000"])
-def test_tiles_give_the_plain_iteration(check, case):
-    r = subprocess.run([str(check)] + case.split(), capture_output=True, text=True, timeout=60)
+@pytest.mark.parametrize("late", [0, 1], ids=["contacts by patch", "contacts last"])
+def test_tiles_give_the_plain_iteration(check, case, late):
+    r = subprocess.run([str(check)] + case.split() + [str(late)], capture_output=True, text=True, timeout=60)
     print(case, "->", r.stdout.strip())
     assert r.returncode == 0, r.stdout + r.stderr
     if case.split()[4] == "0":   # an instance a tile: nothing runs twice

@@ -629,6 +629,7 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         // (measured: 24 patches), the three-launch one on large meshes (1,875 and
         // 4,116 patches); xpbd_autotune times both
         h->patch_fused = ok && Pt.npatch <= kFusedDefaultMaxPatches;
+        if (h->patch_fused) h->face_patch = fpatch;
     }
     h->sdf_host.assign(n, SdfDev{});
     for (auto& s : h->sdf_host) s.quat[3] = 1.0;

@@ -123,6 +123,7 @@ struct xpbd_handle {
     bool fused_ok = false;           // the patch layout and the faces allow it
     bool patch_fused = false;        // in use (autotuned)
     bool patch_tile = false;         // vertex-tile launches in use
+    std::vector<int32_t> face_patch; // per face slot, where the patch of an element adds its contact (fused default)
     xpbd::JacobiTilePlan jtiles;
     int2* d_pshare = nullptr;
     int32_t* d_pf_off = nullptr;

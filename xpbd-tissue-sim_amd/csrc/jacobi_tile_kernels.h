@@ -14,7 +14,7 @@ struct JacobiTileArgs {
     const int* home;          // per tile element
     const int4* face;         // per tile face
     const int2* group;
-    const int* degree;        // per slot
+    const uint4* sums;        // per slot, two each
     const int2* out;
     float2* lam;              // per tile element
     float2* dlam;             // solver order
@@ -29,6 +29,7 @@ struct JacobiTileArgs {
     int import;               // they are dlam's
     int lam_out;              // the last iteration also writes dlam
     // contacts
+    int late;                 // added after all elements
     const int* flag;
     const double *rest, *cp, *cn, *cb;
     const float4* lo;

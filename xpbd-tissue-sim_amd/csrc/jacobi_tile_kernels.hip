@@ -18,6 +18,75 @@ struct TileTet {
     float2 l;
 };
 
+// an own vertex's JacobiTiles::sums and its group
+struct SumOf {
+    uint4 m, c;
+    int2 g;
+};
+
+constexpr int kAhead = 8;   // corrections read together
+
+// The elements' corrections of one component of a vertex, partial sums by patch; CON:
+// with the contacts' partial sums c, in their order.  What is read past the last
+// correction follows the last end of a partial sum, so it goes nowhere.
+template <bool CON>
+__device__ __forceinline__ float sum_elements(const SumOf& q, const float* r, const float* c)
+{
+    const int nt = q.c.x & 0xffffu;
+    float total = 0.f, s = 0.f;
+    int nc = 0;
+    uint32_t end = q.m.x, con = q.m.z;
+    for (int e0 = 0; e0 < nt; e0 += kAhead) {
+        if (e0 == 32) {
+            end = q.m.y;
+            con = q.m.w;
+        }
+        float v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) v[u] = r[q.g.x + 64 * (e0 + u)];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) {
+            s += v[u];
+            if (CON && (con >> u & 1u)) s += c[64 * nc++];
+            const bool ends = end >> u & 1u;
+            total = ends ? total + s : total;
+            s = ends ? 0.f : s;
+        }
+        end >>= kAhead;
+        con >>= kAhead;
+    }
+    return total;
+}
+
+// The same with contacts: their partial sums go to the front of their slots.  Sums of
+// nothing but zeros (no contact is active) need not be added.
+__device__ __forceinline__ float sum_contacts(const SumOf& q, float* r, int late)
+{
+    const int nf = q.c.x >> 16;
+    float* const c = r + q.g.y;
+    float t = 0.f, all = 0.f;
+    int nc = 0;
+    for (int f0 = 0; f0 < nf; f0 += kAhead) {
+        float v[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) v[u] = c[64 * min(f0 + u, nf - 1)];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++)
+            if (f0 + u < nf) {
+                t += v[u];
+                if (q.c.y >> (f0 + u) & 1u) {
+                    c[64 * nc++] = t;
+                    all = t != 0.f ? t : all;
+                    t = 0.f;
+                }
+            }
+    }
+    if (!__any(all != 0.f)) return sum_elements<false>(q, r, nullptr);
+    if (!late) return sum_elements<true>(q, r, c);
+    const float total = sum_elements<false>(q, r, nullptr);
+    return nf > 0 ? total + c[0] : total;
+}
+
 __device__ __forceinline__ void load_tile_tet(const JacobiTileArgs& A, int i, bool first, TileTet& t)
 {
     t.idx = A.local[i];
@@ -41,7 +110,7 @@ __device__ __forceinline__ void project_tile_tet(TileTet& t, const float4* lb, c
         dd[3 * j] = d.x, dd[3 * j + 1] = d.y, dd[3 * j + 2] = d.z;
         w[j] = b.w;
     }
-    project_tet_split<float>(bb, dd, w, t.q, t.atD, t.atH, t.gm, l, dx);
+    project_tet_split<float, true>(bb, dd, w, t.q, t.atD, t.atH, t.gm, l, dx);
     t.l = make_float2(l[0], l[1]);
 #pragma unroll
     for (int j = 0; j < 4; j++)
@@ -94,7 +163,9 @@ __device__ __forceinline__ void project_tile_face(const JacobiTileArgs& A, int4 
 // instructions.  Tried there: the next element's data in flight while one is
 // projected (copies of 20 registers: 184 us a step against 171), 512 threads and
 // tiles of half the size (173), spare slots instead of branches for other tiles'
-// vertices (no gain, more LDS writes).
+// vertices (no gain, more LDS writes).  The sums keep the patch launches' grouping,
+// and so their bits, for 0.2 us an iteration: Jacobi under contact amplifies rounding
+// tenfold in ten steps.
 template <bool CON>
 __global__ __launch_bounds__(kTileThreads) void k_jacobi_tile(JacobiTileArgs A)
 {
@@ -112,8 +183,17 @@ __global__ __launch_bounds__(kTileThreads) void k_jacobi_tile(JacobiTileArgs A)
         lb[i] = A.base[v0 + i];
         ld[i] = A.din[v0 + i];
     }
-    __syncthreads();
+    // how a thread's first sum is grouped
     const int width = (own + 63) & ~63;
+    auto sum_of = [&](int o) {
+        return SumOf{ A.sums[2 * (size_t)(v0 + o)], A.sums[2 * (size_t)(v0 + o) + 1], A.group[g0 + (o >> 6)] };
+    };
+    SumOf mine{};
+    {
+        const int o = tid - ((tid >= width) + (tid >= 2 * width)) * width;
+        if (o < own) mine = sum_of(o);
+    }
+    __syncthreads();
     for (int it = 0; it < A.niter; it++) {
         const bool first = it == 0, last = it == A.niter - 1;
         for (int i = tid; i < nt; i += nthreads) {
@@ -139,20 +219,15 @@ __global__ __launch_bounds__(kTileThreads) void k_jacobi_tile(JacobiTileArgs A)
             for (int i = tid; i < nf; i += nthreads)
                 project_tile_face(A, A.face[f0 + i], v0, first && A.lam_zero, lb, ld, red);
         __syncthreads();
-        // a thread sums one component of one vertex, the elements' corrections in
-        // solver order, then the contacts'
+        // a thread sums one component of one vertex, grouped as the patch launches do
         for (int x = tid; x < 3 * width; x += nthreads) {
-            const int k = x / width, o = x - k * width;
+            const int k = (x >= width) + (x >= 2 * width), o = x - k * width;
             if (o >= own) continue;
-            const int deg = A.degree[v0 + o];
-            const int2 g = A.group[g0 + (o >> 6)];
-            const float* r = red + k * A.slots + (o & 63);
-            float s = 0.f;
-#pragma unroll 8
-            for (int e = 0; e < (deg & 0xffff); e++) s += r[g.x + 64 * e];
-            if (CON)
-                for (int e = 0; e < (deg >> 16); e++) s += r[g.y + 64 * e];
-            reinterpret_cast<float*>(ld)[4 * o + k] += s;
+            const SumOf q = x == tid ? mine : sum_of(o);
+            float total;
+            if constexpr (CON) total = sum_contacts(q, red + k * A.slots + (o & 63), A.late);
+            else total = sum_elements<false>(q, red + k * A.slots + (o & 63), nullptr);
+            reinterpret_cast<float*>(ld)[4 * o + k] += total;
         }
         __syncthreads();
     }
@@ -179,7 +254,8 @@ __global__ __launch_bounds__(256) void k_jacobi_tile_fill(TetArrays ta, const in
 
 }  // namespace
 
-size_t jacobi_tile_smem(int verts, int slots) { return 32 * (size_t)verts + 12 * (size_t)slots; }
+// with the room that a vertex's last reads may run into
+size_t jacobi_tile_smem(int verts, int slots) { return 32 * (size_t)verts + 12 * (size_t)slots + 4 * 64 * kAhead; }
 
 hipError_t jacobi_tile_prepare()
 {

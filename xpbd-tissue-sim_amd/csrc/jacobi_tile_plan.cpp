@@ -41,10 +41,10 @@ int put(xpbd_handle* h, const D** dst, const std::vector<T>& v)
 // Tiles of a plan, 0 for a tile an instance, -1 for no plan.  us a step of 10 iterations against the
 // patch launches:
 // - an instance a tile, all iterations in a launch, while an instance's elements are
-//   one a thread: 4^3 cells 33 against 62 (22 tiles of few vertices: 57), 5^3 37
-//   against 65; 6^3 is more, 57 against 52 by tiles.
+//   one a thread: 4^3 cells 33 against 61 (tiles of few vertices: 57), 5^3 39 against
+//   65; 6^3 is more, a tile 57 either way.
 // - else a tile a compute unit, which is all that fit side by side: 12^3 56 against
-//   76, 24^3 68 against 102, 40^3 143 against 166, beam 200x20x20 168 against 195.
+//   75, 24^3 67 against 103, 40^3 147 against 167, beam 200x20x20 172 against 195.
 //   Of fewer than 12 vertices a tile is mostly border (12^3 with 9: 59).
 // A tile's corrections have to fit in LDS, up to some 400 vertices.  With more tiles
 // than units the border's extra elements and the second round take what is gained
@@ -73,7 +73,8 @@ int make_tiles(xpbd_handle* h)
     if (e == hipSuccess && h->nf > 0)
         e = hipMemcpy(faces.data(), h->d_faces, sizeof(int32_t) * faces.size(), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_err(h, e, "element table");
-    const JacobiMesh M{ h->nv, h->nt, h->nf, tets.data(), faces.data(), h->v_off, h->rest };
+    const JacobiMesh M{ h->nv,        h->nt,    h->nf, tets.data(), faces.data(), jacobi_patch_size(),
+                        h->face_patch, h->v_off, h->rest };
     const int threads = h->nt < 20000 ? 1 : 8;
     JacobiTiles J;
     if (!build_jacobi_tiles(M, parts, threads, J) || jacobi_tile_smem(J.verts, J.slots) > kLds)
@@ -87,7 +88,7 @@ int make_tiles(xpbd_handle* h)
     if (!rc) rc = put(h, &A.home, J.home);
     if (!rc) rc = put(h, &A.face, J.face);
     if (!rc) rc = put(h, &A.group, J.group);
-    if (!rc) rc = put(h, &A.degree, J.degree);
+    if (!rc) rc = put(h, &A.sums, J.sums);
     if (!rc) rc = put(h, &A.out, J.out);
     if (!rc) rc = put(h, &A.vert, J.vert);
     if (!rc) rc = put(h, &P.owner, J.owner);
@@ -109,6 +110,7 @@ int make_tiles(xpbd_handle* h)
     A.verts = J.verts;
     A.slots = J.slots;
     A.ntiles = J.ntiles;
+    A.late = h->face_patch.empty();
     A.flag = h->d_flag;
     A.rest = h->d_rest;
     A.lo = h->d_lo;

@@ -72,7 +72,8 @@ void incidence(int nv, int n, int per, int stride, const int32_t* items, std::ve
 
 // One tile's lists, before its place among the others is known.
 struct Tile {
-    std::vector<int32_t> vert, home, face, group, degree;
+    std::vector<int32_t> vert, home, face, group;
+    std::vector<uint32_t> sums;
     std::vector<uint16_t> local;
     int own = 0, slots = 0;
     bool fits = true;
@@ -108,8 +109,11 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
     std::vector<Tile> tiles(J.ntiles);
     std::atomic<int> next{ 0 };
     std::atomic<bool> bad{ false };
+    auto patch_of = [&](int face) { return M.face_patch.empty() ? 0 : M.face_patch[face]; };
+    auto by_patch = [&](int f, int g) { return patch_of(f) != patch_of(g) ? patch_of(f) < patch_of(g) : f < g; };
     auto work = [&] {
         try {
+            std::vector<int32_t> mine;
             std::vector<int32_t> seen(nv, -1), place(nv, 0), taken(M.nt, -1), used, elements, faces;
             for (int t; (t = next++) < J.ntiles && !bad;) {
                 Tile& L = tiles[t];
@@ -131,7 +135,7 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
                     faces.insert(faces.end(), flist.begin() + foff[v], flist.begin() + foff[v + 1]);
                 }
                 std::sort(elements.begin(), elements.end());
-                std::sort(faces.begin(), faces.end());
+                std::sort(faces.begin(), faces.end(), by_patch);
                 faces.erase(std::unique(faces.begin(), faces.end()), faces.end());
                 for (int i = 0; i < L.own; i++) {
                     seen[L.vert[i]] = t;
@@ -146,20 +150,42 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
                     return place[v];
                 };
                 const int groups = (L.own + 63) / 64;
-                L.degree.assign(L.own, 0);
+                L.sums.assign(JacobiTiles::kSums * (size_t)L.own, 0);
                 L.group.assign(2 * (size_t)groups, 0);
                 for (int g = 0; g < groups; g++) {
                     int td = 0, fd = 0;
                     for (int i = 64 * g; i < std::min(L.own, 64 * g + 64); i++) {
                         const int v = L.vert[i];
-                        td = std::max(td, toff[v + 1] - toff[v]);
-                        fd = std::max(fd, foff[v + 1] - foff[v]);
-                        L.degree[i] = (toff[v + 1] - toff[v]) | (foff[v + 1] - foff[v]) << 16;
+                        const int nt = toff[v + 1] - toff[v], nf = foff[v + 1] - foff[v];
+                        td = std::max(td, nt);
+                        fd = std::max(fd, nf);
+                        if (nt > 64 || nf > 32) {
+                            L.fits = false;
+                            continue;
+                        }
+                        const int32_t* te = &tlist[toff[v]];
+                        mine.assign(flist.begin() + foff[v], flist.begin() + foff[v + 1]);
+                        std::sort(mine.begin(), mine.end(), by_patch);
+                        uint64_t end = 0, con = 0;
+                        uint32_t fend = 0;
+                        for (int k = 0; k < nt; k++) {
+                            const int p = te[k] / M.patch_size;
+                            if (k + 1 < nt && te[k + 1] / M.patch_size == p) continue;
+                            end |= 1ull << k;
+                            for (int f : mine)
+                                if (!M.face_patch.empty() && patch_of(f) == p) con |= 1ull << k;
+                        }
+                        for (int k = 0; k < nf; k++)
+                            if (k + 1 == nf || patch_of(mine[k + 1]) != patch_of(mine[k])) fend |= 1u << k;
+                        uint32_t* q = &L.sums[JacobiTiles::kSums * (size_t)i];
+                        q[0] = (uint32_t)end, q[1] = (uint32_t)(end >> 32);
+                        q[2] = (uint32_t)con, q[3] = (uint32_t)(con >> 32);
+                        q[4] = (uint32_t)nt | (uint32_t)nf << 16;
+                        q[5] = fend;
                     }
                     L.group[2 * (size_t)g] = L.slots;
                     L.group[2 * (size_t)g + 1] = L.slots + 64 * td;
                     L.slots += 64 * (td + fd);
-                    L.fits = L.fits && td < 0x8000 && fd < 0x8000;
                 }
                 // corrections in the order of the items, vertex by vertex
                 used.assign(2 * (size_t)L.own, 0);
@@ -224,7 +250,7 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
         nout += L.vert.size();   // an entry a slot that reads
     }
     J.vert.reserve(v0);
-    J.degree.reserve(v0);
+    J.sums.reserve(JacobiTiles::kSums * v0);
     J.local.reserve(8 * nt);
     J.home.reserve(nt);
     J.out.reserve(2 * nout);
@@ -249,8 +275,8 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
         J.home.insert(J.home.end(), L.home.begin(), L.home.end());
         J.face.insert(J.face.end(), L.face.begin(), L.face.end());
         J.group.insert(J.group.end(), L.group.begin(), L.group.end());
-        J.degree.insert(J.degree.end(), L.degree.begin(), L.degree.end());
-        J.degree.resize(J.vert.size(), 0);
+        J.sums.insert(J.sums.end(), L.sums.begin(), L.sums.end());
+        J.sums.resize(JacobiTiles::kSums * J.vert.size(), 0);
     }
     return true;
 }

@@ -15,6 +15,8 @@ struct JacobiMesh {
     int nv, nt, nf;
     const int32_t* tets;    // 4 vertices an element, solver order
     const int32_t* faces;   // 4 ints a face slot: vertices, instance
+    int patch_size;
+    const std::vector<int32_t>& face_patch;   // per face slot; empty: contacts at the end
     const std::vector<int64_t>& v_off;   // vertices by instance
     const std::vector<double>& rest;     // 3 a vertex
 };
@@ -34,13 +36,16 @@ struct JacobiTiles {
     std::vector<int32_t> face;       // per tile face: 2 * face slot + as above, vertices 0 | 1 << 16, vertex 2 |
                                      // correction slot 0 << 16, slots 1 | 2 << 16
     std::vector<int32_t> group;      // per 64 own vertices: first correction slot of elements, of faces
-    std::vector<int32_t> degree;     // per slot: an own vertex's elements | faces << 16
+    // per slot, of an own vertex: its elements' ends of partial sums (64 bits), which of these ends have contacts
+    // to add (64), elements | faces << 16, its faces' ends of partial sums, 2 unused
+    static constexpr int kSums = 8;
+    std::vector<uint32_t> sums;
     std::vector<int32_t> out;        // own vertex, slot that reads it
     std::vector<int32_t> owner;      // vertex -> its owner's slot
 };
 
 // parts <= 0: a tile an instance.  threads: to build with.  False if a tile is too
-// large for its 16-bit numbers.
+// large for its 16-bit numbers, or a vertex has more than 64 elements or 32 faces.
 bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles& J);
 
 }  // namespace xpbd

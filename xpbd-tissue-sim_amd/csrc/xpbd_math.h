@@ -157,7 +157,9 @@ XPBD_HD void constraint_gradients(const R* F, const R* Q, R CD, R J, R* gD, R* g
 //   atD/atH compliance divided by dt^2 (alpha tilde)
 //   lam[2]  multipliers, updated in place
 //   dx[12]  position corrections for the four vertices
-template <typename R>
+//   LAM_FMA the multipliers' sums rounded once, wherever the compiler may not see
+//           that it can (it does in straight-line code)
+template <typename R, bool LAM_FMA = false>
 XPBD_HD void project_tet_F(const R* F, const R* w, const R* Q, R atD, R atH, R gamma,
                            R* lam, R* dx)
 {
@@ -185,10 +187,15 @@ XPBD_HD void project_tet_F(const R* F, const R* w, const R* Q, R atD, R atH, R g
     // projection is then skipped instead of dividing by it
     const R det = A00 * A11 - A01 * A01;
     const R inv_det = det > R(0) ? xrcp<R>(det) : R(0);
-    const R d0 = (b0 * A11 - b1 * A01) * inv_det;
-    const R d1 = (b1 * A00 - b0 * A01) * inv_det;
-    lam[0] += d0;
-    lam[1] += d1;
+    const R n0 = b0 * A11 - b1 * A01, n1 = b1 * A00 - b0 * A01;
+    const R d0 = n0 * inv_det, d1 = n1 * inv_det;
+    if constexpr (LAM_FMA) {
+        lam[0] = fma(n0, inv_det, lam[0]);
+        lam[1] = fma(n1, inv_det, lam[1]);
+    } else {
+        lam[0] += d0;
+        lam[1] += d1;
+    }
 #pragma unroll
     for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -205,13 +212,13 @@ XPBD_HD void project_tet(const R* u, const R* w, const R* Q, R atD, R atH, R gam
 }
 
 // Projection with vertex positions given as base + delta (see deformation_gradient_split).
-template <typename R>
+template <typename R, bool LAM_FMA = false>
 XPBD_HD void project_tet_split(const R* b, const R* d, const R* w, const R* Q, R atD, R atH,
                                R gamma, R* lam, R* dx)
 {
     R F[9];
     deformation_gradient_split<R>(b, d, Q, F);
-    project_tet_F<R>(F, w, Q, atD, atH, gamma, lam, dx);
+    project_tet_F<R, LAM_FMA>(F, w, Q, atD, atH, gamma, lam, dx);
 }
 
 }  // namespace xpbd
