@@ -1,5 +1,5 @@
-"""The training kernels at the edges of their tiles of 32 rows and 256 workgroups
-(a workgroup takes a second tile past 8,192 rows), against the oracle with the
+"""The training kernels at the edges of their tiles of 32 rows and of their runs of
+rows (split from 256 rows on, longer past 4,096), against the oracle with the
 same BF16 rounding of the products' operands.
 
 A hidden value whose FP32 rounding differs by an ulp may round to another BF16
@@ -30,7 +30,7 @@ def _blocks(g):
     return {name: np.asarray(g[a:b], np.float64) for (name, _), a, b in zip(M.SIZES, at, at[1:])}
 
 
-@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 1000, 8192, 8193, 20000])
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 255, 256, 257, 1000, 4096, 4097, 8192, 8193, 20000])
 def test_gradient(n):
     p, x, t, mean, std = _data(n, n)
     net = X.Network(p)

@@ -54,23 +54,26 @@ __device__ __forceinline__ float dsilu(float z)
 }
 
 // ---------------------------------------------------------------------------
-// Training.  One launch takes a minibatch from its rows to its weight gradients:
-// a workgroup of 8 waves takes tiles of 32 rows, wave w the hidden features
-// 16w..16w+15 of every layer, so that what a wave needs of its own (the
-// pre-activations for SiLU's derivative, its rows of a weight gradient) stays in
-// its registers, and only the activations and their gradients go through LDS, as
-// BF16: row by row as a product's A operand, and feature by feature (a lane leaves
-// four rows of a feature together) as the operands of the weight gradients, whose
-// K is the rows.  Weights are B operands read once per workgroup from a copy in
-// operand order that the update keeps beside the FP32 master.  The gradients of a
-// workgroup's tiles add up in its registers and end in its part of `part`, which
-// the update launch sums in workgroup order: the same result on every run.
+// Training, three launches a minibatch.
+//   rows     forward and back: a workgroup of 8 waves takes 32 rows, wave w the
+//            hidden features 16w..16w+15 of every layer, so that the pre-activations
+//            stay in its registers and only the activations and their gradients go
+//            through LDS, as the BF16 A operand of the next product.  Weights are B
+//            operands, read once from a copy in operand order that the update keeps
+//            beside the FP32 master.  Activations (BF16) and gradients (FP32) are
+//            left feature by feature, a lane's four rows together.
+//   weights  the weight gradients' products, whose K is the rows, by runs of rows,
+//            and the bias gradients' column sums
+//   update   sums of the runs in order, Adam, the weights' operand copies
+// Every sum is formed in the order of a plain product by 32 rows at a time with its
+// runs of rows added up in turn, whatever the grid: a last bit that differs can round
+// an activation to another BF16 number, and over some epochs that shows.
 //
-// 4,096 rows: 24 launches before, 175 us with the update, 16 + 5 us in two now.
-// Bound by the chain of a tile: seven small products, a barrier after each, and the
-// SiLUs' divisions between.
+// 4,096 rows: 24 launches before, 175 us with the update, now 13.5 + 9.8 + 3.7 us in three.  Bound by the
+// chain of a tile of rows: five small products, a barrier after each, and the SiLUs'
+// divisions between.
 // ---------------------------------------------------------------------------
-constexpr int kTrainRows = 32, kTrainWaves = kH / 16, kTrainThreads = 64 * kTrainWaves, kTrainGroups = 256;
+constexpr int kTrainRows = 32, kTrainWaves = kH / 16, kTrainThreads = 64 * kTrainWaves;
 // operand copies of the weights: products of 64 lanes x 8 values
 constexpr int kK2 = kH / 32;   // K steps over the hidden features
 constexpr int fW1 = 0, fW2 = fW1 + kTrainWaves, fW2T = fW2 + kTrainWaves * kK2, fW3 = fW2T + kTrainWaves * kK2,
@@ -122,26 +125,47 @@ __device__ __forceinline__ f32x4 mfma(bf16x8 a, bf16x8 b, f32x4 c)
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// A minibatch's activations and gradients, feature by feature: ld values (its rows up
+// to a multiple of 32, zero gradients past them) each.
+struct TrainRows {
+    int ld = 0;
+    __bf16 *x = nullptr, *h1 = nullptr, *h2 = nullptr;           // kInP, kH, kH features
+    float *d1 = nullptr, *d2 = nullptr, *dy = nullptr;           // kH, kH, kOut
+    double* loss = nullptr;                                      // per 32 rows
+
+    static size_t bytes(size_t ld) { return ld * (2 * (kInP + 2 * kH) + 4 * (2 * kH + kOut)) + 8 * (ld / kTrainRows); }
+    void place(char* p, int rows)
+    {
+        ld = rows;
+        const size_t n = (size_t)rows;
+        d1 = reinterpret_cast<float*>(p);
+        d2 = d1 + kH * n;
+        dy = d2 + kH * n;
+        x = reinterpret_cast<__bf16*>(dy + kOut * n);
+        h1 = x + kInP * n;
+        h2 = h1 + kH * n;
+        loss = reinterpret_cast<double*>(h2 + kH * n);
+    }
+};
+
 // Row r of the minibatch is row perm[(b0 + r) % nall] of X and T (perm null: r).
 // Loss in output units of the network: mean over rows * 3 of (Y - T / scale)^2,
 // i.e. the squared error of the correction measured in units of scale (the
 // physical corrections are ~1e-5 m; a loss in metres would leave gradients far
-// below Adam's epsilon).  dY = 2 (Y - T / scale) / (rows * 3); lpart: a workgroup's
-// part of the sum of squares.
-__global__ __launch_bounds__(kTrainThreads) void k_mlp_grad(const float* __restrict__ X, const float* __restrict__ T,
-                                                           const int* __restrict__ perm, int b0, int nall, int rows,
-                                                           const float* __restrict__ mean,
-                                                           const float* __restrict__ istd, float inv_scale,
-                                                           const float* __restrict__ p, const __bf16* __restrict__ w,
-                                                           float* __restrict__ part, double* __restrict__ lpart)
+// below Adam's epsilon).  dY = 2 (Y - T / scale) / (rows * 3).
+__global__ __launch_bounds__(kTrainThreads) void k_train_rows(const float* __restrict__ X, const float* __restrict__ T,
+                                                             const int* __restrict__ perm, int b0, int nall, int rows,
+                                                             const float* __restrict__ mean,
+                                                             const float* __restrict__ istd, float inv_scale,
+                                                             const float* __restrict__ p, const __bf16* __restrict__ w,
+                                                             TrainRows out)
 {
     constexpr int R = kTrainRows, LR = R + 8, LH = kH + 8;   // padded: rows of 16-byte multiples, banks apart
-    __shared__ alignas(16) __bf16 aX[R][LR], xT[kInP][LR], aH1[R][LH], aH2[R][LH], aD2[R][LH], aY[R][LR], yT[16][LR],
-        h1T[kH][LR], h2T[kH][LR], d1T[kH][LR], d2T[kH][LR];
+    __shared__ alignas(16) __bf16 aX[R][LR], aH1[R][LH], aH2[R][LH], aD2[R][LH], aY[R][LR];
     __shared__ float sT[R][4];
     __shared__ double sl[2 * 64];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 15, q = lane >> 4;
-    const int col = 16 * wv + c;   // this lane's hidden feature
+    const int col = 16 * wv + c, r0 = blockIdx.x * R;   // col: this lane's hidden feature
     auto frag = [&](int f) { return reinterpret_cast<const bf16x8*>(w)[64 * f + lane]; };
     const bf16x8 w1 = frag(fW1 + wv), w3t = frag(fW3T + wv);
     bf16x8 w2[kK2], w2t[kK2], w3[kK2];
@@ -153,172 +177,231 @@ __global__ __launch_bounds__(kTrainThreads) void k_mlp_grad(const float* __restr
     }
     const float b1 = p[oB1 + col], b2 = p[oB2 + col], b3 = c < kOut ? p[oB3 + c] : 0.f;
     const f32x4 zero = { 0.f, 0.f, 0.f, 0.f };
-    f32x4 g1[2] = { zero, zero }, g2[kTrainWaves], g3 = zero;
-#pragma unroll
-    for (int t = 0; t < kTrainWaves; t++) g2[t] = zero;
-    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f;
-    double loss = 0.0;
     for (int i = tid; i < R * LR; i += kTrainThreads) aY[i / LR][i % LR] = (__bf16)0.f;   // its columns 16.. stay zero
-    const int ntiles = (rows + R - 1) / R;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int r0 = tile * R;
-        __syncthreads();   // the last tile's operands are read
-        for (int i = tid; i < R * kInP; i += kTrainThreads) {
-            const int r = i / kInP, k = i % kInP;
-            float x = 0.f;
-            if (r0 + r < rows) {
-                const int src = perm ? perm[(b0 + r0 + r) % nall] : r0 + r;
-                if (k < kIn) x = (X[(size_t)src * kIn + k] - mean[k]) * istd[k];
-                else if (k < kIn + kOut) sT[r][k - kIn] = T[(size_t)src * kOut + k - kIn];
-            }
-            aX[r][k] = (__bf16)x;
-            xT[k][r] = (__bf16)x;
+    for (int i = tid; i < R * kInP; i += kTrainThreads) {
+        const int r = i / kInP, k = i % kInP;
+        float x = 0.f;
+        if (r0 + r < rows) {
+            const int src = perm ? perm[(b0 + r0 + r) % nall] : r0 + r;
+            if (k < kIn) x = (X[(size_t)src * kIn + k] - mean[k]) * istd[k];
+            else if (k < kIn + kOut) sT[r][k - kIn] = T[(size_t)src * kOut + k - kIn];
         }
-        __syncthreads();
-        // forward: lane (q, c) has rows 16 m + 4q + 0..3 of feature col
-        f32x4 z1[2], z2[2];
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            z1[m] = mfma(*reinterpret_cast<const bf16x8*>(&aX[16 * m + c][8 * q]), w1, zero);
-            float h[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                z1[m][j] += b1;
-                h[j] = silu(z1[m][j]);
-                aH1[16 * m + 4 * q + j][col] = (__bf16)h[j];
-            }
-            put4(&h1T[col][16 * m + 4 * q], h);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            z2[m] = zero;
-#pragma unroll
-            for (int k = 0; k < kK2; k++)
-                z2[m] = mfma(*reinterpret_cast<const bf16x8*>(&aH1[16 * m + c][32 * k + 8 * q]), w2[k], z2[m]);
-            float h[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                z2[m][j] += b2;
-                h[j] = silu(z2[m][j]);
-                aH2[16 * m + 4 * q + j][col] = (__bf16)h[j];
-            }
-            put4(&h2T[col][16 * m + 4 * q], h);
-        }
-        __syncthreads();
-        // output and its gradient: waves 0 and 1, 16 rows each
-        if (wv < 2) {
-            f32x4 y = zero;
-#pragma unroll
-            for (int k = 0; k < kK2; k++)
-                y = mfma(*reinterpret_cast<const bf16x8*>(&aH2[16 * wv + c][32 * k + 8 * q]), w3[k], y);
-            float d[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = 16 * wv + 4 * q + j;
-                const bool on = c < kOut && r0 + r < rows;
-                const float e = on ? y[j] + b3 - sT[r][c & 3] * inv_scale : 0.f;
-                d[j] = on ? 2.0f * e / (float)(rows * kOut) : 0.f;
-                loss += (double)e * (double)e;
-                gb3 += d[j];
-                aY[r][c] = (__bf16)d[j];
-            }
-            put4(&yT[c][16 * wv + 4 * q], d);
-        }
-        __syncthreads();
-        // back through layer 3, its weight gradient
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            const f32x4 h = mfma(*reinterpret_cast<const bf16x8*>(&aY[16 * m + c][8 * q]), w3t, zero);
-            float d[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                d[j] = h[j] * dsilu(z2[m][j]);
-                gb2 += d[j];
-                aD2[16 * m + 4 * q + j][col] = (__bf16)d[j];
-            }
-            put4(&d2T[col][16 * m + 4 * q], d);
-        }
-        g3 = mfma(*reinterpret_cast<const bf16x8*>(&yT[c][8 * q]), *reinterpret_cast<const bf16x8*>(&h2T[col][8 * q]), g3);
-        __syncthreads();
-        // back through layer 2, the weight gradients of layers 2 and 1: rows 16 w.. of them
-#pragma unroll
-        for (int m = 0; m < 2; m++) {
-            f32x4 h = zero;
-#pragma unroll
-            for (int k = 0; k < kK2; k++)
-                h = mfma(*reinterpret_cast<const bf16x8*>(&aD2[16 * m + c][32 * k + 8 * q]), w2t[k], h);
-            float d[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                d[j] = h[j] * dsilu(z1[m][j]);
-                gb1 += d[j];
-            }
-            put4(&d1T[col][16 * m + 4 * q], d);
-        }
-        const bf16x8 d2 = *reinterpret_cast<const bf16x8*>(&d2T[col][8 * q]);
-#pragma unroll
-        for (int t = 0; t < kTrainWaves; t++)
-            g2[t] = mfma(d2, *reinterpret_cast<const bf16x8*>(&h1T[16 * t + c][8 * q]), g2[t]);
-        __syncthreads();
-        const bf16x8 d1 = *reinterpret_cast<const bf16x8*>(&d1T[col][8 * q]);
-#pragma unroll
-        for (int t = 0; t < 2; t++) g1[t] = mfma(d1, *reinterpret_cast<const bf16x8*>(&xT[16 * t + c][8 * q]), g1[t]);
+        aX[r][k] = (__bf16)x;
+        out.x[(size_t)k * out.ld + r0 + r] = (__bf16)x;
     }
-    float* const o = part + (size_t)blockIdx.x * kNParams;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int row = 16 * wv + 4 * q + j;
-#pragma unroll
-        for (int t = 0; t < kTrainWaves; t++) o[oW2 + row * kH + 16 * t + c] = g2[t][j];
-#pragma unroll
-        for (int t = 0; t < 2; t++)
-            if (16 * t + c < kIn) o[oW1 + row * kIn + 16 * t + c] = g1[t][j];
-        if (4 * q + j < kOut) o[oW3 + (4 * q + j) * kH + col] = g3[j];
-    }
-    // biases: the four lanes of a feature
-    gb1 += __shfl_xor(gb1, 16);
-    gb2 += __shfl_xor(gb2, 16);
-    gb3 += __shfl_xor(gb3, 16);
-    gb1 += __shfl_xor(gb1, 32);
-    gb2 += __shfl_xor(gb2, 32);
-    gb3 += __shfl_xor(gb3, 32);
-    if (q == 0) {
-        o[oB1 + col] = gb1;
-        o[oB2 + col] = gb2;
-    }
-    __syncthreads();   // sT and the first tile's yT are free: wave 1's bias sums by way of sT
-    if (wv < 2) sl[64 * wv + lane] = loss;
-    if (wv == 1 && lane < kOut) sT[0][lane] = gb3;
     __syncthreads();
-    if (wv == 0 && lane < kOut) o[oB3 + lane] = gb3 + sT[0][lane];
+    // this lane's rows of feature f among those left: 16 m + 4q + 0..3
+    auto at = [&](int f, int m) { return (size_t)f * out.ld + r0 + 16 * m + 4 * q; };
+    // forward
+    f32x4 z1[2], z2[2];
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        z1[m] = mfma(*reinterpret_cast<const bf16x8*>(&aX[16 * m + c][8 * q]), w1, zero);
+        float h[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            z1[m][j] += b1;
+            h[j] = silu(z1[m][j]);
+            aH1[16 * m + 4 * q + j][col] = (__bf16)h[j];
+        }
+        put4(out.h1 + at(col, m), h);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        z2[m] = zero;
+#pragma unroll
+        for (int k = 0; k < kK2; k++)
+            z2[m] = mfma(*reinterpret_cast<const bf16x8*>(&aH1[16 * m + c][32 * k + 8 * q]), w2[k], z2[m]);
+        float h[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            z2[m][j] += b2;
+            h[j] = silu(z2[m][j]);
+            aH2[16 * m + 4 * q + j][col] = (__bf16)h[j];
+        }
+        put4(out.h2 + at(col, m), h);
+    }
+    __syncthreads();
+    // output and its gradient: waves 0 and 1, 16 rows each
+    if (wv < 2) {
+        f32x4 y = zero;
+#pragma unroll
+        for (int k = 0; k < kK2; k++)
+            y = mfma(*reinterpret_cast<const bf16x8*>(&aH2[16 * wv + c][32 * k + 8 * q]), w3[k], y);
+        float d[4];
+        double loss = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int r = 16 * wv + 4 * q + j;
+            const bool on = c < kOut && r0 + r < rows;
+            const float e = on ? fmaf(-sT[r][c & 3], inv_scale, y[j] + b3) : 0.f;
+            d[j] = on ? 2.0f * e / (float)(rows * kOut) : 0.f;
+            loss += (double)e * (double)e;
+            aY[r][c] = (__bf16)d[j];
+        }
+        if (c < kOut) *reinterpret_cast<float4*>(out.dy + at(c, wv)) = make_float4(d[0], d[1], d[2], d[3]);
+        sl[64 * wv + lane] = loss;
+    }
+    __syncthreads();
+    // back through layer 3
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        const f32x4 h = mfma(*reinterpret_cast<const bf16x8*>(&aY[16 * m + c][8 * q]), w3t, zero);
+        float d[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            d[j] = h[j] * dsilu(z2[m][j]);
+            aD2[16 * m + 4 * q + j][col] = (__bf16)d[j];
+        }
+        *reinterpret_cast<float4*>(out.d2 + at(col, m)) = make_float4(d[0], d[1], d[2], d[3]);
+    }
     if (tid == 0) {
         double l = 0.0;
         for (int i = 0; i < 2 * 64; i++) l += sl[i];
-        lpart[blockIdx.x] = l;
+        out.loss[blockIdx.x] = l;
+    }
+    __syncthreads();
+    // and layer 2
+#pragma unroll
+    for (int m = 0; m < 2; m++) {
+        f32x4 h = zero;
+#pragma unroll
+        for (int k = 0; k < kK2; k++)
+            h = mfma(*reinterpret_cast<const bf16x8*>(&aD2[16 * m + c][32 * k + 8 * q]), w2t[k], h);
+        float d[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = h[j] * dsilu(z1[m][j]);
+        *reinterpret_cast<float4*>(out.d1 + at(col, m)) = make_float4(d[0], d[1], d[2], d[3]);
     }
 }
 
-// The sum of the workgroups' gradients, in four runs of them side by side, and with
-// ADAM the update of the master, the moments and the operand copies; otherwise into g.
-template <bool ADAM>
-__global__ __launch_bounds__(256) void k_mlp_update(const float* __restrict__ part, int ngroups, float* __restrict__ g,
-                                                   float* __restrict__ p, float* __restrict__ m, float* __restrict__ v,
-                                                   __bf16* __restrict__ w, float lr, float b1, float b2, float c1,
-                                                   float c2, float eps)
+// Runs of rows that a weight gradient of `tiles` output tiles of 32 x 32 is formed
+// by: of at least 128 rows, up to 512 tiles' worth and kMaxRuns of them.
+constexpr int kMaxRuns = 64, kRuns2 = 32;
+struct Runs {
+    int rows, n;
+};
+inline Runs runs_of(int rows, int tiles)
 {
-    __shared__ float run[4][64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
-    const int per = (ngroups + 3) / 4, z0 = wv * per, z1 = min(ngroups, z0 + per);
-    float s = 0.f;
-    if (i < kNParams) {
-#pragma unroll 16
-        for (int z = z0; z < z1; z++) s += part[(size_t)z * kNParams + i];
+    int n = 1;
+    if (rows >= 256) n = std::min(std::min((512 + tiles - 1) / tiles, (rows + 127) / 128), kMaxRuns);
+    const int len = ((rows + n - 1) / n + 31) / 32 * 32;
+    return { len, (rows + len - 1) / len };
+}
+
+// eight rows of one feature's gradient as an operand
+__device__ __forceinline__ bf16x8 as_operand(const float* d)
+{
+    const float4 a = reinterpret_cast<const float4*>(d)[0], b = reinterpret_cast<const float4*>(d)[1];
+    return bf16x8{ (__bf16)a.x, (__bf16)a.y, (__bf16)a.z, (__bf16)a.w, (__bf16)b.x, (__bf16)b.y, (__bf16)b.z, (__bf16)b.w };
+}
+
+// Blocks 4 z + k: rows 32k..32k+31 of layer 2's weight gradient over run z of r2; then
+// one a run of r13 for layers 1 and 3; then one a bias.  A wave has 16 x 64 outputs of
+// layer 2 (32 x 32 of layer 1, 16 x 32 of layer 3), 32 rows of the minibatch a step.
+__global__ __launch_bounds__(256) void k_train_weights(TrainRows in, int rows, Runs r2, Runs r13,
+                                                      float* __restrict__ part2, float* __restrict__ part13,
+                                                      float* __restrict__ bias)
+{
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 15, q = lane >> 4;
+    const size_t ld = (size_t)in.ld;
+    const f32x4 zero = { 0.f, 0.f, 0.f, 0.f };
+    int b = blockIdx.x;
+    if (b < 4 * r2.n) {
+        const int z = b >> 2, o0 = 32 * (b & 3) + 16 * (wv >> 1), i0 = 64 * (wv & 1);
+        const int k0 = z * r2.rows, k1 = min(rows, k0 + r2.rows);
+        f32x4 g[4] = { zero, zero, zero, zero };
+#pragma unroll 4
+        for (int k = k0; k < k1; k += 32) {
+            const bf16x8 d = as_operand(in.d2 + (o0 + c) * ld + k + 8 * q);
+#pragma unroll
+            for (int t = 0; t < 4; t++)
+                g[t] = mfma(d, *reinterpret_cast<const bf16x8*>(in.h1 + (i0 + 16 * t + c) * ld + k + 8 * q), g[t]);
+        }
+        float* const o = part2 + (size_t)z * kH * kH;
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[(o0 + 4 * q + j) * kH + i0 + 16 * t + c] = g[t][j];
+        return;
     }
-    run[wv][lane] = s;
+    b -= 4 * r2.n;
+    if (b < r13.n) {
+        const int k0 = b * r13.rows, k1 = min(rows, k0 + r13.rows);
+        f32x4 g1[2][2] = { { zero, zero }, { zero, zero } }, g3[2] = { zero, zero };
+#pragma unroll 2
+        for (int k = k0; k < k1; k += 32) {
+            bf16x8 y{};
+            if (c < kOut) y = as_operand(in.dy + c * ld + k + 8 * q);
+            bf16x8 x[2];
+#pragma unroll
+            for (int t = 0; t < 2; t++) x[t] = *reinterpret_cast<const bf16x8*>(in.x + (16 * t + c) * ld + k + 8 * q);
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int f = 32 * wv + 16 * t + c;
+                const bf16x8 d = as_operand(in.d1 + f * ld + k + 8 * q);
+                g1[t][0] = mfma(d, x[0], g1[t][0]);
+                g1[t][1] = mfma(d, x[1], g1[t][1]);
+                g3[t] = mfma(y, *reinterpret_cast<const bf16x8*>(in.h2 + f * ld + k + 8 * q), g3[t]);
+            }
+        }
+        float* const o = part13 + (size_t)b * (kH * kIn + kOut * kH);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int f = 32 * wv + 16 * t, row = 4 * q + j;
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+                    if (16 * u + c < kIn) o[(f + row) * kIn + 16 * u + c] = g1[t][u][j];
+                if (row < kOut) o[kH * kIn + row * kH + f + c] = g3[t][j];
+            }
+        return;
+    }
+    b -= r13.n;   // a column sum: rows 256 apart by thread, then by halves
+    __shared__ float sh[256];
+    const float* d = b < kH ? in.d1 + b * ld : b < 2 * kH ? in.d2 + (b - kH) * ld : in.dy + (b - 2 * kH) * ld;
+    float s = 0.f;
+    for (int r = tid; r < rows; r += 256) s += d[r];
+    sh[tid] = s;
     __syncthreads();
-    if (wv != 0 || i >= kNParams) return;
-    const float gi = ((run[0][lane] + run[1][lane]) + run[2][lane]) + run[3][lane];
+    for (int k = 128; k > 0; k >>= 1) {
+        if (tid < k) sh[tid] += sh[tid + k];
+        __syncthreads();
+    }
+    if (tid == 0) bias[b] = sh[0];
+}
+
+// The sum of the runs, in order, and with ADAM the update of the master, the moments
+// and the operand copies; otherwise into g.
+template <bool ADAM>
+__global__ __launch_bounds__(256) void k_train_update(const float* __restrict__ part2, int n2,
+                                                     const float* __restrict__ part13, int n13,
+                                                     const float* __restrict__ bias, float* __restrict__ g,
+                                                     float* __restrict__ p, float* __restrict__ m,
+                                                     float* __restrict__ v, __bf16* __restrict__ w, float lr, float b1,
+                                                     float b2, float c1, float c2, float eps)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= kNParams) return;
+    float gi = 0.f;
+    const float* part = nullptr;
+    size_t stride = kH * kIn + kOut * kH;
+    int n = n13;
+    if (i < oB1) part = part13 + i;
+    else if (i < oW2) gi = bias[i - oB1];
+    else if (i < oB2) {
+        part = part2 + (i - oW2);
+        stride = kH * kH;
+        n = n2;
+    } else if (i < oW3) gi = bias[kH + i - oB2];
+    else if (i < oB3) part = part13 + kH * kIn + (i - oW3);
+    else gi = bias[2 * kH + i - oB3];
+    if (part) {
+#pragma unroll 16
+        for (int z = 0; z < n; z++) gi += part[z * stride];
+    }
     if constexpr (!ADAM) {
         g[i] = gi;
         return;
@@ -613,8 +696,9 @@ struct xpbd_mlp {
     float* d_mean = nullptr;
     float* d_istd = nullptr;
     __bf16* d_wt = nullptr;   // BF16 copies in the training products' operand order
-    float* d_part = nullptr;  // gradients by workgroup
-    double* d_lpart = nullptr;
+    float* d_part = nullptr;  // weight gradients by run of rows, bias gradients
+    char* d_rows = nullptr;   // a minibatch's TrainRows
+    int cap_rows = 0;
     float scale = 1.f;
     // Identifies the network and its output scale (the scale is a launch
     // argument of the inference, so graphs that captured it go stale when it
@@ -664,7 +748,7 @@ hipError_t room(T** p, size_t n)
     return hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T));
 }
 
-// rows of inputs and outputs; train: of targets and of a permutation, and the gradient's parts, too
+// rows of inputs and outputs; train: of targets and of a permutation, too
 hipError_t ensure_ws(xpbd_mlp* m, int rows, bool train)
 {
     const size_t r = (size_t)rows;
@@ -684,35 +768,64 @@ hipError_t ensure_ws(xpbd_mlp* m, int rows, bool train)
         m->cap = rows;
         m->cap_train = keep_train ? rows : 0;
     }
-    if (train && !m->d_lpart) {
-        e = room(&m->d_wt, 512 * (size_t)kFrags);
-        if (e == hipSuccess) e = room(&m->d_part, (size_t)kTrainGroups * kNParams);
-        if (e == hipSuccess) e = xpbd::launch_fill_zero(m->stream, m->d_wt, sizeof(__bf16) * 512 * kFrags);
-        if (e == hipSuccess) e = room(&m->d_lpart, kTrainGroups);
-        if (e != hipSuccess) release(m->d_wt, m->d_part, m->d_lpart);
-    }
     return e;
 }
 
-int train_groups(int rows) { return std::min(kTrainGroups, (rows + kTrainRows - 1) / kTrainRows); }
+constexpr size_t kPart2 = (size_t)kRuns2 * kH * kH, kPart13 = (size_t)kMaxRuns * (kH * kIn + kOut * kH);
+
+// what a minibatch of `rows` rows leaves from launch to launch
+hipError_t ensure_minibatch(xpbd_mlp* m, int rows, TrainRows* t)
+{
+    hipError_t e = hipSuccess;
+    if (!m->d_wt) {
+        e = room(&m->d_wt, 512 * (size_t)kFrags);
+        if (e == hipSuccess) e = room(&m->d_part, kPart2 + kPart13 + 2 * kH + kOut);
+        if (e == hipSuccess) e = xpbd::launch_fill_zero(m->stream, m->d_wt, sizeof(__bf16) * 512 * kFrags);
+        if (e != hipSuccess) release(m->d_wt, m->d_part);
+    }
+    const int ld = (rows + kTrainRows - 1) / kTrainRows * kTrainRows;
+    if (e == hipSuccess && ld > m->cap_rows) {
+        (void)hipStreamSynchronize(m->stream);
+        release(m->d_rows);
+        m->cap_rows = 0;
+        e = room(&m->d_rows, TrainRows::bytes(ld));
+        if (e == hipSuccess) m->cap_rows = ld;
+    }
+    if (e == hipSuccess) t->place(m->d_rows, ld);
+    return e;
+}
 
 void train_pack(xpbd_mlp* m)
 {
     hipLaunchKernelGGL(k_train_pack, dim3(nb(kNParams)), dim3(256), 0, m->stream, m->d_p, m->d_wt);
 }
 
-// Gradient parts of `rows` rows of d_X, d_T: from b0 on through the permutation of nall, or (nall 0) as they lie.
-void gradient(xpbd_mlp* m, int rows, int b0, int nall)
+// Gradients of `rows` rows of d_X, d_T, from b0 on through the permutation of nall or (nall 0) as they
+// lie, up to their runs' sums; then the sums, into d_g or (lr > 0) into the weights.
+struct Adam {
+    float lr = 0.f, b1 = 0.f, b2 = 0.f, c1 = 0.f, c2 = 0.f, eps = 0.f;
+};
+void train_step(xpbd_mlp* m, const TrainRows& t, int rows, int b0, int nall, const Adam& a)
 {
-    hipLaunchKernelGGL(k_mlp_grad, dim3(train_groups(rows)), dim3(kTrainThreads), 0, m->stream, m->d_X, m->d_T,
-                       nall > 0 ? m->d_perm : nullptr, b0, nall, rows, m->d_mean, m->d_istd, 1.0f / m->scale, m->d_p,
-                       m->d_wt, m->d_part, m->d_lpart);
+    const Runs r2 = runs_of(rows, 16), r13 = runs_of(rows, 4);   // tiles of 32 x 32: 128 x 128; 128 x 24 and 3 x 128
+    float *part13 = m->d_part + kPart2, *bias = part13 + kPart13;
+    hipLaunchKernelGGL(k_train_rows, dim3((rows + kTrainRows - 1) / kTrainRows), dim3(kTrainThreads), 0, m->stream, m->d_X,
+                       m->d_T, nall > 0 ? m->d_perm : nullptr, b0, nall, rows, m->d_mean, m->d_istd, 1.0f / m->scale,
+                       m->d_p, m->d_wt, t);
+    hipLaunchKernelGGL(k_train_weights, dim3(4 * r2.n + r13.n + 2 * kH + kOut), dim3(256), 0, m->stream, t, rows, r2, r13,
+                       m->d_part, part13, bias);
+    if (a.lr > 0.f)
+        hipLaunchKernelGGL(k_train_update<true>, dim3(nb(kNParams)), dim3(256), 0, m->stream, m->d_part, r2.n, part13,
+                           r13.n, bias, nullptr, m->d_p, m->d_m, m->d_v, m->d_wt, a.lr, a.b1, a.b2, a.c1, a.c2, a.eps);
+    else
+        hipLaunchKernelGGL(k_train_update<false>, dim3(nb(kNParams)), dim3(256), 0, m->stream, m->d_part, r2.n, part13,
+                           r13.n, bias, m->d_g, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
 }
 
-double read_loss(xpbd_mlp* m, int rows)
+double read_loss(xpbd_mlp* m, const TrainRows& t, int rows)
 {
-    std::vector<double> lp(train_groups(rows));
-    (void)hipMemcpyAsync(lp.data(), m->d_lpart, sizeof(double) * lp.size(), hipMemcpyDeviceToHost, m->stream);
+    std::vector<double> lp((rows + kTrainRows - 1) / kTrainRows);
+    (void)hipMemcpyAsync(lp.data(), t.loss, sizeof(double) * lp.size(), hipMemcpyDeviceToHost, m->stream);
     (void)hipStreamSynchronize(m->stream);
     double s = 0;
     for (double v : lp) s += v;
@@ -787,7 +900,7 @@ extern "C" int xpbd_mlp_destroy(xpbd_mlp* m)
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     free_ws(m);
     release(m->d_p, m->d_g, m->d_m, m->d_v, m->d_w1, m->d_w2, m->d_w3, m->d_mean, m->d_istd, m->d_wt, m->d_part,
-            m->d_lpart);
+            m->d_rows);
     if (m->stream) (void)hipStreamDestroy(m->stream);
     delete m;
     return XPBD_OK;
@@ -1000,18 +1113,18 @@ extern "C" int xpbd_mlp_loss_grad(xpbd_mlp* m, int32_t n, const float* x, const 
 {
     if (!m || n <= 0 || !x || !y || !loss) return XPBD_E_INVALID_ARG;
     hipError_t e = ensure_ws(m, n, true);
+    TrainRows t;
+    if (e == hipSuccess) e = ensure_minibatch(m, n, &t);
     if (e != hipSuccess) return merr(m, XPBD_E_NOMEM, hipGetErrorString(e));
     e = hipMemcpyAsync(m->d_X, x, sizeof(float) * kIn * (size_t)n, hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(m->d_T, y, sizeof(float) * kOut * (size_t)n, hipMemcpyHostToDevice, m->stream);
     if (e != hipSuccess) return merr(m, XPBD_E_HIP, hipGetErrorString(e));
     train_pack(m);
-    gradient(m, n, 0, 0);
-    hipLaunchKernelGGL(k_mlp_update<false>, dim3((kNParams + 63) / 64), dim3(256), 0, m->stream, m->d_part,
-                       train_groups(n), m->d_g, nullptr, nullptr, nullptr, nullptr, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f);
+    train_step(m, t, n, 0, 0, Adam{});
     e = hipGetLastError();
     if (e != hipSuccess) return merr(m, XPBD_E_HIP, hipGetErrorString(e));
-    *loss = read_loss(m, n);
+    *loss = read_loss(m, t, n);
     if (grad) {
         e = hipMemcpyAsync(grad, m->d_g, sizeof(float) * kNParams, hipMemcpyDeviceToHost, m->stream);
         if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
@@ -1028,6 +1141,8 @@ extern "C" int xpbd_mlp_train(xpbd_mlp* m, int32_t n, const float* x, const floa
     // all samples live on the device; each epoch takes its minibatches through a
     // seeded permutation
     hipError_t e = ensure_ws(m, n, true);
+    TrainRows t;
+    if (e == hipSuccess) e = ensure_minibatch(m, batch, &t);
     if (e != hipSuccess) return merr(m, XPBD_E_NOMEM, hipGetErrorString(e));
     e = hipMemcpyAsync(m->d_X, x, sizeof(float) * kIn * (size_t)n, hipMemcpyHostToDevice, m->stream);
     if (e == hipSuccess)
@@ -1047,15 +1162,13 @@ extern "C" int xpbd_mlp_train(xpbd_mlp* m, int32_t n, const float* x, const floa
         std::shuffle(perm.begin(), perm.end(), rng);
         e = hipMemcpyAsync(m->d_perm, perm.data(), sizeof(int) * (size_t)n, hipMemcpyHostToDevice, m->stream);
         for (int bi = 0; bi < nbatch && e == hipSuccess; bi++) {
-            gradient(m, batch, bi * batch, n);
             m->adam_t++;
             const float c1 = 1.f - std::pow(b1, (float)m->adam_t), c2 = 1.f - std::pow(b2, (float)m->adam_t);
-            hipLaunchKernelGGL(k_mlp_update<true>, dim3((kNParams + 63) / 64), dim3(256), 0, m->stream, m->d_part,
-                               train_groups(batch), nullptr, m->d_p, m->d_m, m->d_v, m->d_wt, lr, b1, b2, c1, c2, eps);
+            train_step(m, t, batch, bi * batch, n, Adam{ lr, b1, b2, c1, c2, eps });
             e = hipGetLastError();
         }
         // the host permutation is rewritten next epoch: wait for its copy
-        if (e == hipSuccess) last = read_loss(m, batch);
+        if (e == hipSuccess) last = read_loss(m, t, batch);
     }
     if (e == hipSuccess) e = pack(m);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
