@@ -845,13 +845,13 @@ int enqueue_contacts_jacobi(xpbd_handle* h, bool first)
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "contacts_jacobi launch");
 }
 
-static Prediction prediction(const xpbd_handle* h)
+Prediction prediction(const xpbd_handle* h)
 {
     const double dt = h->params.dt;
     return { h->d_vel, h->params.first_order ? h->d_dz1 : nullptr, (float)dt, (float)(-h->params.g * dt * dt) };
 }
 
-static HitLists hit_lists(const xpbd_handle* h)
+HitLists hit_lists(const xpbd_handle* h)
 {
     HitLists H;
     H.flag = h->d_flag;
@@ -888,7 +888,7 @@ static bool runs_tiled_jacobi(const xpbd_handle* h, int iters)
            h->natt == 0 && iters > 0;
 }
 
-static int enqueue_finish(xpbd_handle* h, const MotionSource& from)
+int enqueue_finish(xpbd_handle* h, const MotionSource& from)
 {
     hipError_t e = launch_finish(h->stream, h->d_pos, h->d_lo, h->d_vel, h->nv, (float)h->params.dt, h->d_step, from);
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "finish launch");
@@ -1202,7 +1202,7 @@ int enqueue_local_collision(xpbd_handle* h)
     return XPBD_OK;
 }
 
-static int enqueue_flags(xpbd_handle* h)
+int enqueue_flags(xpbd_handle* h)
 {
     hipError_t e = launch_detect(h->stream, h->d_faces, h->d_rest, h->d_pos, h->d_lo, h->d_sdf, h->d_step, h->params.dt,
                                  h->d_flag, hit_lists(h), h->d_cp, h->d_cn, h->d_cb);

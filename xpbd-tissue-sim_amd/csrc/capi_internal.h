@@ -203,6 +203,10 @@ int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_lambda 
 int enqueue_detect(xpbd_handle* h);
 int enqueue_predict(xpbd_handle* h);
 int enqueue_finish(xpbd_handle* h);
+int enqueue_finish(xpbd_handle* h, const MotionSource& from);
+int enqueue_flags(xpbd_handle* h);   // detection without its lists
+Prediction prediction(const xpbd_handle* h);
+HitLists hit_lists(const xpbd_handle* h);
 int enqueue_local_collision(xpbd_handle* h);
 // Jacobi contact pass into the accumulator (fixed order in the deterministic patch mode).
 int enqueue_contacts_jacobi(xpbd_handle* h, bool first);

@@ -60,6 +60,9 @@ struct MotionSource {
     const int* soff = nullptr;
     const float4* prd = nullptr;
     const float4* brd = nullptr;
+    // with cprev: the solver's correction, motion minus pred (0 at pins), goes there
+    const float4* pred = nullptr;
+    float4* cprev = nullptr;
 };
 hipError_t launch_finish(hipStream_t s, float4* pos, float4* lo, float4* vel, int nv, float dt,
                          unsigned long long* step_counter, const MotionSource& from = MotionSource{});

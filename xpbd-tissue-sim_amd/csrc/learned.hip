@@ -30,6 +30,7 @@
 
 #include "capi_internal.h"
 #include "kernels.h"
+#include "step_ops.h"
 #include "xpbd_math.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -640,6 +641,36 @@ __global__ void k_copy_delta(const float4* __restrict__ pos, float4* __restrict_
 {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i < nv) pred[i] = pos[2 * (size_t)i + 1];
+}
+
+// The start of a learned step in one launch: the state's snapshot for a fallback,
+// the prediction and its copy, and the lists of a detection's hits, which were seven
+// small launches and copies.
+__global__ __launch_bounds__(xpbd::kStepBlock) void k_learned_begin(float4* __restrict__ pos,
+                                                                   const float4* __restrict__ lo,
+                                                                   const float4* __restrict__ vel, int nv,
+                                                                   const unsigned long long* __restrict__ step,
+                                                                   float4* __restrict__ save,
+                                                                   unsigned long long* __restrict__ step_save,
+                                                                   float4* __restrict__ pred, xpbd::Prediction P,
+                                                                   xpbd::HitLists H, int nblocks)
+{
+    __shared__ int ws[2 * xpbd::kStepWaves];
+    if ((int)blockIdx.x >= nblocks) {
+        xpbd::scatter_hits(H, blockIdx.x - nblocks, gridDim.x - nblocks, ws);
+        return;
+    }
+    const int i = blockIdx.x * xpbd::kStepBlock + threadIdx.x;
+    if (i == 0) step_save[0] = step[0];
+    if (i >= nv) return;
+    const size_t n = (size_t)nv;
+    save[2 * (size_t)i] = pos[2 * (size_t)i];
+    save[2 * (size_t)i + 1] = pos[2 * (size_t)i + 1];
+    save[2 * n + i] = lo[i];
+    save[3 * n + i] = vel[i];
+    const float4 d = xpbd::predicted(P, i);
+    pos[2 * (size_t)i + 1] = d;
+    pred[i] = d;
 }
 
 // start of the solve moved by the network's correction (free vertices only)
@@ -1462,16 +1493,16 @@ static int enqueue_learned_attempt(xpbd_handle* h, int32_t iters, bool det, bool
     const int nv = h->nv;
     hipStream_t s = h->stream;
     int rc;
-    if (det && (rc = enqueue_detect(h))) return rc;
-    hipError_t e = hipMemcpyAsync(L->d_save, h->d_pos, sizeof(float4) * 2 * (size_t)nv, hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(L->d_save + 2 * (size_t)nv, h->d_lo, sizeof(float4) * nv, hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(L->d_save + 3 * (size_t)nv, h->d_vel, sizeof(float4) * nv, hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(L->d_step_save, h->d_step, sizeof(unsigned long long), hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) return hip_err(h, e, "learned snapshot");
-    if ((rc = enqueue_predict(h)) || (rc = enqueue_copy_pred(h)) || (rc = enqueue_features(h))) return rc;
+    det = det && h->nf > 0;
+    if (det && (rc = enqueue_flags(h))) return rc;
+    const HitLists H = det ? hit_lists(h) : HitLists{};
+    hipLaunchKernelGGL(k_learned_begin, dim3(nb(nv) + (det ? compact_blocks(h->nf) : 0)), dim3(kStepBlock), 0, s, h->d_pos,
+                       h->d_lo, h->d_vel, nv, h->d_step, L->d_save, L->d_step_save, L->d_pred, prediction(h), H,
+                       (int)nb(nv));
+    hipError_t e = hipGetLastError();
+    if (e == hipSuccess && h->primary_residual) e = launch_keep_prediction(s, h->d_pos, h->d_pred, nv);
+    if (e != hipSuccess) return hip_err(h, e, "learned start");
+    if ((rc = enqueue_features(h))) return rc;
     if (timed) (void)hipEventRecord(L->ev0, s);
     e = mlp_infer(L->mlp, s, L->d_feat, nv, L->d_corr);
     if (timed) (void)hipEventRecord(L->ev1, s);
@@ -1488,8 +1519,10 @@ static int enqueue_learned_attempt(xpbd_handle* h, int32_t iters, bool det, bool
     if (e != hipSuccess) return hip_err(h, e, "learned residual");
     if (records_residuals(h) && (rc = enqueue_step_residual(h))) return rc;
     if ((rc = enqueue_local_collision(h))) return rc;
-    if ((rc = enqueue_store_cprev(h)) || (rc = enqueue_finish(h))) return rc;
-    return XPBD_OK;
+    MotionSource from;
+    from.pred = L->d_pred;
+    from.cprev = L->d_cprev;
+    return enqueue_finish(h, from);
 }
 
 // Launch the attempt from a captured graph (built on first use of its shape).

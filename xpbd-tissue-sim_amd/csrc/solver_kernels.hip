@@ -118,6 +118,10 @@ __global__ __launch_bounds__(kBlock) void k_finish(float4* __restrict__ pos, flo
     }
     float4 l = lo[i];
     float4 v = vel[i];
+    if (from.cprev) {
+        const float4 p = from.pred[i];
+        from.cprev[i] = v.w != 0.f ? make_float4(0.f, 0.f, 0.f, 0.f) : make_float4(d.x - p.x, d.y - p.y, d.z - p.z, 0.f);
+    }
     if (v.w != 0.0f) d = make_float4(0.f, 0.f, 0.f, 0.f);
     v.x = d.x / dt;
     v.y = d.y / dt;
