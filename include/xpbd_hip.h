@@ -344,9 +344,9 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
 #define XPBD_QUAD_SPLIT 1000
 /* The quad block value of the fused-colour launches, the untuned default where
  * the mesh's size suits them: several consecutive colours share one launch, in
- * which a workgroup runs them on a spatial tile of the mesh (same element order;
- * the same results up to FP32 rounding within an element).  Handles with
- * attachments run the 256-thread quad shape instead. */
+ * which a workgroup runs them on a spatial tile of the mesh (same element order,
+ * the same results).  Handles with attachments run the 256-thread quad shape
+ * instead. */
 #define XPBD_QUAD_TILE 4000
 /* The patch block value of the vertex-tile Jacobi launches, the untuned default
  * where the mesh's size suits them: a workgroup owns a set of vertices and

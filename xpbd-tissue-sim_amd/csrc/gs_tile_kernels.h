@@ -9,6 +9,8 @@ namespace xpbd {
 
 constexpr size_t kGsTileLds = 160 * 1024;   // LDS of a workgroup, gfx950
 
+constexpr int kLaneRow = 224;   // float4s of 64 elements' data with one lane a cluster
+
 // Which tile kernel: lanes per cluster (4 or 1), element rows of a block at
 // most (6 or 8), and whether every block has that many (always so with one lane).
 struct GsTileShape {
@@ -26,7 +28,7 @@ struct GsTileArgs {
     const int* home;         // one lane a cluster: per block and lane 2 * first solver position + whether it writes dlam
     const float4* stream;    // four lanes a cluster, 64 per row: lane j of a quad (Q's row j, then alpha tilde D / H /
                              // gamma); a block's first row: eight 16-bit slots a lane.
-                             // One lane a cluster, 320 per row: see k_gs_tile_lane
+                             // One lane a cluster, kLaneRow per row: see k_gs_tile_lane
     float2* lam;             // 16 (64) per row; with four lanes a block's first row: as home
     float2* dlam;            // solver order
     const float4* din;       // in-step motion, by slot of this group

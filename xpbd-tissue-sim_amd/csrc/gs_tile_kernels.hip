@@ -336,16 +336,36 @@ __global__ __launch_bounds__(256) void k_gs_tile_fill(GsTileFill A)
     if (j == 0) A.lam[row * 16 + quad] = make_float2(__int_as_float(2 * e0 + (A.own[i >> 2] ? 1 : 0)), 0.f);
 }
 
+// The sums that project_quad forms over a quad's lanes, in one lane: every product
+// rounded, (0 + 1) + (2 + 3).
+__device__ __forceinline__ float sum_of_products(const float (&a)[4], const float (&b)[4])
+{
+#pragma clang fp contract(off)
+    const float x0 = a[0] * b[0], x1 = a[1] * b[1], x2 = a[2] * b[2], x3 = a[3] * b[3];
+    return (x0 + x1) + (x2 + x3);
+}
+__device__ __forceinline__ float sum_of_products(float a0, float b0, float a1, float b1, float a2, float b2)
+{
+#pragma clang fp contract(off)   // the fourth is zero: a position relative to itself
+    const float x0 = a0 * b0, x1 = a1 * b1, x2 = a2 * b2;
+    return (x0 + x1) + x2;
+}
+
+__device__ __forceinline__ float sum3(float a0, float b0, float a1, float b1, float a2, float b2)
+{
+    return fmaf(a2, b2, fmaf(a0, b0, a1 * b1));
+}
+
 // One element in one lane: b its vertices' bases (and inverse masses), d their
-// in-step motions, q column-major Q, M = sum_i w_i q_i q_i^T over Q's rows q_i and
-// q_3 = -(q_0 + q_1 + q_2), as (00, 11, 22, 2 * 01, 2 * 02, 2 * 12).
-// The gradients of C_D and C_H at vertex i are F q_i / C_D and f cof(F) q_i with
-// f = dC_H / dJ, so the 2x2 system's sums over the vertices are
-// <F^T F, M> / C_D^2, J tr(M) f / C_D (as F^T cof(F) = J I) and
-// f^2 <cof(F)^T cof(F), M>, and the correction of vertex i is
-// w_i (d0 / C_D F + d1 f cof(F)) q_i: no gradient is formed.
+// in-step motions, q column-major Q.  The same operations, in the same order, as
+// project_quad, so the same bits, with the gradients of all four vertices in turn;
+// the FMAs that the compiler makes of its expressions are written out, as it does
+// not choose them alike here.  (The 2x2 system's sums by way of M = sum w q q^T need
+// 15 % fewer instructions and 24 bytes more an element; but another order of
+// operations is another last bit, and where a contact comes or goes by it, another
+// motion.)
 __device__ __forceinline__ void project_lane(const float (&q)[9], const float atD, const float atH, const float gamma,
-                                             const float (&M)[6], const float4 (&b)[4], float (&d)[4][3], float2& lam)
+                                             const float4 (&b)[4], float (&d)[4][3], float2& lam)
 {
     float D[3][3];
 #pragma unroll
@@ -359,58 +379,61 @@ __device__ __forceinline__ void project_lane(const float (&q)[9], const float at
     for (int c = 0; c < 3; c++)
 #pragma unroll
         for (int r = 0; r < 3; r++) {
-            const float sum = D[0][r] * q[3 * c] + D[1][r] * q[3 * c + 1] + D[2][r] * q[3 * c + 2];
+            const float sum = sum_of_products(D[0][r], q[3 * c], D[1][r], q[3 * c + 1], D[2][r], q[3 * c + 2]);
             F[3 * c + r] = r == c ? sum + 1.f : sum;
         }
-    auto dot = [](const float* x, const float* y) { return x[0] * y[0] + x[1] * y[1] + x[2] * y[2]; };
-    const float c00 = dot(F, F), c11 = dot(F + 3, F + 3), c22 = dot(F + 6, F + 6);
-    const float c01 = dot(F, F + 3), c02 = dot(F, F + 6), c12 = dot(F + 3, F + 6);
-    const float CD = xsqrt<float>(c00 + c11 + c22);
+    float ss = fmaf(F[0], F[0], F[1] * F[1]);
+#pragma unroll
+    for (int i = 2; i < 9; i++) ss = fmaf(F[i], F[i], ss);
+    const float CD = xsqrt<float>(ss);
+    auto cross = [](float p, float r, float s, float t) { return fmaf(p, r, -(s * t)); };
     float Fc[9];
-    Fc[0] = F[4] * F[8] - F[5] * F[7];
-    Fc[1] = F[5] * F[6] - F[3] * F[8];
-    Fc[2] = F[3] * F[7] - F[4] * F[6];
-    Fc[3] = F[7] * F[2] - F[8] * F[1];
-    Fc[4] = F[8] * F[0] - F[6] * F[2];
-    Fc[5] = F[6] * F[1] - F[7] * F[0];
-    Fc[6] = F[1] * F[5] - F[2] * F[4];
-    Fc[7] = F[2] * F[3] - F[0] * F[5];
-    Fc[8] = F[0] * F[4] - F[1] * F[3];
-    const float J = dot(F, Fc);
-    const float a = J - 1.f;
+    Fc[0] = cross(F[4], F[8], F[5], F[7]);
+    Fc[1] = cross(F[5], F[6], F[3], F[8]);
+    Fc[2] = cross(F[3], F[7], F[4], F[6]);
+    Fc[3] = cross(F[7], F[2], F[8], F[1]);
+    Fc[4] = cross(F[8], F[0], F[6], F[2]);
+    Fc[5] = cross(F[6], F[1], F[7], F[0]);
+    Fc[6] = cross(F[1], F[5], F[2], F[4]);
+    Fc[7] = cross(F[2], F[3], F[0], F[5]);
+    Fc[8] = cross(F[0], F[4], F[1], F[3]);
+    const float J = sum3(F[0], Fc[0], F[1], Fc[1], F[2], Fc[2]);
+    const float a = J - 1.f, aa = a * a;
     const float ch_log = -gamma + xlog<float>(J);
-    const float ch_series = -gamma + a - a * a * 0.5f + a * a * a * (1.f / 3.f);
+    const float ch_series = fmaf(aa * a, 1.f / 3.f, fmaf(aa, -0.5f, a - gamma));
     const float CH = J >= 1.f ? ch_log : ch_series;
     const float inv_C = xrcp<float>(CD);
-    const float fac = (J >= 1.f) ? xrcp<float>(J) : 1.f - a + a * a;
-    const float s00 = M[0] * c00 + M[1] * c11 + M[2] * c22 + M[3] * c01 + M[4] * c02 + M[5] * c12;
-    const float s11 = M[0] * dot(Fc, Fc) + M[1] * dot(Fc + 3, Fc + 3) + M[2] * dot(Fc + 6, Fc + 6) +
-                      M[3] * dot(Fc, Fc + 3) + M[4] * dot(Fc, Fc + 6) + M[5] * dot(Fc + 3, Fc + 6);
-    const float s01 = J * (M[0] + M[1] + M[2]);
-    const float A00 = atD + s00 * (inv_C * inv_C), A11 = atH + s11 * (fac * fac), A01 = s01 * (inv_C * fac);
-    const float b0 = -CD - atD * lam.x;
-    const float b1 = -CH - atH * lam.y;
-    // a non-positive FP32 determinant (slivers) skips the projection, as in project_tet_F
-    const float det = A00 * A11 - A01 * A01;
-    const float inv_det = det > 0.f ? xrcp<float>(det) : 0.f;
-    const float d0 = (b0 * A11 - b1 * A01) * inv_det;
-    const float d1 = (b1 * A00 - b0 * A01) * inv_det;
-    lam.x += d0;
-    lam.y += d1;
-    const float e0 = d0 * inv_C, e1 = d1 * fac;
-    float G[9], g3[3] = { 0.f, 0.f, 0.f };
+    const float fac = (J >= 1.f) ? xrcp<float>(J) : fmaf(a, a, 1.f - a);
+    float gD[4][3], gH[4][3], w[4], dd[4], dh[4], hh[4];
 #pragma unroll
-    for (int i = 0; i < 9; i++) G[i] = e0 * F[i] + e1 * Fc[i];
+    for (int j = 0; j < 4; j++) {
+        float qj[3];
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+        for (int c = 0; c < 3; c++) qj[c] = j < 3 ? q[3 * c + j] : -(q[3 * c] + q[3 * c + 1] + q[3 * c + 2]);
 #pragma unroll
         for (int r = 0; r < 3; r++) {
-            const float g = G[r] * q[i] + G[3 + r] * q[3 + i] + G[6 + r] * q[6 + i];
-            g3[r] = i == 0 ? g : g3[r] + g;
-            d[i][r] += b[i].w * g;
+            gD[j][r] = inv_C * sum3(F[r], qj[0], F[3 + r], qj[1], F[6 + r], qj[2]);
+            gH[j][r] = fac * sum3(Fc[r], qj[0], Fc[3 + r], qj[1], Fc[6 + r], qj[2]);
         }
+        w[j] = b[j].w;
+        dd[j] = sum3(gD[j][0], gD[j][0], gD[j][1], gD[j][1], gD[j][2], gD[j][2]);
+        dh[j] = sum3(gD[j][0], gH[j][0], gD[j][1], gH[j][1], gD[j][2], gH[j][2]);
+        hh[j] = sum3(gH[j][0], gH[j][0], gH[j][1], gH[j][1], gH[j][2], gH[j][2]);
+    }
+    const float A01 = sum_of_products(w, dh);
+    const float A00 = atD + sum_of_products(w, dd), A11 = atH + sum_of_products(w, hh);
+    const float b0 = fmaf(-atD, lam.x, -CD), b1 = fmaf(-atH, lam.y, -CH);
+    // a non-positive FP32 determinant (slivers) skips the projection, as in project_tet_F
+    const float det = cross(A00, A11, A01, A01);
+    const float inv_det = det > 0.f ? xrcp<float>(det) : 0.f;
+    const float n0 = cross(b0, A11, b1, A01), n1 = cross(b1, A00, b0, A01);
+    const float d0 = n0 * inv_det, d1 = n1 * inv_det;
+    lam.x = fmaf(n0, inv_det, lam.x);
+    lam.y = fmaf(n1, inv_det, lam.y);
 #pragma unroll
-    for (int r = 0; r < 3; r++) d[3][r] -= b[3].w * g3[r];
+    for (int j = 0; j < 4; j++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) d[j][k] = fmaf(w[j], fmaf(gD[j][k], d0, gH[j][k] * d1), d[j][k]);
 }
 
 // The tile kernel with one lane a cluster: 64 clusters a block, N rows each
@@ -435,18 +458,23 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
     TileStage<kStageLane> g;
     tile_load(A, t, threadIdx.x, g);
     __builtin_amdgcn_sched_barrier(0);   // these return first
-    // a row: Q (9), alpha tilde D, H, gamma, M (6), four 16-bit slots (as byte offsets)
-    float4 S[RING][5];
+    // a row: Q (9), alpha tilde D, H, gamma; four 16-bit slots (as byte offsets)
+    float4 S[RING][3];
+    uint2 V[RING];
     float2 L[RING];
-    const float4* const st0 = A.stream + tw * A.rows * 320 + 128 + lane;   // 128: a row within +-2048 bytes
+    const float4* const st0 = A.stream + tw * A.rows * kLaneRow + lane;
+    const uint2* const sv0 = reinterpret_cast<const uint2*>(A.stream + tw * A.rows * kLaneRow + 192) + lane;
     float2* const sl0 = A.lam + tw * A.rows * 64 + lane;
     const int* home = A.home + tw * A.blocks * 64 + lane;   // 2 * first solver position + whether this copy writes dlam
     const float4* st = st0;   // the next row to load
+    const uint2* sv = sv0;
     auto load_row = [&](const float2* sl, int k, int c) {
 #pragma unroll
-        for (int p = 0; p < 5; p++) S[c][p] = st[p * 64 - 128];
+        for (int p = 0; p < 3; p++) S[c][p] = st[p * 64];
+        V[c] = *sv;
         if (!IMPORT) L[c] = sl[k * 64];
-        st += 320;
+        st += kLaneRow;
+        sv += 2 * kLaneRow;
     };
     int H = 0;
     const int nb = wave < A.waves ? head.x : 0;
@@ -474,7 +502,7 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
         uint32_t v[4];
         float4 b[4];
         auto load_base = [&](int c) {
-            const uint32_t i01 = __float_as_uint(S[c][4].z), i23 = __float_as_uint(S[c][4].w);
+            const uint32_t i01 = V[c].x, i23 = V[c].y;
             v[0] = i01 & 0xffffu;
             v[1] = i01 >> 16;
             v[2] = i23 & 0xffffu;
@@ -498,9 +526,8 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
 #pragma unroll
                 for (int k = 0; k < N; k++) {
                     const int c = k % RING;
-                    const float4 e0 = S[c][0], e1 = S[c][1], e2 = S[c][2], e3 = S[c][3], e4 = S[c][4];
+                    const float4 e0 = S[c][0], e1 = S[c][1], e2 = S[c][2];
                     const float q[9] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w, e2.x };
-                    const float M[6] = { e3.x, e3.y, e3.z, e3.w, e4.x, e4.y };
                     float2 l = L[c];
                     if (zero) l = make_float2(0.f, 0.f);
                     if (IMPORT) l = A.dlam[min((H >> 1) + k, A.nt - 1)];
@@ -520,7 +547,7 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
                         d[m][1] = f[m].y;
                         d[m][2] = f[m].z;
                     }
-                    project_lane(q, e2.y, e2.z, e2.w, M, bb, d, l);
+                    project_lane(q, e2.y, e2.z, e2.w, bb, d, l);
 #pragma unroll
                     for (int m = 0; m < 4; m++)
                         *reinterpret_cast<float4*>(lb + u[m] + 16 * CAP) = make_float4(d[m][0], d[m][1], d[m][2], 0.f);
@@ -528,7 +555,10 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
                     if (out) {
                         if ((H & 1) && u[0] != 16u * (A.slots - 1)) A.dlam[(H >> 1) + k] = l;
                     }
-                    if (k + RING == N && wrap) st = st0;
+                    if (k + RING == N && wrap) {
+                        st = st0;
+                        sv = sv0;
+                    }
                     load_row(k + RING < N ? sl : sln, k + RING < N ? k + RING : k + RING - N, c);
                 }
                 for (int n = cur >> 4; n > 0; n--) lds_barrier();
@@ -553,8 +583,8 @@ __global__ __launch_bounds__(256) void k_gs_tile_lane_fill(GsTileFill A)
     const int rows = A.list[b] & 15;
     const size_t row = (size_t)A.row[b];
     for (int k = 0; k < rows; k++) {
-        float f[20];
-        for (int m = 0; m < 20; m++) f[m] = 0.f;
+        float f[12];
+        for (int m = 0; m < 12; m++) f[m] = 0.f;
         uint32_t v[4];
         for (int m = 0; m < 4; m++) v[m] = (uint32_t)(A.slots - 1);
         if (k < n) {
@@ -564,28 +594,11 @@ __global__ __launch_bounds__(256) void k_gs_tile_lane_fill(GsTileFill A)
             f[9] = at.x;
             f[10] = at.y;
             f[11] = A.ta.gamma[e];
-            const int4 t = A.ta.tet[e];
-            const int vid[4] = { t.x, t.y, t.z, t.w };
-            double M[6] = { 0.0, 0.0, 0.0, 0.0, 0.0, 0.0 };
-            for (int m = 0; m < 4; m++) {
-                double x[3];
-                for (int cc = 0; cc < 3; cc++)
-                    x[cc] = m < 3 ? (double)f[3 * cc + m] : (double)f[3 * cc] + (double)f[3 * cc + 1] + (double)f[3 * cc + 2];
-                const double w = (double)A.pos[2 * (size_t)vid[m]].w;
-                M[0] += w * x[0] * x[0];
-                M[1] += w * x[1] * x[1];
-                M[2] += w * x[2] * x[2];
-                M[3] += 2.0 * w * x[0] * x[1];
-                M[4] += 2.0 * w * x[0] * x[2];
-                M[5] += 2.0 * w * x[1] * x[2];
-                v[m] = A.vert[(size_t)i * 8 + ((A.tloc[e] >> (4 * m)) & 15u)];
-            }
-            for (int m = 0; m < 6; m++) f[12 + m] = (float)M[m];
+            for (int m = 0; m < 4; m++) v[m] = A.vert[(size_t)i * 8 + ((A.tloc[e] >> (4 * m)) & 15u)];
         }
-        f[18] = __uint_as_float(16 * v[0] | v[1] << 20);
-        f[19] = __uint_as_float(16 * v[2] | v[3] << 20);
-        for (int p = 0; p < 5; p++)
-            A.stream[((row + k) * 5 + p) * 64 + lane] = make_float4(f[4 * p], f[4 * p + 1], f[4 * p + 2], f[4 * p + 3]);
+        float4* const st = A.stream + (row + k) * kLaneRow;
+        for (int p = 0; p < 3; p++) st[p * 64 + lane] = make_float4(f[4 * p], f[4 * p + 1], f[4 * p + 2], f[4 * p + 3]);
+        reinterpret_cast<uint2*>(st + 192)[lane] = make_uint2(16 * v[0] | v[1] << 20, 16 * v[2] | v[3] << 20);
         A.lam[(row + k) * 64 + lane] = make_float2(0.f, 0.f);
     }
 }

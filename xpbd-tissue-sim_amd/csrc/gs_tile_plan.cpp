@@ -60,7 +60,7 @@ int upload(xpbd_handle* h, const GsTileGroup& G, const GsTileDeal& deal, const G
     if (!rc) rc = put(h, &own, G.own);
     if (!rc) rc = put(h, &vert, G.vert);
     if (!rc && shape.lanes == 1) rc = room(h, &home, (size_t)nblocks * deal.per_block);
-    if (!rc) rc = room(h, &stream, rows * 64 * (shape.lanes == 1 ? 5 : 1));
+    if (!rc) rc = room(h, &stream, rows * (shape.lanes == 1 ? kLaneRow : 64));
     if (!rc) rc = room(h, &lam, rows * deal.per_block);
     if (!rc) rc = room(h, &L.d[0], slots);
     if (rc) return rc;
@@ -113,8 +113,8 @@ struct TileTry {
 // One plan from the mesh's size.  P is the most clusters of a colour, tp = P over
 // the compute units, the clusters of a colour that a tile owns when every unit
 // has one workgroup: with more tiles than units the launch takes a second round
-// for the rest (56^3 cells, one lane a cluster, 3 colours: 556 us a step of 10
-// iterations with 256 tiles, 868 us with 400).
+// for the rest (56^3 cells, one lane a cluster: 1.56 times as long with 400 tiles as
+// with 256).
 //
 // whole: every instance a tile, all colours in a launch, all iterations too while
 // no contacts come between: few enough clusters that each SIMD of one unit has
@@ -123,19 +123,21 @@ struct TileTry {
 // colours, where copies would be most of the work (51 colours of 4,448 elements:
 // 853 against 1,922).
 //
-// Four lanes a cluster where a tile's phases then fill at most about one wave a
-// SIMD: shortest chain (36^3: 390 us, one lane 435).  One lane above, half the
-// instructions for a cluster (beam 200x20x20: 433, four lanes 479; 56^3: 556,
-// four lanes 793).  More colours a launch save launches and cost copies: four
-// while a tile's fullest phase still has a wave for each SIMD and no more.
-// Above tp = 175 (2.1M elements) the copies' traffic is what a launch takes:
-// no plan, colour launches (75^3: 1,272 against 1,315).
+// Four lanes a cluster have the shorter chain, one lane half the instructions for a
+// cluster.  Up to tp = 65 a phase's chain counts (us a step of 10 iterations, four
+// lanes and 2 colours a launch, against the best of one lane: 36^3 363 and 487, beam
+// 200x20x20 476 and 506, 46^3 519 and 519, 50^3 549 and 549), above the instructions
+// (56^3 679 and 611, 66^3 905 and 739).  More colours a launch save launches and cost
+// copies: four while the colours are small (30^3 340, 2 colours 360), three with one
+// lane while a tile's fullest phase has a wave for each SIMD and no more (56^3 611,
+// 2 colours 649; 66^3 805 and 739).
+// Above tp = 175 (2.1M elements) the copies' traffic is what a launch takes: no plan,
+// colour launches (75^3: 1,272 against 1,315).
 void tile_tries(int tp, std::vector<TileTry>& t)
 {
     if (tp <= 11) t.push_back({ 4, 4, 16, 32 });
-    if (tp <= 34) t.push_back({ 2, 4, 16, 22 });
+    if (tp <= 65) t.push_back({ 2, 4, 64, 22 });
     else if (tp <= 175) {
-        if (tp <= 70) t.push_back({ 4, 1, 4, 22 });
         if (tp <= 90) t.push_back({ 3, 1, 4, 22 });
         t.push_back({ 2, 1, 8, 22 });
     }
