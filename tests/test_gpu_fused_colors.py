@@ -122,6 +122,7 @@ LANE = {
     "cube": lambda: _grid(52, 52, 52),
     "ragged": lambda: _grid(91, 43, 37),
     "two colours": lambda: _grid(61, 59, 60),
+    "three million elements": lambda: _grid(81, 79, 80),
     "8-element clusters": lambda: _eight_element_cells(52, 53, 51, seed=23),
 }
 

@@ -6,7 +6,7 @@
 // cluster kernel and the quad kernel at 64, 128 or 256 threads per workgroup
 // and to the fused-colour launches (gs_tiles.h)
 // without rebuilding anything (same clusters, colours and order, so the same
-// results up to FP32 summation order within an element).  Patch Jacobi handles
+// results; the one-thread kernel up to FP32 summation order within an element).  Patch Jacobi handles
 // time the fused one-launch iteration against the patch + shared-vertex +
 // contact launches (the same sums; with contacts the contact corrections are
 // added in another order).  Cluster and patch kernels are also timed with and

@@ -42,7 +42,6 @@ struct GsTileArgs {
 
 struct GsTileFill {
     TetArrays ta;
-    const float4* pos;       // vertex records (inverse masses)
     const int* cstart;
     const uint32_t* tloc;
     const int* list;

@@ -69,7 +69,6 @@ int upload(xpbd_handle* h, const GsTileGroup& G, const GsTileDeal& deal, const G
     if (e != hipSuccess) return hip_err(h, e, "tile set-up");
     GsTileFill F{};
     F.ta = tet_arrays(h);
-    F.pos = h->d_pos;
     F.cstart = h->d_cstart;
     F.tloc = h->d_tloc;
     F.list = list;
@@ -128,16 +127,18 @@ struct TileTry {
 // lanes and 2 colours a launch, against the best of one lane: 36^3 363 and 487, beam
 // 200x20x20 476 and 506, 46^3 519 and 519, 50^3 549 and 549), above the instructions
 // (56^3 679 and 611, 66^3 905 and 739).  More colours a launch save launches and cost
-// copies: four while the colours are small (30^3 340, 2 colours 360), three with one
-// lane while a tile's fullest phase has a wave for each SIMD and no more (56^3 611,
-// 2 colours 649; 66^3 805 and 739).
-// Above tp = 175 (2.1M elements) the copies' traffic is what a launch takes: no plan,
-// colour launches (75^3: 1,272 against 1,315).
+// copies: four while the colours are small (10^3 253, 2 colours 293; 16^3 255 and 291;
+// level from 20^3 on, 302 and 305), three with one lane while a tile's fullest phase
+// has a wave for each SIMD and no more (56^3 611, 2 colours 649; 66^3 805 and 739).
+// Two launches' phases hold up to 8 blocks of 64 clusters, a wave each.  Where they
+// fit they win (72^3 990, colour launches 1,085; 80^3 1,044 and 1,312; 96^3, tp = 432,
+// 1,562 and 2,156).  Where a tile's phases or vertices do not fit (88^3), and above
+// tp = 512, there is no plan.
 void tile_tries(int tp, std::vector<TileTry>& t)
 {
     if (tp <= 11) t.push_back({ 4, 4, 16, 32 });
     if (tp <= 65) t.push_back({ 2, 4, 64, 22 });
-    else if (tp <= 175) {
+    else if (tp <= 512) {
         if (tp <= 90) t.push_back({ 3, 1, 4, 22 });
         t.push_back({ 2, 1, 8, 22 });
     }
