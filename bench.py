@@ -40,6 +40,16 @@ sys.path.insert(0, os.path.join(ROOT, "xpbd-tissue-sim_amd"))
 HBM_PEAK_GBS = 8000.0
 KERNEL_NAMES = {"cluster": "k_gs_cluster x colours", "quad": "k_gs_cluster_quad x colours",
                 "simple": "k_gs_color x colours / k_jacobi_project", "patch": "k_jacobi_patch + k_jacobi_shared"}
+
+
+def kernel_name(launch):
+    if launch[0] == "quad" and launch[1] == 4000:
+        return "k_gs_tile / k_gs_tile_lane, several colours a launch"
+    if launch[0] == "patch" and launch[1] == 2:
+        return "k_jacobi_tile"
+    return KERNEL_NAMES.get(launch[0], launch[0])
+
+
 METRIC = "sim steps/sec & tet projections/sec at equal residual, learned vs plain, 1 GPU"
 
 
@@ -167,7 +177,7 @@ def measure(s, cfg, workload, steps, warmup, timing_steps, no_graph=False, tune_
     traffic, traffic_kernel, note = traffic_for(workload, cfg["solver"], launch)
     roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-            "kernel": KERNEL_NAMES.get(launch[0], launch[0]) + " (one solver iteration)",
+            "kernel": kernel_name(launch) + " (one solver iteration)",
             "launch_config": launch, "us_per_iteration": us_per_iter,
             "algorithmic_bytes_per_iteration": bytes_iter, "iterations_timed": nit, "graph_replay": not no_graph}
     if traffic_kernel:
