@@ -894,6 +894,19 @@ int enqueue_finish(xpbd_handle* h, const MotionSource& from)
     return e == hipSuccess ? XPBD_OK : hip_err(h, e, "finish launch");
 }
 
+// Where the tile launches of a warm-started solve find the multipliers that it keeps.
+// Tiles share elements, each copy starts from the multipliers in solver order, and one
+// of the copies writes them back after the last iteration.  A solve of one iteration
+// would do both in the same launch, with nothing to order a tile's reads before another's
+// writes: it reads from a copy.  (Closed plans share nothing.)
+static hipError_t kept_multipliers(xpbd_handle* h, int iters, bool closed, float2* copy, const float2** kept)
+{
+    *kept = h->d_lam;
+    if (iters != 1 || closed) return hipSuccess;
+    *kept = copy;
+    return hipMemcpyAsync(copy, h->d_lam, sizeof(float2) * (size_t)h->nt, hipMemcpyDeviceToDevice, h->stream);
+}
+
 // The iterations by fused-colour launches (gs_tiles.h).  A launch reads its
 // group's slots and writes the next group's; a closed plan's tiles depend on
 // nothing outside them and update in place, all iterations in one launch when
@@ -911,6 +924,9 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
     hipError_t e = launch_gs_tile_load(s, h->d_pos, P.slot_vert, P.nslots, P.launches[0].nslots, P.launches[0].d[0],
                                        P.base, ends.predict ? &predict : nullptr, ends.hits ? &hits : nullptr);
     if (e != hipSuccess) return hip_err(h, e, "gs_tile_load launch");
+    const float2* kept = nullptr;
+    if (!reset_lambda) e = kept_multipliers(h, iters, P.closed, P.kept, &kept);
+    if (e != hipSuccess) return hip_err(h, e, "kept multipliers");
     for (int it = 0, inner; it < iters; it += inner) {
         const bool import = it == 0 && !reset_lambda;
         inner = P.closed && !con && !import ? iters - it : 1;
@@ -920,6 +936,7 @@ static int enqueue_tiled_iterations(xpbd_handle* h, int iters, bool timed, bool 
             GsTileArgs A = L.args;
             A.din = L.d[swap ? cur : 0];
             A.dout = swap ? L.d[1 - cur] : P.launches[(g + 1) % ng].d[0];
+            A.kept = kept;
             A.niter = inner;
             A.lam_zero = it == 0 && reset_lambda;
             A.lam_out = it + inner == iters;
@@ -961,12 +978,16 @@ static int enqueue_tiled_jacobi(xpbd_handle* h, int iters, bool timed, bool rese
     hipError_t e = launch_gs_tile_load(s, h->d_pos, P.args.vert, P.nslots, P.nslots, P.d[0], P.base,
                                        ends.predict ? &predict : nullptr, ends.hits ? &hits : nullptr);
     if (e != hipSuccess) return hip_err(h, e, "gs_tile_load launch");
+    const float2* kept = nullptr;
+    if (!reset_lambda) e = kept_multipliers(h, iters, P.closed, P.kept, &kept);
+    if (e != hipSuccess) return hip_err(h, e, "kept multipliers");
     int cur = 0;
     for (int it = 0, inner; it < iters; it += inner) {
         inner = P.closed ? iters : 1;
         JacobiTileArgs A = P.args;
         A.din = P.d[cur];
         A.dout = P.d[1 - cur];
+        A.kept = kept;
         A.niter = inner;
         A.xcd = h->xcd_map ? 1 : 0;
         A.lam_zero = it == 0 && reset_lambda;

@@ -31,6 +31,7 @@ struct JacobiTilePlan {
     float4* d[2] = {};                   // motions by slot, in turn
     float4* base = nullptr;
     const int32_t* owner = nullptr;      // vertex -> its owner's slot
+    float2* kept = nullptr;              // not closed: solver-order multipliers of a warm start (kept_multipliers)
     int nslots = 0, threads = 0;
 };
 
@@ -45,6 +46,7 @@ struct GsTilePlan {
     const int32_t* owner = nullptr;      // vertex -> the owner's slot of the first group
     const int32_t* copy_off = nullptr;   // vertex -> its slots of the first group
     const int32_t* copy = nullptr;
+    float2* kept = nullptr;              // not closed: solver-order multipliers of a warm start (kept_multipliers)
 };
 }
 

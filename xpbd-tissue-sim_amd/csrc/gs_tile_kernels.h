@@ -31,6 +31,8 @@ struct GsTileArgs {
                              // One lane a cluster, kLaneRow per row: see k_gs_tile_lane
     float2* lam;             // 16 (64) per row; with four lanes a block's first row: as home
     float2* dlam;            // solver order
+    const float2* kept;      // solver order, what an import reads: not dlam where this launch writes that and tiles
+                             // share clusters
     const float4* din;       // in-step motion, by slot of this group
     float4* dout;            // by slot of the next
     const float4* base;      // base displacement, inverse mass, by slot
@@ -59,7 +61,7 @@ size_t gs_tile_smem(int slots, const GsTileShape& S);
 int gs_tile_cap(int slots);   // 0: too many for one lane a cluster
 // once per shape, outside any capture: lets the kernel use kGsTileLds bytes of LDS
 hipError_t gs_tile_prepare(const GsTileShape& S);
-// import: the first iteration's multipliers come from dlam
+// import: the first iteration's multipliers come from kept
 hipError_t launch_gs_tile(hipStream_t s, const GsTileArgs& A, const GsTileShape& S, int ntiles, int threads, size_t smem,
                           bool import);
 hipError_t launch_gs_tile_fill(hipStream_t s, const GsTileFill& A, const GsTileShape& S);

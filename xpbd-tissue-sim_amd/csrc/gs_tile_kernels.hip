@@ -175,7 +175,7 @@ __device__ __forceinline__ void tile_write(const GsTileArgs& A, const TileOut& r
 // launch loads its first one again, so that every path issues the same loads
 // and the waits count them exactly.
 // FULL: every block has MT element rows (each cluster a hexahedral cell).
-// IMPORT: the multipliers come from the solver-order array (launches of one iteration).
+// IMPORT: the multipliers come from a solver-order array (launches of one iteration).
 template <int MT, bool FULL, bool IMPORT>
 __global__ __launch_bounds__(1024) void k_gs_tile(GsTileArgs A)
 {
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(1024) void k_gs_tile(GsTileArgs A)
     auto load_row = [&](const float4* st, const float2* sl, int k, int rows, bool import, int h) {
         const int r = 1 + (FULL ? k : max(0, min(k, rows - 1)));
         S[k] = st[r * 64];
-        L[k] = import ? A.dlam[min((h >> 1) + k, A.nt - 1)] : sl[r * 16];
+        L[k] = import ? A.kept[min((h >> 1) + k, A.nt - 1)] : sl[r * 16];
     };
     const int nb = wave < A.waves ? head.x : 0;
     auto first_rows = [&] {
@@ -530,7 +530,7 @@ __global__ __launch_bounds__(512) void k_gs_tile_lane(GsTileArgs A)
                     const float q[9] = { e0.x, e0.y, e0.z, e0.w, e1.x, e1.y, e1.z, e1.w, e2.x };
                     float2 l = L[c];
                     if (zero) l = make_float2(0.f, 0.f);
-                    if (IMPORT) l = A.dlam[min((H >> 1) + k, A.nt - 1)];
+                    if (IMPORT) l = A.kept[min((H >> 1) + k, A.nt - 1)];
                     uint32_t u[4];
                     float4 bb[4], f[4];
 #pragma unroll

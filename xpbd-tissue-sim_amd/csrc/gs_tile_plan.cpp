@@ -269,6 +269,7 @@ int make_tiles(xpbd_handle* h)
     if (!rc) rc = put(h, &P.owner, G[0].owner);
     if (!rc) rc = put(h, &P.copy_off, off);
     if (!rc) rc = put(h, &P.copy, copy);
+    if (!rc && !P.closed) rc = room(h, &P.kept, (size_t)h->nt);
     // one group that is not closed reads and writes its own slots: two arrays in turn
     if (!rc && G.size() == 1 && !P.closed) {
         rc = room(h, &launches[0].d[1], (size_t)launches[0].nslots);

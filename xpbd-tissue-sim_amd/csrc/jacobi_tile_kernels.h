@@ -18,6 +18,8 @@ struct JacobiTileArgs {
     const int2* out;
     float2* lam;              // per tile element
     float2* dlam;             // solver order
+    const float2* kept;       // solver order, what an import reads: not dlam where this launch writes that and tiles
+                              // share elements
     const float4* din;        // in-step motion by slot
     float4* dout;
     const float4* base;       // base displacement, inverse mass by slot
@@ -26,7 +28,7 @@ struct JacobiTileArgs {
     int verts, slots;         // room in LDS
     int niter, ntiles, xcd;
     int lam_zero;             // the first iteration's multipliers are zero
-    int import;               // they are dlam's
+    int import;               // they are kept's
     int lam_out;              // the last iteration also writes dlam
     // contacts
     int late;                 // added after all elements

@@ -94,7 +94,7 @@ __device__ __forceinline__ void load_tile_tet(const JacobiTileArgs& A, int i, bo
     t.q[0] = a.x, t.q[1] = a.y, t.q[2] = a.z, t.q[3] = a.w;
     t.q[4] = b.x, t.q[5] = b.y, t.q[6] = b.z, t.q[7] = b.w;
     t.q[8] = c.x, t.atD = c.y, t.atH = c.z, t.gm = c.w;
-    t.l = first && A.lam_zero ? make_float2(0.f, 0.f) : first && A.import ? A.dlam[A.home[i] >> 1] : A.lam[i];
+    t.l = first && A.lam_zero ? make_float2(0.f, 0.f) : first && A.import ? A.kept[A.home[i] >> 1] : A.lam[i];
 }
 
 // An element's projection from the tile's motions; corrections of own vertices to their slots.

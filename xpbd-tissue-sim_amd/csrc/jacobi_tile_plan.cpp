@@ -96,6 +96,7 @@ int make_tiles(xpbd_handle* h)
     if (!rc) rc = room(h, &A.lam, n);
     if (!rc) rc = room(h, &base, slots);
     for (int i = 0; i < 2 && !rc; i++) rc = room(h, &P.d[i], slots);
+    if (!rc && !J.closed) rc = room(h, &P.kept, (size_t)h->nt);
     if (rc) return rc;
     e = launch_fill_zero(h->stream, A.lam, sizeof(float2) * n);
     for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_fill_zero(h->stream, P.d[i], sizeof(float4) * slots);
