@@ -163,7 +163,7 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
                             L.fits = false;
                             continue;
                         }
-                        const int32_t* te = &tlist[toff[v]];
+                        const int32_t* te = tlist.data() + toff[v];   // past the end for a last vertex without elements
                         mine.assign(flist.begin() + foff[v], flist.begin() + foff[v + 1]);
                         std::sort(mine.begin(), mine.end(), by_patch);
                         uint64_t end = 0, con = 0;
