@@ -46,9 +46,13 @@ static int dalloc(xpbd_handle* h, T** p, size_t n)
 {
     *p = nullptr;
     if (n == 0) n = 1;
+    h->allocs.push_back(nullptr);   // its place first: this may throw
     hipError_t e = hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T));
-    if (e != hipSuccess) return set_err(h, XPBD_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
-    h->allocs.push_back(*p);
+    if (e != hipSuccess) {
+        h->allocs.pop_back();
+        return set_err(h, XPBD_E_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
+    }
+    h->allocs.back() = *p;
     return XPBD_OK;
 }
 

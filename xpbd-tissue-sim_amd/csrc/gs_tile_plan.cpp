@@ -5,14 +5,12 @@
 #include <algorithm>
 #include <atomic>
 #include <exception>
-#include <new>
-#include <system_error>
-#include <thread>
 #include <utility>
 
 #include "capi_internal.h"
 #include "gs_tile_kernels.h"
 #include "gs_tiles.h"
+#include "host_threads.h"
 
 using namespace xpbd;
 
@@ -154,26 +152,16 @@ bool build_groups(const GsClusters& C, int nc, int m, int tp, bool whole, const 
         try {
             const int c0 = (int)g * m, c1 = std::min(nc, c0 + m), n = C.color_off[c1] - C.color_off[c0];
             build_gs_tiles(C, c0, c1, whole ? 0 : (n + (c1 - c0) * tp - 1) / ((c1 - c0) * tp), deal, G[g]);
-        } catch (const std::bad_alloc&) {
+        } catch (const std::exception&) {
             bad[g] = 1;
         }
     };
-    std::vector<std::thread> pool;
     // threads pay for themselves on meshes that take a thread some milliseconds
     const size_t nthreads = C.color_off[nc] < 20000 ? 1 : std::min<size_t>(4, G.size());
     std::atomic<size_t> next{ 0 };
-    auto work = [&] {
+    on_threads(nthreads, [&] {
         for (size_t g; (g = next++) < G.size();) build(g);
-    };
-    for (size_t i = 1; i < nthreads; i++) {
-        try {
-            pool.emplace_back(work);
-        } catch (const std::system_error&) {
-            break;   // no thread to be had: this one does it all
-        }
-    }
-    work();
-    for (auto& t : pool) t.join();
+    });
     return std::find(bad.begin(), bad.end(), 1) == bad.end();
 }
 
@@ -295,7 +283,7 @@ int xpbd::ensure_gs_tiles(xpbd_handle* h)
     int rc;
     try {
         rc = make_tiles(h);
-    } catch (const std::exception&) {   // host memory
+    } catch (const std::exception&) {   // host memory: a text that needs none
         rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }
     if (rc) {   // the handle goes on with its other launch shapes

@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <exception>
-#include <thread>
 
 #include "capi_internal.h"
 #include "jacobi_tile_kernels.h"
@@ -137,8 +136,8 @@ int xpbd::ensure_jacobi_tiles(xpbd_handle* h)
     int rc;
     try {
         rc = make_tiles(h);
-    } catch (const std::exception&) {   // host memory
-        rc = set_err(h, XPBD_E_NOMEM, "Jacobi tile plan");
+    } catch (const std::exception&) {   // host memory: a text that needs none
+        rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }
     if (rc) {   // the handle goes on with its other launch shapes
         for (; h->allocs.size() > kept; h->allocs.pop_back()) (void)hipFree(h->allocs.back());

@@ -3,9 +3,9 @@
 #include <algorithm>
 #include <atomic>
 #include <cstddef>
-#include <new>
-#include <system_error>
-#include <thread>
+#include <exception>
+
+#include "host_threads.h"
 
 namespace xpbd {
 
@@ -215,20 +215,11 @@ bool build_jacobi_tiles(const JacobiMesh& M, int parts, int threads, JacobiTiles
                 L.fits = L.fits && L.vert.size() < 0x7fff && L.slots < 0xffff;
                 if (!L.fits) bad = true;
             }
-        } catch (const std::bad_alloc&) {
+        } catch (const std::exception&) {
             bad = true;
         }
     };
-    std::vector<std::thread> pool;
-    for (int i = 1; i < std::min(threads, J.ntiles); i++) {
-        try {
-            pool.emplace_back(work);
-        } catch (const std::system_error&) {
-            break;   // no thread to be had: those there are do it all
-        }
-    }
-    work();
-    for (auto& t : pool) t.join();
+    on_threads(std::min(threads, J.ntiles), work);
     if (bad) return false;
     // side by side
     J.owner.assign(nv, 0);
