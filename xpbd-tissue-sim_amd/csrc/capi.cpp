@@ -484,15 +484,17 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
     rc |= dalloc(h, &h->d_cn, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_cb, 3 * (size_t)nf);
     rc |= dalloc(h, &h->d_clam, nf);
-    // state readers: two pieces of pinned memory
+    // state readers: two pieces of pinned memory, or none (read_records)
     if (rc == XPBD_OK) {
         h->read_bytes = std::min<size_t>(kReadPiece, 3 * sizeof(double) * (size_t)nv);
-        hipError_t re = hipHostMalloc(reinterpret_cast<void**>(&h->h_read), 2 * h->read_bytes, hipHostMallocDefault);
+        hipError_t re = hipSuccess;
         for (hipEvent_t& ev : h->read_done)
             if (re == hipSuccess) re = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (re == hipSuccess)
+            re = hipHostMalloc(reinterpret_cast<void**>(&h->h_read), 2 * h->read_bytes, hipHostMallocDefault);
         if (re != hipSuccess) {
             (void)hipGetLastError();
-            rc = XPBD_E_NOMEM;
+            h->h_read = nullptr;
         }
     }
     // Gauss-Seidel contacts: room for what a solve's first contact pass leaves to
@@ -1402,6 +1404,27 @@ int download_f4(xpbd_handle* h, std::vector<float4>& hu, const float4* src, size
 }
 }  // namespace xpbd
 
+// What read_state does, by copies of the records, for handles without pinned memory.
+template <typename T>
+static int read_records(xpbd_handle* h, bool velocities, int64_t v0, int64_t v1, T* out)
+{
+    std::vector<float4> hp, hl;
+    int rc = velocities ? download_f4(h, hp, h->d_vel, h->nv) : download_f4(h, hp, h->d_pos, 2 * (size_t)h->nv);
+    if (!rc && !velocities) rc = download_f4(h, hl, h->d_lo, h->nv);
+    if (rc) return rc;
+    for (int64_t i = v0; i < v1; i++, out += 3) {
+        if (velocities) {
+            out[0] = (T)hp[i].x, out[1] = (T)hp[i].y, out[2] = (T)hp[i].z;
+            continue;
+        }
+        const float4 b = hp[2 * i], d = hp[2 * i + 1], l = hl[i];
+        out[0] = (T)(h->rest[3 * i] + ((double)b.x + (double)l.x + (double)d.x));
+        out[1] = (T)(h->rest[3 * i + 1] + ((double)b.y + (double)l.y + (double)d.y));
+        out[2] = (T)(h->rest[3 * i + 2] + ((double)b.z + (double)l.z + (double)d.z));
+    }
+    return XPBD_OK;
+}
+
 // position = rest + base + low part + in-step motion (zero between steps), or the
 // velocity, of vertices [v0, v1).  The kernel packs a caller's 12 or 24 bytes a vertex
 // (the records hold 48) straight into pinned host memory, and the host copies them
@@ -1411,6 +1434,9 @@ int download_f4(xpbd_handle* h, std::vector<float4>& hu, const float4* src, size
 // into device memory and copied from there: 14, 49 and 151 each.
 static int read_state(xpbd_handle* h, bool velocities, int64_t v0, int64_t v1, bool f32, void* out)
 {
+    if (!h->h_read)
+        return f32 ? read_records(h, velocities, v0, v1, static_cast<float*>(out))
+                   : read_records(h, velocities, v0, v1, static_cast<double*>(out));
     const size_t per = 3 * (f32 ? sizeof(float) : sizeof(double));
     const int64_t piece = (int64_t)(h->read_bytes / per);
     std::lock_guard<std::mutex> lock(h->read_mutex);

@@ -84,8 +84,8 @@ struct xpbd_handle {
     // are one run: fci_off[c * (ninst + 1) + i] is where instance i's faces of
     // colour c start (i = ninst: the colour's end)
     std::vector<int32_t> fci_off;
-    // what the state's readers are given, in two pieces of pinned memory; for one
-    // reader at a time
+    // what the state's readers are given, in two pieces of pinned memory (null: none to
+    // be had); for one reader at a time
     std::mutex read_mutex;
     char* h_read = nullptr;
     size_t read_bytes = 0;   // of a piece
