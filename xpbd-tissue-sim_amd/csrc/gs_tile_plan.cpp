@@ -113,7 +113,7 @@ struct TileTry {
 // for the rest (56^3 cells, one lane a cluster: 1.56 times as long with 400 tiles as
 // with 256).
 //
-// whole: every instance a tile, all colours in a launch, all iterations too while
+// whole: every instance a tile (or several, pack_instances), all colours in a launch, all iterations too while
 // no contacts come between: few enough clusters that each SIMD of one unit has
 // one wave (4^3 cells: 196 us against 381 us for colour launches, 8^3: 211
 // against 407; 10^3, two waves each: 316, against 256 below), or many small
@@ -140,6 +140,41 @@ void tile_tries(int tp, std::vector<TileTry>& t)
         if (tp <= 90) t.push_back({ 3, 1, 4, 22 });
         t.push_back({ 2, 1, 8, 22 });
     }
+}
+
+// Of a batch of more objects than units, most of them small beside the largest:
+// several objects a tile.  All tiles of a group are stored alike (gs_tiles.h), so with an
+// object each they would take, and stage, the largest object's slots times their number
+// (10,000 cells and a cube of 8^3: 3.0 GB and 515 us a step of 10 iterations, with contacts
+// 1,957, where colour launches take 450 and 1,347; packed 0.1 GB, 211 and 1,113; 1,000
+// cubes of 4^3 and one of 8^3 314 us, packed 275).  As many tiles as units, none larger than the largest object, none with more clusters of a colour than
+// `most`.  cinst: instance of each cluster, then its tile.
+void pack_instances(const xpbd_handle* h, int units, int64_t largest, int most, std::vector<int32_t>& cinst)
+{
+    const int64_t nv = h->nv;
+    if (h->ninst <= units || h->ninst * largest <= 4 * nv) return;
+    const int nc = h->ncolors;
+    const int64_t room = std::min(largest, (nv + units - 1) / units);
+    std::vector<int32_t> count((size_t)h->ninst * nc, 0), held(nc, 0), tile(h->ninst);
+    for (int c = 0; c < nc; c++)
+        for (int i = h->color_off[c]; i < h->color_off[c + 1]; i++) count[(size_t)cinst[i] * nc + c]++;
+    int64_t verts = 0;
+    int t = 0;
+    for (int i = 0; i < h->ninst; i++) {
+        const int32_t* n = &count[(size_t)i * nc];
+        const int64_t v = h->v_off[i + 1] - h->v_off[i];
+        bool fits = verts + v <= room;
+        for (int c = 0; c < nc; c++) fits = fits && held[c] + n[c] <= most;
+        if (!fits && verts > 0) {
+            t++;
+            verts = 0;
+            std::fill(held.begin(), held.end(), 0);
+        }
+        verts += v;
+        for (int c = 0; c < nc; c++) held[c] += n[c];
+        tile[i] = t;
+    }
+    for (int32_t& i : cinst) i = tile[i];
 }
 
 // The groups of one try, on a thread each; false if memory ran out.
@@ -208,9 +243,13 @@ int make_tiles(xpbd_handle* h)
     }
     const GsClusters C{ h->nv, cverts, h->color_off, h->cl_start, cinst, centre };
     const int rows = h->cluster_max_tets <= 6 ? 6 : 8;
-    const bool whole = whole_most <= (nc > 16 ? 256 : 64) && verts < 65535 &&
+    const int whole_limit = nc > 16 ? 256 : 64;
+    const bool whole = whole_most <= whole_limit && verts < 65535 &&
                        gs_tile_smem((int)verts + 1, GsTileShape{}) <= kGsTileLds;
-    if (whole) tries = { { nc, 4, 1 << 30, 1 << 20 } };
+    if (whole) {
+        tries = { { nc, 4, 1 << 30, 1 << 20 } };
+        pack_instances(h, units, verts, whole_limit, cinst);
+    }
     std::vector<GsTileGroup> G;
     GsTileDeal deal{};
     for (const TileTry& t : tries) {

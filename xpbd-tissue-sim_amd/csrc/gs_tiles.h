@@ -67,7 +67,7 @@ struct GsClusters {
     const std::vector<float>& centre;
 };
 // Cuts colours [c0, c1) into `parts` tiles (at most one per cluster), or with
-// parts <= 0 makes every instance a tile.
+// parts <= 0 makes every instance (every value of cinst) a tile.
 void build_gs_tiles(const GsClusters& C, int c0, int c1, int parts, const GsTileDeal& deal, GsTileGroup& G);
 // Slots of each vertex: copy[off[v] .. off[v + 1]).
 void gs_tile_copies(int nv, const GsTileGroup& G, std::vector<int32_t>& off, std::vector<int32_t>& copy);
