@@ -11,6 +11,7 @@
 #include "gs_tile_kernels.h"
 #include "gs_tiles.h"
 #include "host_threads.h"
+#include "pack.h"
 
 using namespace xpbd;
 
@@ -142,38 +143,24 @@ void tile_tries(int tp, std::vector<TileTry>& t)
     }
 }
 
-// Of a batch of more objects than units, most of them small beside the largest:
-// several objects a tile.  All tiles of a group are stored alike (gs_tiles.h), so with an
-// object each they would take, and stage, the largest object's slots times their number
-// (10,000 cells and a cube of 8^3: 3.0 GB and 515 us a step of 10 iterations, with contacts
-// 1,957, where colour launches take 450 and 1,347; packed 0.1 GB, 211 and 1,113; 1,000
-// cubes of 4^3 and one of 8^3 314 us, packed 275).  As many tiles as units, none larger than the largest object, none with more clusters of a colour than
-// `most`.  cinst: instance of each cluster, then its tile.
-void pack_instances(const xpbd_handle* h, int units, int64_t largest, int most, std::vector<int32_t>& cinst)
+// Of a batch of more objects than units: several small objects a tile, as many tiles as
+// units, none of them with more clusters of a colour than `most`.  With an object a tile
+// the launch takes rounds of tiles that each leave a wave's lanes nearly empty, and all
+// tiles are stored alike (gs_tiles.h), so that they take, and stage, the largest object's
+// slots times their number.  us a step of 10 iterations with an object each, with colour
+// launches, and packed: 3,000 cells 111, 66, 38; 20,000 cells 573, 98, 61; 2,000 cubes of
+// 3^3 495, 507, 268; 10,000 cells and a cube of 8^3 516, 450, 211 (3.0 GB, packed 0.1).
+// cinst: instance of each cluster, then its tile.
+void pack_instances(const xpbd_handle* h, int units, int most, std::vector<int32_t>& cinst)
 {
-    const int64_t nv = h->nv;
-    if (h->ninst <= units || h->ninst * largest <= 4 * nv) return;
+    if (h->ninst <= units) return;
     const int nc = h->ncolors;
-    const int64_t room = std::min(largest, (nv + units - 1) / units);
-    std::vector<int32_t> count((size_t)h->ninst * nc, 0), held(nc, 0), tile(h->ninst);
+    std::vector<int64_t> load((size_t)h->ninst * (nc + 1), 0), limit(nc + 1, most);
+    limit[nc] = (h->nv + units - 1) / units;
+    for (int i = 0; i < h->ninst; i++) load[(size_t)i * (nc + 1) + nc] = h->v_off[i + 1] - h->v_off[i];
     for (int c = 0; c < nc; c++)
-        for (int i = h->color_off[c]; i < h->color_off[c + 1]; i++) count[(size_t)cinst[i] * nc + c]++;
-    int64_t verts = 0;
-    int t = 0;
-    for (int i = 0; i < h->ninst; i++) {
-        const int32_t* n = &count[(size_t)i * nc];
-        const int64_t v = h->v_off[i + 1] - h->v_off[i];
-        bool fits = verts + v <= room;
-        for (int c = 0; c < nc; c++) fits = fits && held[c] + n[c] <= most;
-        if (!fits && verts > 0) {
-            t++;
-            verts = 0;
-            std::fill(held.begin(), held.end(), 0);
-        }
-        verts += v;
-        for (int c = 0; c < nc; c++) held[c] += n[c];
-        tile[i] = t;
-    }
+        for (int i = h->color_off[c]; i < h->color_off[c + 1]; i++) load[(size_t)cinst[i] * (nc + 1) + c]++;
+    const std::vector<int32_t> tile = pack_objects(h->ninst, load, limit);
     for (int32_t& i : cinst) i = tile[i];
 }
 
@@ -248,7 +235,7 @@ int make_tiles(xpbd_handle* h)
                        gs_tile_smem((int)verts + 1, GsTileShape{}) <= kGsTileLds;
     if (whole) {
         tries = { { nc, 4, 1 << 30, 1 << 20 } };
-        pack_instances(h, units, verts, whole_limit, cinst);
+        pack_instances(h, units, whole_limit, cinst);
     }
     std::vector<GsTileGroup> G;
     GsTileDeal deal{};

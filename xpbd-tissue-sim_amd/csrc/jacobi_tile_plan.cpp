@@ -7,6 +7,7 @@
 #include "capi_internal.h"
 #include "jacobi_tile_kernels.h"
 #include "jacobi_tiles.h"
+#include "pack.h"
 
 using namespace xpbd;
 
@@ -37,7 +38,7 @@ int put(xpbd_handle* h, const D** dst, const std::vector<T>& v)
     return XPBD_OK;
 }
 
-// Tiles of a plan, 0 for a tile an instance, -1 for no plan.  us a step of 10 iterations against the
+// Tiles of a plan, 0 for a tile an instance (or several, packed), -1 for no plan.  us a step of 10 iterations against the
 // patch launches:
 // - an instance a tile, all iterations in a launch, while an instance's elements are
 //   one a thread: 4^3 cells 33 against 61 (tiles of few vertices: 57), 5^3 39 against
@@ -58,6 +59,31 @@ int tile_count(const xpbd_handle* h, int units)
     return (h->nv + own - 1) / own;
 }
 
+// Where an instance is a tile: the first vertex of each tile, and the end.  Of a batch
+// of more objects than units several small ones share a tile, as many tiles as units, of
+// at most an element a thread and 2,048 vertices (their records and corrections take
+// 88 KB of LDS).  us a step of 10 iterations with an object each, with the patch
+// launches, and packed: 20,000 cells 157, 102, 63; 2,000 cubes of 2^3 (48 elements) 74,
+// 90, 49; 700 of 1..5 cells per axis (162 and 750) 76, 97, 61.  Objects that fill a wave and
+// are alike gain nothing: 600 cubes of 3^3 39, 90, 43; 2,000 of them 72, 131, 85.
+std::vector<int64_t> packed(const xpbd_handle* h, int units)
+{
+    std::vector<int64_t> load, v_off;
+    int64_t most = 0;   // elements of an object
+    for (int i = 0; i < h->ninst; i++) {
+        load.push_back(h->t_off[i + 1] - h->t_off[i]);
+        load.push_back(h->v_off[i + 1] - h->v_off[i]);
+        most = std::max(most, load[2 * (size_t)i]);
+    }
+    if (h->ninst <= units || (h->nt >= 64ll * h->ninst && h->ninst * most <= 3ll * h->nt)) return h->v_off;
+    const std::vector<int32_t> tile =
+        pack_objects(h->ninst, load, { 1024, std::min<int64_t>(2048, (h->nv + units - 1) / units) });
+    for (int i = 0; i < h->ninst; i++)
+        if (i == 0 || tile[i] != tile[i - 1]) v_off.push_back(h->v_off[i]);
+    v_off.push_back(h->nv);
+    return v_off;
+}
+
 int make_tiles(xpbd_handle* h)
 {
     JacobiTilePlan& P = h->jtiles;
@@ -72,8 +98,9 @@ int make_tiles(xpbd_handle* h)
     if (e == hipSuccess && h->nf > 0)
         e = hipMemcpy(faces.data(), h->d_faces, sizeof(int32_t) * faces.size(), hipMemcpyDeviceToHost);
     if (e != hipSuccess) return hip_err(h, e, "element table");
+    const std::vector<int64_t> v_off = parts == 0 ? packed(h, units) : h->v_off;
     const JacobiMesh M{ h->nv,        h->nt,    h->nf, tets.data(), faces.data(), jacobi_patch_size(),
-                        h->face_patch, h->v_off, h->rest };
+                        h->face_patch, v_off, h->rest };
     const int threads = h->nt < 20000 ? 1 : 8;
     JacobiTiles J;
     if (!build_jacobi_tiles(M, parts, threads, J) || jacobi_tile_smem(J.verts, J.slots) > kLds)

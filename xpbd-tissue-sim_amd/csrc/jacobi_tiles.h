@@ -17,7 +17,7 @@ struct JacobiMesh {
     const int32_t* faces;   // 4 ints a face slot: vertices, instance
     int patch_size;
     const std::vector<int32_t>& face_patch;   // per face slot; empty: contacts at the end
-    const std::vector<int64_t>& v_off;   // vertices by instance
+    const std::vector<int64_t>& v_off;   // vertices by instance (or by run of instances that are to be a tile)
     const std::vector<double>& rest;     // 3 a vertex
 };
 
