@@ -229,18 +229,27 @@ struct FwSteps {
     }
 };
 
+// A wave pays for both choices where a lane is not sure.  Faces parallel to a box's tie at
+// every step: after that many such steps the wave goes on with the plain choice alone
+// (259,200 faces inside aligned boxes: 88 -> 71 us, the plain choice in all steps 67).
+// Over a sphere ties pass with a step or two, and giving up costs more (15 -> 17 us).
+constexpr int kQuickTries = 2;
+
 // x: the vertex to start at, then the point found.  Returns the steps that took sdf_grad.
 template <bool BOX, bool QUICK>
 XPBD_HD int face_descent(const PosedSdf& P, const double* p1, const double* p2, const double* p3, double* x)
 {
     constexpr FwSteps steps{};
     const FaceDescent<BOX> D(P, p1, p2, p3);
-    int plain = 0;
+    int plain = 0, tries = kQuickTries;
     double al = steps.a[0];
 #pragma unroll 1
     for (int it = 0; it < 32; it++) {
         const double next = steps.a[it + 1];   // on its way while this step is worked out
-        int j = QUICK ? D.vertex(P, x) : -1;
+        int j = QUICK && tries > 0 ? D.vertex(P, x) : -1;
+#ifdef __HIP_DEVICE_COMPILE__
+        if (BOX && QUICK && tries > 0 && __any(j < 0)) tries--;   // of the wave: the same in every lane
+#endif
         if (j < 0) {
             double g[3];
             sdf_grad(P, x, g);
