@@ -27,3 +27,12 @@ def test_plans_do_not_grow_with_the_number_of_small_objects(case):
     uneven, even = _held(case)
     assert uneven[2] == even[2] == 1   # an object (or several) a tile
     assert uneven[0] <= 2 * max(1, uneven[3] / even[3]) * even[0], (uneven, even)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_contacts_do_not_grow_with_the_number_of_small_objects(case):
+    """A face has its records (under 200 bytes) and a place of 37 doubles and 4 int4 for a contact; the places of
+    objects are alike within a factor of four."""
+    small, count, large, units = (int(v) for v in case.split())
+    faces = 12 * (count * small ** 2 + large ** 2)
+    assert _held(case)[0][1] <= faces * (200 + 4 * (37 * 8 + 4 * 16))

@@ -504,13 +504,28 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         for (int f = 0; f < nf; f++) count[faces[4 * (size_t)f + 3]]++;
         ContactWork& W = h->contact_work;
         W.cap = std::min(compact_block(), *std::max_element(count.begin(), count.end()));
-        const size_t room = (size_t)h->ninst * W.cap, kept = h->allocs.size();
-        if (dalloc(h, &W.head, (size_t)h->ninst) || dalloc(h, &W.where, 3 * room) || dalloc(h, &W.contact, room) ||
+        size_t room = (size_t)h->ninst * W.cap, need = 0;
+        std::vector<int32_t> first(1, 0);
+        for (int32_t c : count) {
+            need += std::max(1, std::min(W.cap, c));   // an empty room is read, too, before its count is known
+            first.push_back((int32_t)need);
+        }
+        // one room's size for all spares the launch a load that all others wait for; not where
+        // many small objects would get the room of a large one (10,000 cells and a cube: 0.9 GB)
+        int32_t* off = nullptr;
+        const size_t kept = h->allocs.size();
+        const bool own_rooms = room > 4 * need;
+        if (own_rooms) room = need;
+        if ((own_rooms && (dalloc(h, &off, first.size()) ||
+                           hipMemcpy(off, first.data(), sizeof(int32_t) * first.size(), hipMemcpyHostToDevice) != hipSuccess)) ||
+            dalloc(h, &W.head, (size_t)h->ninst) || dalloc(h, &W.where, 3 * room) || dalloc(h, &W.contact, room) ||
             dalloc(h, &W.fixed, kContactDoubles * room)) {
             for (; h->allocs.size() > kept; h->allocs.pop_back()) (void)hipFree(h->allocs.back());
             W = ContactWork{};
             (void)hipGetLastError();
             h->err.clear();
+        } else {
+            W.off = off;
         }
     }
     // deterministic patch Jacobi: contact corrections per face slot, gathered per

@@ -244,10 +244,11 @@ struct ContactSlots {
 constexpr int kContactDoubles = 37;
 struct ContactWork {
     int cap = 0;               // contacts of an instance that there is room for, at most compact_block()
+    const int* off = nullptr;  // where instances' rooms differ: the first place of each, and the end
     int4* head = nullptr;      // per instance
-    int4* where = nullptr;     // 3 cap an instance
-    int4* contact = nullptr;   // cap an instance
-    double* fixed = nullptr;   // kContactDoubles * cap an instance
+    int4* where = nullptr;     // 3 a place
+    int4* contact = nullptr;   // a place
+    double* fixed = nullptr;   // kContactDoubles a place
 };
 hipError_t launch_contacts_gs(hipStream_t s, const int4* faces, const int* fci_off, int ncol, int ninst,
                               const int* cpos, const int* clist, const double* rest, float4* pos, const float4* lo,

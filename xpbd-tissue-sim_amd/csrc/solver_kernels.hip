@@ -1588,7 +1588,9 @@ __device__ __forceinline__ void contacts_gs_many(bool first, const int4* __restr
 // the counts; per vertex where its motion lies; per contact its fixed data), from
 // which the later ones (REUSE) start: two levels of loads instead of six.  A pass
 // of a tissue block 6.4 -> 4.5 us, of 48 objects with up to 60 contacts 8.8 -> 4.9.
-template <bool REUSE, int MODE>
+// OWN: instances have rooms of their own size in W, found by a load before all others
+// (10,001 objects, a step of 10 passes: 1,113 -> 1,134 us).
+template <bool REUSE, int MODE, bool OWN>
 __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* __restrict__ faces,
                                                        const int* __restrict__ fci_off, int ncol, int ninst,
                                                        const int* __restrict__ cpos, const int* __restrict__ clist,
@@ -1605,14 +1607,19 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* 
     __shared__ int vert[REUSE ? 1 : 3 * kBlock], nverts;
     float4* const md = motion_array<MODE>(pos, dsep, slots);
     const int tid = threadIdx.x, inst = blockIdx.x;
-    const size_t at = (size_t)inst * W.cap;
+    size_t at = (size_t)inst * W.cap;
+    int cap = W.cap;
+    if constexpr (OWN) {
+        at = W.off[inst];
+        cap = W.off[inst + 1] - W.off[inst];
+    }
     int n = -1, nv = 0, ranks = 0, j = 0, rank = -1, l[3] = { 0, 0, 0 };
     double lam = 0.0;
     FixedContact F;
     int4 where[3];   // of vertices tid, tid + kBlock, tid + 2 kBlock: first place, further slots, their count, one of them
     if constexpr (REUSE) {
         // on the chance that they count, together with the counts
-        const int own = min(tid, W.cap - 1);
+        const int own = min(tid, cap - 1);
         int4 h = W.head[inst], x = W.contact[at + own];
         where[0] = W.where[3 * at + own];
         asm volatile("" : "+v"(h.x), "+v"(h.y), "+v"(h.z), "+v"(x.x), "+v"(x.y), "+v"(x.z), "+v"(x.w));
@@ -1623,7 +1630,7 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* 
         if (n > 0) {
 #pragma unroll
             for (int i = 0; i < 3; i++)
-                if (tid + i * kBlock < nv && (i > 0 || tid >= W.cap)) where[i] = W.where[3 * at + tid + i * kBlock];
+                if (tid + i * kBlock < nv && (i > 0 || tid >= cap)) where[i] = W.where[3 * at + tid + i * kBlock];
             if (tid < n) {
                 j = x.x;
                 rank = x.y;
@@ -1632,7 +1639,7 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* 
                 l[2] = x.w;
                 double* q = reinterpret_cast<double*>(&F);
 #pragma unroll
-                for (int i = 0; i < kContactDoubles; i++) q[i] = W.fixed[(size_t)kContactDoubles * at + (size_t)i * W.cap + tid];
+                for (int i = 0; i < kContactDoubles; i++) q[i] = W.fixed[(size_t)kContactDoubles * at + (size_t)i * cap + tid];
                 lam = clam[j];
             }
         }
@@ -1655,7 +1662,7 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* 
                 ws[kBlock + b.x + (k - r.x)] = b.y;
             }
         }
-        if (n == 0 && tid == 0 && W.cap) W.head[inst] = make_int4(0, 0, 0, 0);
+        if (n == 0 && tid == 0 && cap) W.head[inst] = make_int4(0, 0, 0, 0);
         if (n == 0) return;
         __syncthreads();
         if (n > 0) {
@@ -1693,20 +1700,20 @@ __global__ __launch_bounds__(kBlock) void k_contacts_gs(bool first, const int4* 
                 if (u >= nv) continue;
                 const MotionPlace p = motion_place<MODE>(slots, vert[u]);
                 where[i] = make_int4(p.first, p.more, p.end - p.more, p.end > p.more ? slots.slot[p.more] : 0);
-                if (W.cap) W.where[3 * at + u] = where[i];
+                if (cap) W.where[3 * at + u] = where[i];
             }
-            if (W.cap && n <= W.cap) {
+            if (cap && n <= cap) {
                 if (tid < n) {
                     W.contact[at + tid] = make_int4(j, rank, l[0] | l[1] << 16, l[2]);
                     const double* q = reinterpret_cast<const double*>(&F);
 #pragma unroll
                     for (int i = 0; i < kContactDoubles; i++)
-                        W.fixed[(size_t)kContactDoubles * at + (size_t)i * W.cap + tid] = q[i];
+                        W.fixed[(size_t)kContactDoubles * at + (size_t)i * cap + tid] = q[i];
                 }
             }
         }
     }
-    if (!REUSE && tid == 0 && W.cap) W.head[inst] = make_int4(n, nv, ranks, 0);
+    if (!REUSE && tid == 0 && cap) W.head[inst] = make_int4(n, nv, ranks, 0);
     if (n < 0) {
         contacts_gs_many<MODE>(first, faces, fci_off, ncol, ninst, cpos, clist, rest, pos, dsep, dbase, lo, cp, cn, cb,
                                clam, slots, ws, loc);
@@ -2726,7 +2733,7 @@ hipError_t launch_contacts_gs(hipStream_t s, const int4* faces, const int* fci_o
     const ContactWork w = work ? *work : ContactWork{};
     if (reuse && (first || w.cap <= 0)) return hipErrorInvalidValue;
 #define XPBD_CONTACTS_LAUNCH(R, M)                                                                                    \
-    hipLaunchKernelGGL((k_contacts_gs<R, M>), dim3(ninst), dim3(kBlock), 0, s, first, faces, fci_off, ncol, ninst, cpos, \
+    hipLaunchKernelGGL((w.off ? k_contacts_gs<R, M, true> : k_contacts_gs<R, M, false>), dim3(ninst), dim3(kBlock), 0, s, first, faces, fci_off, ncol, ninst, cpos, \
                        clist, rest, pos, dsep, dbase, lo, cp, cn, cb, clam, sl, w)
     const int mode = slots ? kMotionSlots : dsep && dbase ? kMotionSplit : kMotionRecords;
     switch (2 * mode + (reuse ? 1 : 0)) {
