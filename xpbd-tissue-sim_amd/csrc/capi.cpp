@@ -893,8 +893,8 @@ struct StepEnds {
 
 static bool runs_tiled(const xpbd_handle* h, int iters)
 {
-    return h->variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block == kQuadTile && h->natt == 0 && iters > 0 &&
-           !h->tiles.launches.empty();
+    return h->variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block == kQuadTile && h->natt == 0 &&
+           !h->tiles.launches.empty() && iters >= h->tiles.least;
 }
 
 static bool runs_fused_jacobi(const xpbd_handle* h)

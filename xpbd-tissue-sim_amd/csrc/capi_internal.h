@@ -38,6 +38,7 @@ struct JacobiTilePlan {
 struct GsTilePlan {
     bool built = false;      // tried; launches is empty where no plan fits
     bool closed = false;     // one launch without copies: its tiles can run all iterations
+    int least = 1;           // iterations of a solve from which these launches are the faster ones
     GsTileShape shape;
     std::vector<GsTileLaunch> launches;
     int nslots = 0;                      // of all launches

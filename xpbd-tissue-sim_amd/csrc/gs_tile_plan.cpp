@@ -260,6 +260,11 @@ int make_tiles(xpbd_handle* h)
     }
     if (G.empty()) return XPBD_OK;
     P.closed = G.size() == 1 && G[0].closed;
+    // A solve first brings the bases into their slots.  With one iteration that is most of
+    // what large one-lane plans gain (us a step, tiles and colour launches: tp = 140, 66^3, 111
+    // and 121; 146, 300 cubes of 10^3, 119 and 123; 161, 700 objects, 139 and 122; 182, 72^3, 144
+    // and 126; 250, 80^3, 165 and 151; with two iterations 239 and 232 at 72^3, 262 and 280 at 80^3).
+    P.least = P.shape.lanes == 1 && tp > 150 ? 2 : 1;
     std::vector<int32_t> off, copy;
     for (size_t g = G.size(); g-- > 0;) {
         gs_tile_copies(h->nv, G[(g + 1) % G.size()], off, copy);
