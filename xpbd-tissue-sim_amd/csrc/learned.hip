@@ -739,7 +739,7 @@ struct xpbd_mlp {
     bool has_scaling = false;
     int64_t adam_t = 0;
     // rows of a call (rows = capacity)
-    int cap = 0, cap_train = 0;
+    int cap = 0, cap_out = 0, cap_train = 0;
     float *d_X = nullptr, *d_T = nullptr;
     int* d_perm = nullptr;
     float4* d_out = nullptr;
@@ -770,7 +770,7 @@ void release(P*&... p)
 void free_ws(xpbd_mlp* m)
 {
     release(m->d_X, m->d_T, m->d_perm, m->d_out);
-    m->cap = m->cap_train = 0;
+    m->cap = m->cap_out = m->cap_train = 0;
 }
 
 template <typename T>
@@ -779,27 +779,48 @@ hipError_t room(T** p, size_t n)
     return hipMalloc(reinterpret_cast<void**>(p), n * sizeof(T));
 }
 
-// rows of inputs and outputs; train: of targets and of a permutation, too
+// rows of inputs, and of outputs or (train) of targets and of a permutation
 hipError_t ensure_ws(xpbd_mlp* m, int rows, bool train)
 {
     const size_t r = (size_t)rows;
+    int& cap = train ? m->cap_train : m->cap_out;
+    if (rows <= m->cap && rows <= cap) return hipSuccess;
+    (void)hipStreamSynchronize(m->stream);
     hipError_t e = hipSuccess;
-    if (rows > m->cap || (train && rows > m->cap_train)) {
-        (void)hipStreamSynchronize(m->stream);
-        const bool keep_train = train || m->cap_train > 0;
-        free_ws(m);
+    if (rows > m->cap) {
+        release(m->d_X);
         e = room(&m->d_X, r * kIn);
-        if (e == hipSuccess) e = room(&m->d_out, r);
-        if (e == hipSuccess && keep_train) e = room(&m->d_T, r * kOut);
-        if (e == hipSuccess && keep_train) e = room(&m->d_perm, r);
-        if (e != hipSuccess) {
-            free_ws(m);
-            return e;
-        }
         m->cap = rows;
-        m->cap_train = keep_train ? rows : 0;
     }
+    if (rows > cap) {
+        if (train) {
+            release(m->d_T, m->d_perm);
+            if (e == hipSuccess) e = room(&m->d_T, r * kOut);
+            if (e == hipSuccess) e = room(&m->d_perm, r);
+        } else {
+            release(m->d_out);
+            if (e == hipSuccess) e = room(&m->d_out, r);
+        }
+        cap = rows;
+    }
+    if (e != hipSuccess) free_ws(m);
     return e;
+}
+
+// Rows of training that a network keeps room for between calls, 112 bytes each.  One epoch
+// over more takes far longer than allocating them again.
+constexpr int kKeepRows = 1 << 20;
+
+void trim_ws(xpbd_mlp* m)
+{
+    if (m->cap_train <= kKeepRows) return;
+    release(m->d_T, m->d_perm);
+    m->cap_train = 0;
+    if (m->cap > m->cap_out) {
+        release(m->d_X);
+        m->cap = m->cap_out = 0;
+        release(m->d_out);
+    }
 }
 
 constexpr size_t kPart2 = (size_t)kRuns2 * kH * kH, kPart13 = (size_t)kMaxRuns * (kH * kIn + kOut * kH);
@@ -1204,6 +1225,7 @@ extern "C" int xpbd_mlp_train(xpbd_mlp* m, int32_t n, const float* x, const floa
     if (e == hipSuccess) e = pack(m);
     if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     (void)hipStreamSynchronize(m->stream);
+    trim_ws(m);
     if (final_loss) *final_loss = last;
     return e == hipSuccess ? XPBD_OK : merr(m, XPBD_E_HIP, hipGetErrorString(e));
 }
