@@ -146,7 +146,7 @@ def traffic_for(workload, solver, launch):
     for ent in tj.get("by_launch_config", []):
         if list(ent["launch_config"]) == list(launch):
             return ent["bytes_per_iteration"], tj.get("kernel"), None
-    return None, tj.get("kernel"), f"no counter profile recorded for launch config {list(launch)}"
+    return None, None, f"no counter profile recorded for launch config {list(launch)}"
 
 
 def measure(s, cfg, workload, steps, warmup, timing_steps, no_graph=False, tune_cache=None, variant="auto"):
