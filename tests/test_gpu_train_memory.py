@@ -1,10 +1,10 @@
 """Device memory that a network holds after training: no more than the room of a million
 rows (112 bytes each) beyond a minibatch's, and what it held for its inference calls."""
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
-import torch
 
 import xpbd_amd as X
 
@@ -15,13 +15,14 @@ KEEP = (1 << 20) * 112
 
 def _free(at_least=0):
     """Free device memory, some seconds later at most where memory that was freed is on its way back."""
+    free, total = C.c_size_t(), C.c_size_t()
     for _ in range(50):
-        torch.cuda.synchronize()
-        free = torch.cuda.mem_get_info()[0]
-        if free >= at_least:
+        # from the runtime that the library runs on
+        assert X.lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        if free.value >= at_least:
             break
         time.sleep(0.1)
-    return free
+    return free.value
 
 
 def test_training_gives_large_inputs_back():
