@@ -730,12 +730,12 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
     }
     // untuned default of Gauss-Seidel: fused-colour launches where a plan fits
     if (P->variant == XPBD_VARIANT_AUTO && cluster) {
-        if (ensure_gs_tiles(h) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
+        if (ensure_gs_tiles(h, &cverts_solver) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
         h->err.clear();
     }
     // and of Jacobi: vertex-tile launches
     if (P->variant == XPBD_VARIANT_AUTO && h->variant == XPBD_VARIANT_PATCH) {
-        h->patch_tile = ensure_jacobi_tiles(h) == XPBD_OK && h->jtiles.ready;
+        h->patch_tile = ensure_jacobi_tiles(h, reinterpret_cast<const int32_t*>(hf.data())) == XPBD_OK && h->jtiles.ready;
         h->err.clear();
     }
     *out = h;

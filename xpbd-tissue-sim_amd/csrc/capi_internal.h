@@ -218,8 +218,10 @@ int run_steps(xpbd_handle* h, int32_t nsteps);
 int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes);
 // The fused-colour plan of a Gauss-Seidel handle with clusters (built once;
 // not under capture).  XPBD_OK also where no plan fits the mesh.
-int ensure_gs_tiles(xpbd_handle* h);
-int ensure_jacobi_tiles(xpbd_handle* h);
+// cluster_verts: 8 a cluster, solver order, if the caller has them.
+int ensure_gs_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts = nullptr);
+// faces: 4 ints a face slot, if the caller has them.
+int ensure_jacobi_tiles(xpbd_handle* h, const int32_t* faces = nullptr);
 void timed_begin(xpbd_handle* h);
 void timed_end(xpbd_handle* h);
 int collect_timing(xpbd_handle* h);

@@ -12,84 +12,68 @@
 #include "gs_tiles.h"
 #include "host_threads.h"
 #include "pack.h"
+#include "plan_memory.h"
 
 using namespace xpbd;
 
 namespace {
 
-template <typename T>
-int put(xpbd_handle* h, const T** dst, const std::vector<T>& v)
-{
-    void* p = nullptr;
-    int rc = dalloc_bytes(h, &p, sizeof(T) * v.size());
-    if (rc) return rc;
-    if (!v.empty()) {
-        hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) return hip_err(h, e, "tile lists");
-    }
-    *dst = static_cast<const T*>(p);
-    return XPBD_OK;
-}
-
-template <typename T>
-int room(xpbd_handle* h, T** dst, size_t n)
-{
-    void* p = nullptr;
-    int rc = dalloc_bytes(h, &p, sizeof(T) * n);
-    *dst = static_cast<T*>(p);
-    return rc;
-}
-
-int upload(xpbd_handle* h, const GsTileGroup& G, const GsTileDeal& deal, const GsTileShape& shape, GsTileLaunch& L)
-{
-    const int nblocks = G.ntiles * G.waves * G.blocks;
-    const size_t rows = (size_t)G.ntiles * G.waves * G.rows, slots = (size_t)G.ntiles * G.slots;
-    const int32_t *tile = nullptr, *wave = nullptr, *list = nullptr, *out = nullptr, *row = nullptr, *clu = nullptr;
+// What a group's launch and its set-up take of the plan's memory.
+struct GroupArrays {
+    const int32_t *list = nullptr, *row = nullptr, *clu = nullptr;
+    const int2 *tile = nullptr, *wave = nullptr, *out = nullptr;
     const uint8_t* own = nullptr;
     const uint16_t* vert = nullptr;
     float4* stream = nullptr;
     float2* lam = nullptr;
     int32_t* home = nullptr;
-    int rc = put(h, &tile, G.tile);
-    if (!rc) rc = put(h, &wave, G.wave);
-    if (!rc) rc = put(h, &list, G.list);
-    if (!rc) rc = put(h, &out, G.out);
-    if (!rc) rc = put(h, &row, G.row);
-    if (!rc) rc = put(h, &clu, G.clu);
-    if (!rc) rc = put(h, &own, G.own);
-    if (!rc) rc = put(h, &vert, G.vert);
-    if (!rc && shape.lanes == 1) rc = room(h, &home, (size_t)nblocks * deal.per_block);
-    if (!rc) rc = room(h, &stream, rows * (shape.lanes == 1 ? kLaneRow : 64));
-    if (!rc) rc = room(h, &lam, rows * deal.per_block);
-    if (!rc) rc = room(h, &L.d[0], slots);
-    if (rc) return rc;
-    hipError_t e = launch_fill_zero(h->stream, lam, sizeof(float2) * rows * deal.per_block);
-    if (e == hipSuccess) e = launch_fill_zero(h->stream, L.d[0], sizeof(float4) * slots);
-    if (e != hipSuccess) return hip_err(h, e, "tile set-up");
+};
+
+void reserve(PlanMemory& M, const GsTileGroup& G, const GsTileDeal& deal, const GsTileShape& shape, GroupArrays& A,
+             GsTileLaunch& L)
+{
+    const size_t rows = (size_t)G.ntiles * G.waves * G.rows;
+    L.nslots = G.ntiles * G.slots;
+    M.put(&A.tile, G.tile);
+    M.put(&A.wave, G.wave);
+    M.put(&A.list, G.list);
+    M.put(&A.out, G.out);
+    M.put(&A.row, G.row);
+    M.put(&A.clu, G.clu);
+    M.put(&A.own, G.own);
+    M.put(&A.vert, G.vert);
+    if (shape.lanes == 1) M.room(&A.home, (size_t)G.ntiles * G.waves * G.blocks * deal.per_block);
+    M.room(&A.stream, rows * (shape.lanes == 1 ? kLaneRow : 64));
+    M.zeros(&A.lam, rows * deal.per_block);
+    M.zeros(&L.d[0], (size_t)L.nslots);
+}
+
+int set_up(xpbd_handle* h, const GsTileGroup& G, const GsTileShape& shape, const GroupArrays& M, GsTileLaunch& L)
+{
     GsTileFill F{};
     F.ta = tet_arrays(h);
     F.cstart = h->d_cstart;
     F.tloc = h->d_tloc;
-    F.list = list;
-    F.row = row;
-    F.clu = clu;
-    F.own = own;
-    F.vert = vert;
-    F.stream = stream;
-    F.lam = lam;
-    F.home = home;
-    F.nblocks = nblocks;
+    F.list = M.list;
+    F.row = M.row;
+    F.clu = M.clu;
+    F.own = M.own;
+    F.vert = M.vert;
+    F.stream = M.stream;
+    F.lam = M.lam;
+    F.home = M.home;
+    F.nblocks = G.ntiles * G.waves * G.blocks;
     F.slots = G.slots;
-    e = launch_gs_tile_fill(h->stream, F, shape);
+    hipError_t e = launch_gs_tile_fill(h->stream, F, shape);
     if (e != hipSuccess) return hip_err(h, e, "gs_tile_fill launch");
     GsTileArgs& A = L.args;
-    A.tile = reinterpret_cast<const int2*>(tile);
-    A.wave = reinterpret_cast<const int2*>(wave);
-    A.list = list;
-    A.out = reinterpret_cast<const int2*>(out);
-    A.home = home;
-    A.stream = stream;
-    A.lam = lam;
+    A.tile = M.tile;
+    A.wave = M.wave;
+    A.list = M.list;
+    A.out = M.out;
+    A.home = M.home;
+    A.stream = M.stream;
+    A.lam = M.lam;
     A.dlam = h->d_lam;
     A.waves = G.waves;
     A.slots = G.slots;
@@ -97,9 +81,10 @@ int upload(xpbd_handle* h, const GsTileGroup& G, const GsTileDeal& deal, const G
     A.blocks = G.blocks;
     A.outs = G.outs;
     A.nt = h->nt;
-    L.nslots = (int)slots;
     L.ntiles = G.ntiles;
     L.smem = gs_tile_smem(G.slots, shape);
+    // waves that take no block help with the slots
+    L.threads = 64 * std::max(G.waves, shape.lanes == 1 ? 8 : 4);
     return XPBD_OK;
 }
 
@@ -164,30 +149,50 @@ void pack_instances(const xpbd_handle* h, int units, int most, std::vector<int32
     for (int32_t& i : cinst) i = tile[i];
 }
 
-// The groups of one try, on a thread each; false if memory ran out.
+// work(0..n - 1), on threads if the mesh is worth it (a thread pays for itself from some
+// 0.1 ms on); false if memory ran out
+template <typename Work>
+bool each_group(size_t n, int clusters, const Work& work)
+{
+    std::atomic<bool> bad{ false };
+    std::atomic<size_t> next{ 0 };
+    on_threads(clusters < 300 ? 1 : std::min<size_t>(8, n), [&] {
+        for (size_t g; (g = next++) < n;) {
+            try {
+                work(g);
+            } catch (const std::exception&) {
+                bad = true;
+            }
+        }
+    });
+    return !bad;
+}
+
+// The groups of one try; false if memory ran out.
 bool build_groups(const GsClusters& C, int nc, int m, int tp, bool whole, const GsTileDeal& deal,
                   std::vector<GsTileGroup>& G)
 {
     G.assign((nc + m - 1) / m, GsTileGroup{});
-    std::vector<char> bad(G.size(), 0);
-    auto build = [&](size_t g) {
-        try {
-            const int c0 = (int)g * m, c1 = std::min(nc, c0 + m), n = C.color_off[c1] - C.color_off[c0];
-            build_gs_tiles(C, c0, c1, whole ? 0 : (n + (c1 - c0) * tp - 1) / ((c1 - c0) * tp), deal, G[g]);
-        } catch (const std::exception&) {
-            bad[g] = 1;
-        }
-    };
-    // threads pay for themselves on meshes that take a thread some milliseconds
-    const size_t nthreads = C.color_off[nc] < 20000 ? 1 : std::min<size_t>(4, G.size());
-    std::atomic<size_t> next{ 0 };
-    on_threads(nthreads, [&] {
-        for (size_t g; (g = next++) < G.size();) build(g);
+    return each_group(G.size(), C.color_off[nc], [&](size_t g) {
+        const int c0 = (int)g * m, c1 = std::min(nc, c0 + m), n = C.color_off[c1] - C.color_off[c0];
+        build_gs_tiles(C, c0, c1, whole ? 0 : (n + (c1 - c0) * tp - 1) / ((c1 - c0) * tp), deal, G[g]);
     });
-    return std::find(bad.begin(), bad.end(), 1) == bad.end();
 }
 
-int make_tiles(xpbd_handle* h)
+// Links every group to the next; off, copy: the first group's slots by vertex.
+bool link_groups(int nv, std::vector<GsTileGroup>& G, std::vector<int32_t>& off, std::vector<int32_t>& copy)
+{
+    return each_group(G.size(), nv, [&](size_t g) {
+        std::vector<int32_t> o, c;
+        gs_tile_copies(nv, G[(g + 1) % G.size()], o, c);
+        link_gs_tiles(G[g], o, c);
+        if (g + 1 < G.size()) return;
+        off = std::move(o);
+        copy = std::move(c);
+    });
+}
+
+int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
 {
     GsTilePlan& P = h->tiles;
     if (h->params.solver != XPBD_SOLVER_GS_COLORED || h->nclusters <= 0) return XPBD_OK;
@@ -201,17 +206,28 @@ int make_tiles(xpbd_handle* h)
     std::vector<TileTry> tries;
     tile_tries(tp, tries);
     if (tries.empty()) return XPBD_OK;
-    std::vector<int32_t> cverts(8 * (size_t)ncl), cinst(ncl, 0);
-    e = hipMemcpy(cverts.data(), h->d_cverts, sizeof(int32_t) * cverts.size(), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return hip_err(h, e, "cluster table");
-    std::vector<float> centre(3 * (size_t)ncl);
+    std::vector<int32_t> read, cinst(ncl, 0);
+    if (!cluster_verts) {
+        read.resize(8 * (size_t)ncl);
+        e = hipMemcpy(read.data(), h->d_cverts, sizeof(int32_t) * read.size(), hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return hip_err(h, e, "cluster table");
+    }
+    const std::vector<int32_t>& cverts = cluster_verts ? *cluster_verts : read;
+    std::vector<float> centre(3 * (size_t)ncl), extent(6 * (size_t)ncl);
     for (int i = 0; i < ncl; i++) {
         double s[3] = { 0, 0, 0 };
         int n = 0;
+        float* x = &extent[6 * (size_t)i];
+        for (int a = 0; a < 3; a++) x[2 * a] = 1e30f, x[2 * a + 1] = -1e30f;
         for (int k = 0; k < 8; k++) {
             const int v = cverts[8 * (size_t)i + k];
             if (v < 0) continue;
-            for (int a = 0; a < 3; a++) s[a] += h->rest[3 * (size_t)v + a];
+            for (int a = 0; a < 3; a++) {
+                const double r = h->rest[3 * (size_t)v + a];
+                s[a] += r;
+                x[2 * a] = std::min(x[2 * a], (float)r);
+                x[2 * a + 1] = std::max(x[2 * a + 1], (float)r);
+            }
             n++;
         }
         for (int a = 0; a < 3; a++) centre[3 * (size_t)i + a] = (float)(s[a] / n);
@@ -228,7 +244,7 @@ int make_tiles(xpbd_handle* h)
             for (int i = h->color_off[c]; i < h->color_off[c + 1]; i++) whole_most = std::max(whole_most, ++n[cinst[i]]);
         }
     }
-    const GsClusters C{ h->nv, cverts, h->color_off, h->cl_start, cinst, centre };
+    GsClusters C{ h->nv, cverts, h->color_off, h->cl_start, cinst, centre, &extent };
     const int rows = h->cluster_max_tets <= 6 ? 6 : 8;
     const int whole_limit = nc > 16 ? 256 : 64;
     const bool whole = whole_most <= whole_limit && verts < 65535 &&
@@ -241,6 +257,8 @@ int make_tiles(xpbd_handle* h)
     GsTileDeal deal{};
     for (const TileTry& t : tries) {
         deal = t.lanes == 1 ? GsTileDeal{ 64, 8, rows, 0 } : GsTileDeal{ 16, 16, 0, 1 };
+        const int ngroups = (nc + t.colours - 1) / t.colours;
+        C.threads = ncl < 8000 ? 1 : std::max(1, 8 / ngroups);   // smaller ones are cut in less than threads take
         if (!build_groups(C, nc, t.colours, tp, whole, deal, G)) return set_err(h, XPBD_E_NOMEM, "tile plan");
         int slots = 0, blocks = 0, least = rows;
         int64_t copies = 0;
@@ -265,37 +283,29 @@ int make_tiles(xpbd_handle* h)
     // and 121; 146, 300 cubes of 10^3, 119 and 123; 161, 700 objects, 139 and 122; 182, 72^3, 144
     // and 126; 250, 80^3, 165 and 151; with two iterations 239 and 232 at 72^3, 262 and 280 at 80^3).
     P.least = P.shape.lanes == 1 && tp > 150 ? 2 : 1;
-    std::vector<int32_t> off, copy;
-    for (size_t g = G.size(); g-- > 0;) {
-        gs_tile_copies(h->nv, G[(g + 1) % G.size()], off, copy);
-        link_gs_tiles(G[g], off, copy);
-    }
-    gs_tile_copies(h->nv, G[0], off, copy);
+    std::vector<int32_t> off, copy;   // of the first group
+    if (!link_groups(h->nv, G, off, copy)) return set_err(h, XPBD_E_NOMEM, "tile plan");
     std::vector<GsTileLaunch> launches(G.size());
+    std::vector<GroupArrays> arrays(G.size());
     std::vector<int32_t> sv;
+    PlanMemory M;
     for (size_t g = 0; g < G.size(); g++) {
-        GsTileLaunch& L = launches[g];
-        int rc = upload(h, G[g], deal, P.shape, L);
-        if (rc) return rc;
-        // waves that take no block help with the slots
-        L.threads = 64 * std::max(G[g].waves, P.shape.lanes == 1 ? 8 : 4);
+        reserve(M, G[g], deal, P.shape, arrays[g], launches[g]);
         sv.insert(sv.end(), G[g].slot_vert.begin(), G[g].slot_vert.end());
     }
     P.nslots = (int)sv.size();
-    int rc = put(h, &P.slot_vert, sv);
-    if (!rc) rc = room(h, &P.base, sv.size());
-    for (size_t g = 0, at = 0; g < G.size() && !rc; at += launches[g].nslots, g++) launches[g].args.base = P.base + at;
-    if (!rc) rc = put(h, &P.owner, G[0].owner);
-    if (!rc) rc = put(h, &P.copy_off, off);
-    if (!rc) rc = put(h, &P.copy, copy);
-    if (!rc && !P.closed) rc = room(h, &P.kept, (size_t)h->nt);
+    M.put(&P.slot_vert, sv);
+    M.put(&P.owner, G[0].owner);
+    M.put(&P.copy_off, off);
+    M.put(&P.copy, copy);
+    M.room(&P.base, sv.size());
+    if (!P.closed) M.room(&P.kept, (size_t)h->nt);
     // one group that is not closed reads and writes its own slots: two arrays in turn
-    if (!rc && G.size() == 1 && !P.closed) {
-        rc = room(h, &launches[0].d[1], (size_t)launches[0].nslots);
-        if (!rc) {
-            e = launch_fill_zero(h->stream, launches[0].d[1], sizeof(float4) * (size_t)launches[0].nslots);
-            if (e != hipSuccess) rc = hip_err(h, e, "tile set-up");
-        }
+    if (G.size() == 1 && !P.closed) M.zeros(&launches[0].d[1], (size_t)launches[0].nslots);
+    int rc = M.place(h);
+    for (size_t g = 0, at = 0; g < G.size() && !rc; at += launches[g].nslots, g++) {
+        rc = set_up(h, G[g], P.shape, arrays[g], launches[g]);
+        launches[g].args.base = P.base + at;
     }
     if (rc) return rc;
     e = gs_tile_prepare(P.shape);
@@ -307,13 +317,13 @@ int make_tiles(xpbd_handle* h)
 
 }  // namespace
 
-int xpbd::ensure_gs_tiles(xpbd_handle* h)
+int xpbd::ensure_gs_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
 {
     if (h->tiles.built) return XPBD_OK;
     const size_t kept = h->allocs.size();
     int rc;
     try {
-        rc = make_tiles(h);
+        rc = make_tiles(h, cluster_verts);
     } catch (const std::exception&) {   // host memory: a text that needs none
         rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }

@@ -1,7 +1,13 @@
 #include "gs_tiles.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cstddef>
+#include <cstring>
+#include <exception>
+#include <new>
+
+#include "host_threads.h"
 
 namespace xpbd {
 
@@ -9,86 +15,157 @@ namespace {
 
 constexpr int kV = 8;  // vertices of a cluster
 
+// Whole numbers in the order of finite floats: positions and numbers compare as one.
+uint64_t ordered(float x)
+{
+    x += 0.f;   // one zero
+    uint32_t u;
+    std::memcpy(&u, &x, sizeof u);
+    return u & 0x80000000u ? ~u : u | 0x80000000u;
+}
+
 // Cuts items[b, e) into `parts` parts of about equal size; tile numbers from
 // first on.  Instances are cut apart first; within one, the cut goes across the
 // axis that leaves the fewest vertices on both sides.
 struct Bisect {
-    const std::vector<int32_t>& cverts;
-    const std::vector<int32_t>& cinst;
-    const std::vector<float>& centre;
+    struct Part {
+        int b, e, parts, first;
+    };
+    const GsClusters& C;
     std::vector<int32_t>& items;
     std::vector<int32_t>& tile;   // per item's cluster - base
-    std::vector<int32_t> mark;    // per vertex: stamp of the last lower side that touched it
-    int base, stamp = 0;
+    const int base;
+    std::vector<int32_t> mark = std::vector<int32_t>(C.nv, 0);   // per vertex: stamp of the last lower side that touched it
+    int stamp = 0;
+    std::vector<uint64_t> key{};
 
-    int cut_size(int b, int mid, int e)
+    // A vertex on both sides lies no higher than the lower side reaches and no lower
+    // than the upper side does: clusters that end before that are passed over.
+    int cut_size(int axis, int b, int mid, int e)
     {
+        float low = 1e30f, high = -1e30f;   // lowest of the upper side, highest of the lower
+        const float* ext = C.extent ? C.extent->data() + 2 * axis : nullptr;
+        if (ext) {
+            for (int i = b; i < mid; i++) high = std::max(high, ext[6 * (size_t)items[i] + 1]);
+            for (int i = mid; i < e; i++) low = std::min(low, ext[6 * (size_t)items[i]]);
+        }
         stamp++;
-        for (int i = b; i < mid; i++)
+        for (int i = b; i < mid; i++) {
+            if (ext && ext[6 * (size_t)items[i] + 1] < low) continue;
             for (int k = 0; k < kV; k++) {
-                const int v = cverts[(size_t)kV * items[i] + k];
+                const int v = C.cverts[(size_t)kV * items[i] + k];
                 if (v >= 0) mark[v] = stamp;
             }
+        }
         int n = 0;
-        for (int i = mid; i < e; i++)
+        for (int i = mid; i < e; i++) {
+            if (ext && ext[6 * (size_t)items[i]] > high) continue;
             for (int k = 0; k < kV; k++) {
-                const int v = cverts[(size_t)kV * items[i] + k];
+                const int v = C.cverts[(size_t)kV * items[i] + k];
                 if (v >= 0) n += mark[v] == stamp;
             }
+        }
         return n;
     }
 
+    // items[b, e) with the lower ones along the axis in [b, mid), by position and number
     void along(int axis, int b, int mid, int e)
     {
-        std::nth_element(items.begin() + b, items.begin() + mid, items.begin() + e, [&](int p, int q) {
-            const float x = centre[3 * (size_t)p + axis], y = centre[3 * (size_t)q + axis];
-            return x != y ? x < y : p < q;
-        });
+        key.clear();
+        for (int i = b; i < e; i++) key.push_back(ordered(C.centre[3 * (size_t)items[i] + axis]) << 32 | (uint32_t)items[i]);
+        std::nth_element(key.begin(), key.begin() + (mid - b), key.end());
+        for (int i = b; i < e; i++) items[i] = (int32_t)(key[i - b] & 0xffffffffu);
     }
 
-    void run(int b, int e, int parts, int first)
+    // Two parts of p, or false where it is one tile, which its items then have.
+    bool split(const Part& p, Part& lo, Part& up)
     {
-        if (parts <= 1 || e - b <= 1) {
-            for (int i = b; i < e; i++) tile[items[i] - base] = first;
-            return;
+        const int b = p.b, e = p.e;
+        if (p.parts <= 1 || e - b <= 1) {
+            for (int i = b; i < e; i++) tile[items[i] - base] = p.first;
+            return false;
         }
-        const int lower = parts / 2;
-        int mid = b + (int)((int64_t)(e - b) * lower / parts);
-        auto by_instance = [&](int p, int q) { return cinst[p] != cinst[q] ? cinst[p] < cinst[q] : p < q; };
-        const auto mm = std::minmax_element(items.begin() + b, items.begin() + e,
-                                            [&](int p, int q) { return cinst[p] < cinst[q]; });
-        int lo_parts = lower;
-        if (cinst[*mm.first] != cinst[*mm.second]) {
-            std::sort(items.begin() + b, items.begin() + e, by_instance);
+        const int lower = p.parts / 2;
+        int mid = b + (int)((int64_t)(e - b) * lower / p.parts), lo_parts = lower;
+        auto inst = [&](int i) { return C.cinst[items[i]]; };
+        int32_t least = inst(b), most = least;
+        for (int i = b; i < e; i++) {
+            least = std::min(least, inst(i));
+            most = std::max(most, inst(i));
+        }
+        if (least != most) {
+            std::sort(items.begin() + b, items.begin() + e, [&](int x, int y) {
+                return C.cinst[x] != C.cinst[y] ? C.cinst[x] < C.cinst[y] : x < y;
+            });
             // the instance boundary nearest to the even cut, with parts in proportion
             int up = mid, dn = mid;
-            while (up < e && cinst[items[up]] == cinst[items[up - 1]]) up++;
-            while (dn > b && cinst[items[dn]] == cinst[items[dn - 1]]) dn--;
+            while (up < e && inst(up) == inst(up - 1)) up++;
+            while (dn > b && inst(dn) == inst(dn - 1)) dn--;
             mid = (dn > b && (up >= e || mid - dn <= up - mid)) ? dn : up;
-            lo_parts = (int)(((int64_t)parts * (mid - b) + (e - b) / 2) / (e - b));
-            lo_parts = std::min(parts - 1, std::max(1, lo_parts));
+            lo_parts = (int)(((int64_t)p.parts * (mid - b) + (e - b) / 2) / (e - b));
+            lo_parts = std::min(p.parts - 1, std::max(1, lo_parts));
         } else {
             float lo[3], hi[3];
             for (int a = 0; a < 3; a++) lo[a] = 1e30f, hi[a] = -1e30f;
             for (int i = b; i < e; i++)
                 for (int a = 0; a < 3; a++) {
-                    lo[a] = std::min(lo[a], centre[3 * (size_t)items[i] + a]);
-                    hi[a] = std::max(hi[a], centre[3 * (size_t)items[i] + a]);
+                    lo[a] = std::min(lo[a], C.centre[3 * (size_t)items[i] + a]);
+                    hi[a] = std::max(hi[a], C.centre[3 * (size_t)items[i] + a]);
                 }
             int best = 0, best_cut = INT32_MAX, last = -1;
             for (int a = 0; a < 3; a++) {
                 if (!(hi[a] > lo[a])) continue;
                 along(a, b, mid, e);
                 last = a;
-                const int c = cut_size(b, mid, e);
+                const int c = cut_size(a, b, mid, e);
                 if (c < best_cut) best_cut = c, best = a;
             }
             if (last != best) along(best, b, mid, e);
         }
-        run(b, mid, lo_parts, first);
-        run(mid, e, parts - lo_parts, first + lo_parts);
+        lo = { b, mid, lo_parts, p.first };
+        up = { mid, e, p.parts - lo_parts, p.first + lo_parts };
+        return true;
+    }
+
+    void run(const Part& p)
+    {
+        Part lo, up;
+        if (!split(p, lo, up)) return;
+        run(lo);
+        run(up);
     }
 };
+
+// All of items into parts: the first cuts one by one, what they leave on threads.
+void bisect(const GsClusters& C, std::vector<int32_t>& items, std::vector<int32_t>& tile, int base, int parts)
+{
+    Bisect B{ C, items, tile, base };
+    std::vector<Bisect::Part> left{ { 0, (int)items.size(), parts, 0 } };
+    for (size_t i = 0; C.threads > 1 && i < left.size() && left.size() < 4 * (size_t)C.threads; i++) {
+        Bisect::Part lo, up;   // breadth first: the largest parts are cut first
+        const bool more = B.split(left[i], lo, up);
+        left[i].parts = 0;   // done
+        if (!more) continue;
+        left.push_back(lo);
+        left.push_back(up);
+    }
+    left.erase(std::remove_if(left.begin(), left.end(), [](const Bisect::Part& p) { return p.parts == 0; }), left.end());
+    if (C.threads <= 1) {
+        for (const Bisect::Part& p : left) B.run(p);
+        return;
+    }
+    std::atomic<size_t> next{ 0 };
+    std::atomic<bool> bad{ false };
+    on_threads(C.threads, [&] {
+        try {
+            Bisect mine{ C, items, tile, base };
+            for (size_t i; (i = next++) < left.size();) mine.run(left[i]);
+        } catch (const std::exception&) {
+            bad = true;
+        }
+    });
+    if (bad) throw std::bad_alloc();
+}
 
 }  // namespace
 
@@ -109,8 +186,7 @@ void build_gs_tiles(const GsClusters& C, int c0, int c1, int parts, const GsTile
     if (whole) {
         for (int i = 0; i < n; i++) ctile[i] = C.cinst[base + i];
     } else {
-        Bisect B{ cverts, C.cinst, C.centre, items, ctile, std::vector<int32_t>(nv, 0), base };
-        B.run(0, n, parts, 0);
+        bisect(C, items, ctile, base, parts);
     }
     G.ntiles = parts;
     // per vertex the last cluster of the group that touches it; per cluster and

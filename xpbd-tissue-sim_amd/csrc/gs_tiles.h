@@ -65,6 +65,10 @@ struct GsClusters {
     int nv;
     const std::vector<int32_t>&cverts, &color_off, &cstart, &cinst;
     const std::vector<float>& centre;
+    // lowest and highest vertex of each cluster along x, y, z (6 a cluster): where the same
+    // plan is found sooner
+    const std::vector<float>* extent = nullptr;
+    int threads = 1;   // to cut with
 };
 // Cuts colours [c0, c1) into `parts` tiles (at most one per cluster), or with
 // parts <= 0 makes every instance (every value of cinst) a tile.

@@ -8,35 +8,13 @@
 #include "jacobi_tile_kernels.h"
 #include "jacobi_tiles.h"
 #include "pack.h"
+#include "plan_memory.h"
 
 using namespace xpbd;
 
 namespace {
 
 constexpr size_t kLds = 160 * 1024;   // of a workgroup, gfx950
-
-template <typename T>
-int room(xpbd_handle* h, T** dst, size_t n)
-{
-    void* p = nullptr;
-    int rc = dalloc_bytes(h, &p, sizeof(T) * n);
-    *dst = static_cast<T*>(p);
-    return rc;
-}
-
-template <typename D, typename T>
-int put(xpbd_handle* h, const D** dst, const std::vector<T>& v)
-{
-    char* p = nullptr;
-    int rc = room(h, &p, sizeof(T) * v.size());
-    if (rc) return rc;
-    if (!v.empty()) {
-        hipError_t e = hipMemcpy(p, v.data(), sizeof(T) * v.size(), hipMemcpyHostToDevice);
-        if (e != hipSuccess) return hip_err(h, e, "Jacobi tile lists");
-    }
-    *dst = reinterpret_cast<const D*>(p);
-    return XPBD_OK;
-}
 
 // Tiles of a plan, 0 for a tile an instance (or several, packed), -1 for no plan.  us a step of 10 iterations against the
 // patch launches:
@@ -84,7 +62,7 @@ std::vector<int64_t> packed(const xpbd_handle* h, int units)
     return v_off;
 }
 
-int make_tiles(xpbd_handle* h)
+int make_tiles(xpbd_handle* h, const int32_t* faces)
 {
     JacobiTilePlan& P = h->jtiles;
     if (h->variant != XPBD_VARIANT_PATCH || h->params.deterministic == 0 || h->nt <= 0) return XPBD_OK;
@@ -93,15 +71,19 @@ int make_tiles(xpbd_handle* h)
     if (e != hipSuccess || units <= 0) return hip_err(h, e, "device attribute");
     const int parts = tile_count(h, units);
     if (parts < 0) return XPBD_OK;
-    std::vector<int32_t> tets(4 * (size_t)h->nt), faces(4 * (size_t)h->nf);
-    e = hipMemcpy(tets.data(), h->d_tet, sizeof(int32_t) * tets.size(), hipMemcpyDeviceToHost);
-    if (e == hipSuccess && h->nf > 0)
-        e = hipMemcpy(faces.data(), h->d_faces, sizeof(int32_t) * faces.size(), hipMemcpyDeviceToHost);
-    if (e != hipSuccess) return hip_err(h, e, "element table");
+    std::vector<int32_t> tets, read;
+    tets.reserve(4 * (size_t)h->nt);
+    for (int32_t t : h->order) tets.insert(tets.end(), &h->tets_host[4 * (size_t)t], &h->tets_host[4 * (size_t)t] + 4);
+    if (!faces && h->nf > 0) {
+        read.resize(4 * (size_t)h->nf);
+        e = hipMemcpy(read.data(), h->d_faces, sizeof(int32_t) * read.size(), hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return hip_err(h, e, "element table");
+        faces = read.data();
+    }
     const std::vector<int64_t> v_off = parts == 0 ? packed(h, units) : h->v_off;
-    const JacobiMesh M{ h->nv,        h->nt,    h->nf, tets.data(), faces.data(), jacobi_patch_size(),
+    const JacobiMesh M{ h->nv,        h->nt,    h->nf, tets.data(), faces, jacobi_patch_size(),
                         h->face_patch, v_off, h->rest };
-    const int threads = h->nt < 20000 ? 1 : 8;
+    const int threads = h->nt < 2000 ? 1 : h->nt < 8000 ? 4 : 8;   // a thread pays for itself from some 0.1 ms on
     JacobiTiles J;
     if (!build_jacobi_tiles(M, parts, threads, J) || jacobi_tile_smem(J.verts, J.slots) > kLds)
         return XPBD_OK;
@@ -109,24 +91,24 @@ int make_tiles(xpbd_handle* h)
     const size_t n = J.home.size(), slots = J.vert.size();
     float4* stream = nullptr;
     float4* base = nullptr;
-    int rc = put(h, &A.head, J.head);
-    if (!rc) rc = put(h, &A.local, J.local);
-    if (!rc) rc = put(h, &A.home, J.home);
-    if (!rc) rc = put(h, &A.face, J.face);
-    if (!rc) rc = put(h, &A.group, J.group);
-    if (!rc) rc = put(h, &A.sums, J.sums);
-    if (!rc) rc = put(h, &A.out, J.out);
-    if (!rc) rc = put(h, &A.vert, J.vert);
-    if (!rc) rc = put(h, &P.owner, J.owner);
-    if (!rc) rc = room(h, &stream, 3 * n);
-    if (!rc) rc = room(h, &A.lam, n);
-    if (!rc) rc = room(h, &base, slots);
-    for (int i = 0; i < 2 && !rc; i++) rc = room(h, &P.d[i], slots);
-    if (!rc && !J.closed) rc = room(h, &P.kept, (size_t)h->nt);
+    PlanMemory memory;
+    memory.put(&A.head, J.head);
+    memory.put(&A.local, J.local);
+    memory.put(&A.home, J.home);
+    memory.put(&A.face, J.face);
+    memory.put(&A.group, J.group);
+    memory.put(&A.sums, J.sums);
+    memory.put(&A.out, J.out);
+    memory.put(&A.vert, J.vert);
+    memory.put(&P.owner, J.owner);
+    memory.room(&stream, 3 * n);
+    memory.zeros(&A.lam, n);
+    memory.room(&base, slots);
+    for (float4*& d : P.d) memory.zeros(&d, slots);
+    if (!J.closed) memory.room(&P.kept, (size_t)h->nt);
+    int rc = memory.place(h);
     if (rc) return rc;
-    e = launch_fill_zero(h->stream, A.lam, sizeof(float2) * n);
-    for (int i = 0; i < 2 && e == hipSuccess; i++) e = launch_fill_zero(h->stream, P.d[i], sizeof(float4) * slots);
-    if (e == hipSuccess) e = launch_jacobi_tile_fill(h->stream, tet_arrays(h), A.home, (int)n, stream);
+    e = launch_jacobi_tile_fill(h->stream, tet_arrays(h), A.home, (int)n, stream);
     if (e == hipSuccess) e = jacobi_tile_prepare();
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_err(h, e, "Jacobi tile set-up");
@@ -156,13 +138,13 @@ int make_tiles(xpbd_handle* h)
 
 }  // namespace
 
-int xpbd::ensure_jacobi_tiles(xpbd_handle* h)
+int xpbd::ensure_jacobi_tiles(xpbd_handle* h, const int32_t* faces)
 {
     if (h->jtiles.built) return XPBD_OK;
     const size_t kept = h->allocs.size();
     int rc;
     try {
-        rc = make_tiles(h);
+        rc = make_tiles(h, faces);
     } catch (const std::exception&) {   // host memory: a text that needs none
         rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }

@@ -4,6 +4,7 @@
 #include <atomic>
 #include <cstddef>
 #include <exception>
+#include <utility>
 
 #include "host_threads.h"
 
@@ -18,6 +19,7 @@ struct Cut {
     std::vector<int32_t>& items;
     std::vector<int32_t>& tile;
     const std::vector<int32_t>& inst;
+    std::vector<std::pair<double, int32_t>> key{};
 
     void run(int b, int e, int parts, int first)
     {
@@ -46,10 +48,10 @@ struct Cut {
             int axis = 0;
             for (int a = 1; a < 3; a++)
                 if (hi[a] - lo[a] > hi[axis] - lo[axis]) axis = a;
-            std::nth_element(items.begin() + b, items.begin() + mid, items.begin() + e, [&](int p, int q) {
-                const double x = M.rest[3 * (size_t)p + axis], y = M.rest[3 * (size_t)q + axis];
-                return x != y ? x < y : p < q;
-            });
+            key.clear();   // by position and number
+            for (int i = b; i < e; i++) key.emplace_back(M.rest[3 * (size_t)items[i] + axis], items[i]);
+            std::nth_element(key.begin(), key.begin() + (mid - b), key.end());
+            for (int i = b; i < e; i++) items[i] = key[i - b].second;
         }
         run(b, mid, lower, first);
         run(mid, e, parts - lower, first + lower);
