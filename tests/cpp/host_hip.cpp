@@ -13,6 +13,7 @@
 namespace host_hip {
 int units = 256;
 bool no_pinned = false;
+int64_t mallocs_left = INT64_MAX;
 int64_t device_bytes = 0, mallocs = 0;
 }  // namespace host_hip
 
@@ -41,7 +42,7 @@ hipError_t hipGetLastError(void)
 
 hipError_t hipMalloc(void** p, size_t n)
 {
-    if (!(*p = std::malloc(n ? n : 1))) return done(hipErrorOutOfMemory);
+    if (host_hip::mallocs_left-- <= 0 || !(*p = std::malloc(n ? n : 1))) return done(hipErrorOutOfMemory);
     std::memset(*p, 0xa5, n);   // what was never written is no zero
     sizes[*p] = n;
     host_hip::device_bytes += (int64_t)n;

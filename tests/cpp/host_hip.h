@@ -10,6 +10,7 @@ namespace host_hip {
 
 extern int units;              // compute units of the device
 extern bool no_pinned;         // hipHostMalloc fails
+extern int64_t mallocs_left;   // device allocations until one fails, and all after it
 extern int64_t device_bytes;   // allocated now
 extern int64_t mallocs;        // device allocations so far
 

@@ -26,6 +26,12 @@ void* operator new(size_t n)
     if (void* p = std::malloc(n ? n : 1)) return p;
     throw std::bad_alloc();
 }
+void* operator new(size_t n, const std::nothrow_t&) noexcept
+{
+    if (left.fetch_sub(1) > 0) return std::malloc(n ? n : 1);
+    refused++;
+    return nullptr;
+}
 void operator delete(void* p) noexcept { std::free(p); }
 void operator delete(void* p, size_t) noexcept { std::free(p); }
 

@@ -64,6 +64,12 @@ int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes)
     return rc;
 }
 
+int device_units(xpbd_handle* h, int* units)
+{
+    hipError_t e = hipDeviceGetAttribute(units, hipDeviceAttributeMultiprocessorCount, h->device);
+    return e == hipSuccess && *units > 0 ? XPBD_OK : hip_err(h, e, "device attribute");
+}
+
 static void release_graphs(xpbd_handle* h)
 {
     for (int i = 0; i < 2; i++) {
@@ -428,11 +434,14 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         }
     }
 
+    // the tile plans' host work goes on beside the allocations and copies that follow
+    if (P->variant == XPBD_VARIANT_AUTO && cluster) begin_gs_tiles(h, cverts_solver);
+
     // ---- device buffers
     hipError_t he = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
     if (he != hipSuccess) {
         int rc = hip_err(nullptr, he, "hipStreamCreate");
-        delete h;
+        xpbd_destroy(h);
         return rc;
     }
     int rc = 0;
@@ -652,6 +661,8 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
         h->patch_fused = ok && Pt.npatch <= kFusedDefaultMaxPatches;
         if (h->patch_fused) h->face_patch = fpatch;
     }
+    if (P->variant == XPBD_VARIANT_AUTO && h->variant == XPBD_VARIANT_PATCH)
+        begin_jacobi_tiles(h, reinterpret_cast<const int32_t*>(hf.data()));
     h->sdf_host.assign(n, SdfDev{});
     for (auto& s : h->sdf_host) s.quat[3] = 1.0;
 #define UP(dst, src, bytes)                                                      \
@@ -730,12 +741,12 @@ static int build(int32_t n, const xpbd_mesh_desc* meshes, const xpbd_params* P, 
     }
     // untuned default of Gauss-Seidel: fused-colour launches where a plan fits
     if (P->variant == XPBD_VARIANT_AUTO && cluster) {
-        if (ensure_gs_tiles(h, &cverts_solver) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
+        if (ensure_gs_tiles(h) == XPBD_OK && !h->tiles.launches.empty()) h->quad_block = kQuadTile;
         h->err.clear();
     }
     // and of Jacobi: vertex-tile launches
     if (P->variant == XPBD_VARIANT_AUTO && h->variant == XPBD_VARIANT_PATCH) {
-        h->patch_tile = ensure_jacobi_tiles(h, reinterpret_cast<const int32_t*>(hf.data())) == XPBD_OK && h->jtiles.ready;
+        h->patch_tile = ensure_jacobi_tiles(h) == XPBD_OK && h->jtiles.ready;
         h->err.clear();
     }
     *out = h;
@@ -756,6 +767,8 @@ extern "C" int xpbd_batch_create(int32_t n, const xpbd_mesh_desc* meshes, const 
 extern "C" int xpbd_destroy(xpbd_handle* h)
 {
     if (!h) return XPBD_OK;
+    h->gs_begun.reset();   // ends their threads, which read this handle
+    h->jacobi_begun.reset();
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     release_graphs(h);
     for (auto& ev : h->events) {

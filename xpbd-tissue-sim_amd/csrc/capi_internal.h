@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -16,6 +17,8 @@
 
 namespace xpbd {
 struct Learned;
+struct GsPlanHost;
+struct JacobiPlanHost;
 
 // The fused-colour launches of one Gauss-Seidel iteration (gs_tiles.h).
 struct GsTileLaunch {
@@ -77,6 +80,8 @@ struct xpbd_handle {
     std::vector<int32_t> cl_start;             // cluster variant: tet range of each cluster (solver order)
     int nclusters = 0;
     xpbd::GsTilePlan tiles;                    // cluster variants: fused-colour launches
+    std::shared_ptr<xpbd::GsPlanHost> gs_begun;           // begin_gs_tiles: its thread reads this handle
+    std::shared_ptr<xpbd::JacobiPlanHost> jacobi_begun;
     xpbd::Patches patches;                     // patch variant (host copy)
     std::vector<int32_t> fperm;                // solver face position -> caller's face index
     std::vector<int32_t> fcol_off;
@@ -216,12 +221,17 @@ int enqueue_contacts_jacobi(xpbd_handle* h, bool first);
 bool detect_this_step(const xpbd_handle* h);
 int run_steps(xpbd_handle* h, int32_t nsteps);
 int dalloc_bytes(xpbd_handle* h, void** p, size_t bytes);
+int device_units(xpbd_handle* h, int* units);   // compute units
 // The fused-colour plan of a Gauss-Seidel handle with clusters (built once;
 // not under capture).  XPBD_OK also where no plan fits the mesh.
-// cluster_verts: 8 a cluster, solver order, if the caller has them.
-int ensure_gs_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts = nullptr);
-// faces: 4 ints a face slot, if the caller has them.
-int ensure_jacobi_tiles(xpbd_handle* h, const int32_t* faces = nullptr);
+int ensure_gs_tiles(xpbd_handle* h);
+// Begins the host's part of it on a thread, while a handle is being created; its lists
+// of vertices, elements, clusters and colours have to stay as they are.  cluster_verts: 8
+// a cluster, solver order.
+void begin_gs_tiles(xpbd_handle* h, const std::vector<int32_t>& cluster_verts);
+int ensure_jacobi_tiles(xpbd_handle* h);
+// faces: 4 ints a face slot.
+void begin_jacobi_tiles(xpbd_handle* h, const int32_t* faces);
 void timed_begin(xpbd_handle* h);
 void timed_end(xpbd_handle* h);
 int collect_timing(xpbd_handle* h);

@@ -5,6 +5,8 @@
 #include <algorithm>
 #include <atomic>
 #include <exception>
+#include <memory>
+#include <thread>
 #include <utility>
 
 #include "capi_internal.h"
@@ -149,14 +151,15 @@ void pack_instances(const xpbd_handle* h, int units, int most, std::vector<int32
     for (int32_t& i : cinst) i = tile[i];
 }
 
-// work(0..n - 1), on threads if the mesh is worth it (a thread pays for itself from some
-// 0.1 ms on); false if memory ran out
+constexpr int kThreadClusters = 300;   // a thread pays for itself from some 0.1 ms on
+
+// work(0..n - 1), on threads if the mesh is worth it; false if memory ran out
 template <typename Work>
 bool each_group(size_t n, int clusters, const Work& work)
 {
     std::atomic<bool> bad{ false };
     std::atomic<size_t> next{ 0 };
-    on_threads(clusters < 300 ? 1 : std::min<size_t>(8, n), [&] {
+    on_threads(clusters < kThreadClusters ? 1 : std::min<size_t>(8, n), [&] {
         for (size_t g; (g = next++) < n;) {
             try {
                 work(g);
@@ -192,27 +195,39 @@ bool link_groups(int nv, std::vector<GsTileGroup>& G, std::vector<int32_t>& off,
     });
 }
 
-int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
-{
-    GsTilePlan& P = h->tiles;
-    if (h->params.solver != XPBD_SOLVER_GS_COLORED || h->nclusters <= 0) return XPBD_OK;
-    const int ncl = h->nclusters, nc = h->ncolors;
+}  // namespace
+
+// What a plan is on the host: all of it that takes no device memory.
+struct xpbd::GsPlanHost {
     int units = 0;
-    hipError_t e = hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, h->device);
-    if (e != hipSuccess || units <= 0) return hip_err(h, e, "device attribute");
+    std::vector<int32_t> cverts;
+    int rc = XPBD_OK;
+    std::vector<GsTileGroup> G;   // empty where no plan fits
+    GsTileDeal deal{};
+    GsTileShape shape;
+    bool closed = false;
+    int least = 1;
+    std::vector<int32_t> off, copy, slot_vert;   // off, copy: the first group's slots by vertex
+    std::thread worker;
+    ~GsPlanHost()
+    {
+        if (worker.joinable()) worker.join();
+    }
+};
+
+namespace {
+
+int plan_host(const xpbd_handle* h, GsPlanHost& H)
+{
+    const int units = H.units, ncl = h->nclusters, nc = h->ncolors;
+    const std::vector<int32_t>& cverts = H.cverts;
     int most = 0, whole_most = 0;   // clusters of a colour; of a colour and instance
     for (int c = 0; c < nc; c++) most = std::max(most, h->color_off[c + 1] - h->color_off[c]);
     const int tp = std::max(8, (most + units - 1) / units);
     std::vector<TileTry> tries;
     tile_tries(tp, tries);
     if (tries.empty()) return XPBD_OK;
-    std::vector<int32_t> read, cinst(ncl, 0);
-    if (!cluster_verts) {
-        read.resize(8 * (size_t)ncl);
-        e = hipMemcpy(read.data(), h->d_cverts, sizeof(int32_t) * read.size(), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return hip_err(h, e, "cluster table");
-    }
-    const std::vector<int32_t>& cverts = cluster_verts ? *cluster_verts : read;
+    std::vector<int32_t> cinst(ncl, 0);
     std::vector<float> centre(3 * (size_t)ncl), extent(6 * (size_t)ncl);
     for (int i = 0; i < ncl; i++) {
         double s[3] = { 0, 0, 0 };
@@ -253,13 +268,13 @@ int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
         tries = { { nc, 4, 1 << 30, 1 << 20 } };
         pack_instances(h, units, whole_limit, cinst);
     }
-    std::vector<GsTileGroup> G;
-    GsTileDeal deal{};
+    std::vector<GsTileGroup>& G = H.G;
+    GsTileDeal& deal = H.deal;
     for (const TileTry& t : tries) {
         deal = t.lanes == 1 ? GsTileDeal{ 64, 8, rows, 0 } : GsTileDeal{ 16, 16, 0, 1 };
         const int ngroups = (nc + t.colours - 1) / t.colours;
         C.threads = ncl < 8000 ? 1 : std::max(1, 8 / ngroups);   // smaller ones are cut in less than threads take
-        if (!build_groups(C, nc, t.colours, tp, whole, deal, G)) return set_err(h, XPBD_E_NOMEM, "tile plan");
+        if (!build_groups(C, nc, t.colours, tp, whole, deal, G)) return XPBD_E_NOMEM;
         int slots = 0, blocks = 0, least = rows;
         int64_t copies = 0;
         for (const GsTileGroup& g : G) {
@@ -268,37 +283,67 @@ int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
             least = std::min(least, g.min_rows);
             copies += g.copies;
         }
-        P.shape.lanes = t.lanes;
-        P.shape.rows = rows;
-        P.shape.full = least == 6;
-        P.shape.cap = t.lanes == 1 ? gs_tile_cap(slots) : 0;
-        const bool fits = slots <= 65535 && (t.lanes == 4 || P.shape.cap > 0) && gs_tile_smem(slots, P.shape) <= kGsTileLds;
+        H.shape.lanes = t.lanes;
+        H.shape.rows = rows;
+        H.shape.full = least == 6;
+        H.shape.cap = t.lanes == 1 ? gs_tile_cap(slots) : 0;
+        const bool fits = slots <= 65535 && (t.lanes == 4 || H.shape.cap > 0) && gs_tile_smem(slots, H.shape) <= kGsTileLds;
         if (fits && blocks <= t.most_blocks && 10 * copies <= (int64_t)t.copies_tenths * ncl) break;
         G.clear();
     }
     if (G.empty()) return XPBD_OK;
-    P.closed = G.size() == 1 && G[0].closed;
+    H.closed = G.size() == 1 && G[0].closed;
     // A solve first brings the bases into their slots.  With one iteration that is most of
     // what large one-lane plans gain (us a step, tiles and colour launches: tp = 140, 66^3, 111
     // and 121; 146, 300 cubes of 10^3, 119 and 123; 161, 700 objects, 139 and 122; 182, 72^3, 144
     // and 126; 250, 80^3, 165 and 151; with two iterations 239 and 232 at 72^3, 262 and 280 at 80^3).
-    P.least = P.shape.lanes == 1 && tp > 150 ? 2 : 1;
-    std::vector<int32_t> off, copy;   // of the first group
-    if (!link_groups(h->nv, G, off, copy)) return set_err(h, XPBD_E_NOMEM, "tile plan");
+    H.least = H.shape.lanes == 1 && tp > 150 ? 2 : 1;
+    if (!link_groups(h->nv, G, H.off, H.copy)) return XPBD_E_NOMEM;
+    for (const GsTileGroup& g : G) H.slot_vert.insert(H.slot_vert.end(), g.slot_vert.begin(), g.slot_vert.end());
+    return XPBD_OK;
+}
+
+int plan_host_checked(const xpbd_handle* h, GsPlanHost& H)
+{
+    try {
+        return plan_host(h, H);
+    } catch (const std::exception&) {
+        return XPBD_E_NOMEM;
+    }
+}
+
+int make_tiles(xpbd_handle* h)
+{
+    GsTilePlan& P = h->tiles;
+    if (h->params.solver != XPBD_SOLVER_GS_COLORED || h->nclusters <= 0) return XPBD_OK;
+    std::shared_ptr<GsPlanHost> H = std::move(h->gs_begun);
+    if (H) {
+        H->worker.join();
+    } else {
+        H = std::make_shared<GsPlanHost>();
+        int rc = device_units(h, &H->units);
+        if (rc) return rc;
+        H->cverts.resize(8 * (size_t)h->nclusters);
+        hipError_t e = hipMemcpy(H->cverts.data(), h->d_cverts, sizeof(int32_t) * H->cverts.size(), hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return hip_err(h, e, "cluster table");
+        H->rc = plan_host_checked(h, *H);
+    }
+    if (H->rc) return set_err(h, H->rc, "tile plan");
+    const std::vector<GsTileGroup>& G = H->G;
+    if (G.empty()) return XPBD_OK;
+    P.shape = H->shape;
+    P.closed = H->closed;
+    P.least = H->least;
     std::vector<GsTileLaunch> launches(G.size());
     std::vector<GroupArrays> arrays(G.size());
-    std::vector<int32_t> sv;
     PlanMemory M;
-    for (size_t g = 0; g < G.size(); g++) {
-        reserve(M, G[g], deal, P.shape, arrays[g], launches[g]);
-        sv.insert(sv.end(), G[g].slot_vert.begin(), G[g].slot_vert.end());
-    }
-    P.nslots = (int)sv.size();
-    M.put(&P.slot_vert, sv);
+    for (size_t g = 0; g < G.size(); g++) reserve(M, G[g], H->deal, P.shape, arrays[g], launches[g]);
+    P.nslots = (int)H->slot_vert.size();
+    M.put(&P.slot_vert, H->slot_vert);
     M.put(&P.owner, G[0].owner);
-    M.put(&P.copy_off, off);
-    M.put(&P.copy, copy);
-    M.room(&P.base, sv.size());
+    M.put(&P.copy_off, H->off);
+    M.put(&P.copy, H->copy);
+    M.room(&P.base, H->slot_vert.size());
     if (!P.closed) M.room(&P.kept, (size_t)h->nt);
     // one group that is not closed reads and writes its own slots: two arrays in turn
     if (G.size() == 1 && !P.closed) M.zeros(&launches[0].d[1], (size_t)launches[0].nslots);
@@ -308,7 +353,7 @@ int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
         launches[g].args.base = P.base + at;
     }
     if (rc) return rc;
-    e = gs_tile_prepare(P.shape);
+    hipError_t e = gs_tile_prepare(P.shape);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_err(h, e, "gs_tile set-up");
     P.launches = std::move(launches);
@@ -317,13 +362,26 @@ int make_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
 
 }  // namespace
 
-int xpbd::ensure_gs_tiles(xpbd_handle* h, const std::vector<int32_t>* cluster_verts)
+void xpbd::begin_gs_tiles(xpbd_handle* h, const std::vector<int32_t>& cluster_verts)
+{
+    if (h->nclusters < kThreadClusters) return;
+    try {
+        auto H = std::make_shared<GsPlanHost>();
+        H->cverts = cluster_verts;
+        if (device_units(h, &H->units)) return;
+        H->worker = std::thread([h, p = H.get()] { p->rc = plan_host_checked(h, *p); });
+        h->gs_begun = std::move(H);
+    } catch (const std::exception&) {   // no thread, or no memory for one: planned when it is due
+    }
+}
+
+int xpbd::ensure_gs_tiles(xpbd_handle* h)
 {
     if (h->tiles.built) return XPBD_OK;
     const size_t kept = h->allocs.size();
     int rc;
     try {
-        rc = make_tiles(h, cluster_verts);
+        rc = make_tiles(h);
     } catch (const std::exception&) {   // host memory: a text that needs none
         rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }

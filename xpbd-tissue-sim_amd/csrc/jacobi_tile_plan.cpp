@@ -3,6 +3,8 @@
 
 #include <algorithm>
 #include <exception>
+#include <memory>
+#include <thread>
 
 #include "capi_internal.h"
 #include "jacobi_tile_kernels.h"
@@ -15,6 +17,7 @@ using namespace xpbd;
 namespace {
 
 constexpr size_t kLds = 160 * 1024;   // of a workgroup, gfx950
+constexpr int kThreadElements = 2000;   // a thread pays for itself from some 0.1 ms on
 
 // Tiles of a plan, 0 for a tile an instance (or several, packed), -1 for no plan.  us a step of 10 iterations against the
 // patch launches:
@@ -62,31 +65,71 @@ std::vector<int64_t> packed(const xpbd_handle* h, int units)
     return v_off;
 }
 
-int make_tiles(xpbd_handle* h, const int32_t* faces)
+}  // namespace
+
+// What a plan is on the host.
+struct xpbd::JacobiPlanHost {
+    int units = 0;
+    std::vector<int32_t> faces;
+    int rc = XPBD_OK;
+    bool fits = false;
+    JacobiTiles J;
+    std::thread worker;
+    ~JacobiPlanHost()
+    {
+        if (worker.joinable()) worker.join();
+    }
+};
+
+namespace {
+
+int plan_host(const xpbd_handle* h, JacobiPlanHost& H)
+{
+    try {
+        const int parts = tile_count(h, H.units);
+        if (parts < 0) return XPBD_OK;
+        std::vector<int32_t> tets;
+        tets.reserve(4 * (size_t)h->nt);
+        for (int32_t t : h->order) {
+            const int32_t* v = h->tets_host.data() + 4 * (size_t)t;
+            tets.insert(tets.end(), v, v + 4);
+        }
+        const std::vector<int64_t> v_off = parts == 0 ? packed(h, H.units) : h->v_off;
+        const JacobiMesh M{ h->nv, h->nt, h->nf, tets.data(), H.faces.data(), jacobi_patch_size(), h->face_patch, v_off, h->rest };
+        const int threads = h->nt < kThreadElements ? 1 : h->nt < 8000 ? 4 : 8;
+        H.fits = build_jacobi_tiles(M, parts, threads, H.J) && jacobi_tile_smem(H.J.verts, H.J.slots) <= kLds;
+        return XPBD_OK;
+    } catch (const std::exception&) {
+        return XPBD_E_NOMEM;
+    }
+}
+
+bool plannable(const xpbd_handle* h)
+{
+    return h->variant == XPBD_VARIANT_PATCH && h->params.deterministic != 0 && h->nt > 0;
+}
+
+int make_tiles(xpbd_handle* h)
 {
     JacobiTilePlan& P = h->jtiles;
-    if (h->variant != XPBD_VARIANT_PATCH || h->params.deterministic == 0 || h->nt <= 0) return XPBD_OK;
-    int units = 0;
-    hipError_t e = hipDeviceGetAttribute(&units, hipDeviceAttributeMultiprocessorCount, h->device);
-    if (e != hipSuccess || units <= 0) return hip_err(h, e, "device attribute");
-    const int parts = tile_count(h, units);
-    if (parts < 0) return XPBD_OK;
-    std::vector<int32_t> tets, read;
-    tets.reserve(4 * (size_t)h->nt);
-    for (int32_t t : h->order) tets.insert(tets.end(), &h->tets_host[4 * (size_t)t], &h->tets_host[4 * (size_t)t] + 4);
-    if (!faces && h->nf > 0) {
-        read.resize(4 * (size_t)h->nf);
-        e = hipMemcpy(read.data(), h->d_faces, sizeof(int32_t) * read.size(), hipMemcpyDeviceToHost);
-        if (e != hipSuccess) return hip_err(h, e, "element table");
-        faces = read.data();
+    if (!plannable(h)) return XPBD_OK;
+    std::shared_ptr<JacobiPlanHost> H = std::move(h->jacobi_begun);
+    if (H) {
+        H->worker.join();
+    } else {
+        H = std::make_shared<JacobiPlanHost>();
+        int rc = device_units(h, &H->units);
+        if (rc) return rc;
+        H->faces.resize(4 * (size_t)h->nf);
+        if (h->nf > 0) {
+            hipError_t e = hipMemcpy(H->faces.data(), h->d_faces, sizeof(int32_t) * H->faces.size(), hipMemcpyDeviceToHost);
+            if (e != hipSuccess) return hip_err(h, e, "face table");
+        }
+        H->rc = plan_host(h, *H);
     }
-    const std::vector<int64_t> v_off = parts == 0 ? packed(h, units) : h->v_off;
-    const JacobiMesh M{ h->nv,        h->nt,    h->nf, tets.data(), faces, jacobi_patch_size(),
-                        h->face_patch, v_off, h->rest };
-    const int threads = h->nt < 2000 ? 1 : h->nt < 8000 ? 4 : 8;   // a thread pays for itself from some 0.1 ms on
-    JacobiTiles J;
-    if (!build_jacobi_tiles(M, parts, threads, J) || jacobi_tile_smem(J.verts, J.slots) > kLds)
-        return XPBD_OK;
+    if (H->rc) return set_err(h, H->rc, "tile plan");
+    if (!H->fits) return XPBD_OK;
+    const JacobiTiles& J = H->J;
     JacobiTileArgs A{};
     const size_t n = J.home.size(), slots = J.vert.size();
     float4* stream = nullptr;
@@ -108,7 +151,7 @@ int make_tiles(xpbd_handle* h, const int32_t* faces)
     if (!J.closed) memory.room(&P.kept, (size_t)h->nt);
     int rc = memory.place(h);
     if (rc) return rc;
-    e = launch_jacobi_tile_fill(h->stream, tet_arrays(h), A.home, (int)n, stream);
+    hipError_t e = launch_jacobi_tile_fill(h->stream, tet_arrays(h), A.home, (int)n, stream);
     if (e == hipSuccess) e = jacobi_tile_prepare();
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return hip_err(h, e, "Jacobi tile set-up");
@@ -138,13 +181,26 @@ int make_tiles(xpbd_handle* h, const int32_t* faces)
 
 }  // namespace
 
-int xpbd::ensure_jacobi_tiles(xpbd_handle* h, const int32_t* faces)
+void xpbd::begin_jacobi_tiles(xpbd_handle* h, const int32_t* faces)
+{
+    if (!plannable(h) || h->nt < kThreadElements) return;
+    try {
+        auto H = std::make_shared<JacobiPlanHost>();
+        H->faces.assign(faces, faces + 4 * (size_t)h->nf);
+        if (device_units(h, &H->units)) return;
+        H->worker = std::thread([h, p = H.get()] { p->rc = plan_host(h, *p); });
+        h->jacobi_begun = std::move(H);
+    } catch (const std::exception&) {   // no thread, or no memory for one: planned when it is due
+    }
+}
+
+int xpbd::ensure_jacobi_tiles(xpbd_handle* h)
 {
     if (h->jtiles.built) return XPBD_OK;
     const size_t kept = h->allocs.size();
     int rc;
     try {
-        rc = make_tiles(h, faces);
+        rc = make_tiles(h);
     } catch (const std::exception&) {   // host memory: a text that needs none
         rc = set_err(h, XPBD_E_NOMEM, "tile plan");
     }
