@@ -324,7 +324,8 @@ int xpbd_batch_step(xpbd_batch* b, int32_t nsteps);
  * workgroup mapping) as replays of a captured graph of the handle's
  * iterations, restore the state, and keep the fastest.  The choice is
  * appended to cache_path (may be NULL) as
- * "shape-key variant block xcd ms-per-iteration" and reused from there for the
+ * "shape-key variant block xcd ms-per-iteration" (after XPBD_QUAD_TILE also the
+ * quad block of solves that it does not run) and reused from there for the
  * same shape.  No reference counterpart: the reference has no kernel variants. */
 int xpbd_autotune(xpbd_batch* b, const char* cache_path);
 /* The kernel variant in use (XPBD_VARIANT_*); block: for CLUSTER_QUAD the
@@ -345,8 +346,9 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
 /* The quad block value of the fused-colour launches, the untuned default where
  * the mesh's size suits them: several consecutive colours share one launch, in
  * which a workgroup runs them on a spatial tile of the mesh (same element order,
- * the same results).  Handles with attachments run the 256-thread quad shape
- * instead. */
+ * the same results).  Handles with attachments, and solves of one iteration on
+ * meshes of millions of elements, run a quad shape instead: with 256 threads, or
+ * the fastest that an autotune found. */
 #define XPBD_QUAD_TILE 4000
 /* The patch block value of the vertex-tile Jacobi launches, the untuned default
  * where the mesh's size suits them: a workgroup owns a set of vertices and

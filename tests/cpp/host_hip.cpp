@@ -108,7 +108,11 @@ size_t jacobi_fused_smem(int maxl, bool con)
     return jacobi_patch_smem(maxl, true) + (con ? (size_t)maxl * 12 + (size_t)256 * 40 : 0);
 }
 bool quad_split(int block) { return (block < 0 ? -block : block) > kQuadSplit; }
-bool quad_block_supported(int) { return true; }
+bool quad_block_supported(int block)
+{
+    const int b = (block < 0 ? -block : block) - (quad_split(block) ? kQuadSplit : 0);
+    return b == 64 || b == 128 || b == 256;
+}
 hipError_t launch_fill_zero(hipStream_t, void* p, size_t bytes) { return std::memset(p, 0, bytes), hipSuccess; }
 
 }  // namespace xpbd

@@ -32,6 +32,7 @@ struct Candidate {
     int variant;
     int block;
     int xcd;
+    int plain = 256;   // with the fused-colour launches: the quad shape of solves that they do not run
 };
 
 std::string shape_key(const xpbd_handle* h)
@@ -51,9 +52,11 @@ bool read_cache(const char* path, const std::string& key, Candidate* out)
     while (std::getline(f, line)) {
         std::istringstream is(line);
         std::string k;
-        int v = 0, b = 0, x = 0;
+        int v = 0, b = 0, x = 0, plain = 0;
+        double ms = 0;
         if (is >> k >> v >> b >> x && k == key) {
             *out = { v, b, x };
+            if (is >> ms >> plain) out->plain = plain;
             found = true;  // the last entry for a key wins
         }
     }
@@ -64,13 +67,16 @@ void write_cache(const char* path, const std::string& key, const Candidate& c, d
 {
     if (!path) return;
     std::ofstream f(path, std::ios::app);
-    f << key << " " << c.variant << " " << c.block << " " << c.xcd << " " << ms_per_iter << "\n";
+    f << key << " " << c.variant << " " << c.block << " " << c.xcd << " " << ms_per_iter;
+    if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile) f << " " << c.plain;
+    f << "\n";
 }
 
 bool valid(const xpbd_handle* h, const Candidate& c)
 {
     if (c.variant == XPBD_VARIANT_CLUSTER) return h->nclusters > 0;
-    if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile) return !h->tiles.launches.empty();
+    if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile)
+        return !h->tiles.launches.empty() && quad_block_supported(c.plain) && !quad_split(c.plain);
     if (c.variant == XPBD_VARIANT_CLUSTER_QUAD) return h->nclusters > 0 && quad_block_supported(c.block);
     if (c.variant == XPBD_VARIANT_PATCH) return h->variant == XPBD_VARIANT_PATCH &&
                (c.block == XPBD_PATCH_TILE ? h->jtiles.ready : c.block == 0 || h->fused_ok);
@@ -79,6 +85,10 @@ bool valid(const xpbd_handle* h, const Candidate& c)
 
 void apply(xpbd_handle* h, const Candidate& c)
 {
+    if (c.variant == XPBD_VARIANT_CLUSTER_QUAD && c.block == kQuadTile && h->quad_plain != c.plain) {
+        h->quad_plain = c.plain;
+        invalidate_graphs(h);
+    }
     if (h->variant != c.variant || (c.variant == XPBD_VARIANT_CLUSTER_QUAD && h->quad_block != c.block) ||
         (c.variant == XPBD_VARIANT_PATCH &&
          (h->patch_fused != (c.block == 1) || h->patch_tile != (c.block == XPBD_PATCH_TILE))) || h->xcd_map != (c.xcd != 0)) {
@@ -153,7 +163,8 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     int rc = e == hipSuccess ? XPBD_OK : hip_err(h, e, "autotune set-up");
     const int saved_variant = h->variant, saved_block = h->quad_block;
     const bool saved_xcd = h->xcd_map, saved_fused = h->patch_fused, saved_tile = h->patch_tile;
-    double best_ms = 1e300;
+    double best_ms = 1e300, plain_ms = 1e300;
+    int plain = 256;   // fastest of the shapes that run with attachments, too, on the tiles' workgroup mapping
     Candidate best = cand[0];
     const int iters = h->params.iters > 0 ? h->params.iters : 1;
     for (const Candidate& cd : cand) {
@@ -210,6 +221,11 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
             best_ms = ms_best;
             best = cd;
         }
+        if (!rc && cd.variant == XPBD_VARIANT_CLUSTER_QUAD && cd.block != kQuadTile && !quad_split(cd.block) && cd.xcd &&
+            ms_best < plain_ms) {
+            plain_ms = ms_best;
+            plain = cd.block;
+        }
     }
     if (e0) (void)hipEventDestroy(e0);
     if (e1) (void)hipEventDestroy(e1);
@@ -222,6 +238,7 @@ extern "C" int xpbd_autotune(xpbd_batch* h, const char* cache_path)
     h->patch_fused = saved_fused;
     h->patch_tile = saved_tile;
     if (rc) return rc;
+    best.plain = plain;
     apply(h, best);
     write_cache(cache_path, key, best, best_ms / iters);
     return XPBD_OK;

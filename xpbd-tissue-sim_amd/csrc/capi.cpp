@@ -1122,7 +1122,7 @@ static int enqueue_iterations(xpbd_handle* h, int iters, bool timed, bool reset_
     // which the loop only reads, are copied into one (the attachment pass reads
     // the records, so handles with attachments stay interleaved).
     if (runs_tiled(h, iters)) return enqueue_tiled_iterations(h, iters, timed, reset_lambda, ends);
-    const int quad_block = h->quad_block == kQuadTile ? 256 : h->quad_block;
+    const int quad_block = h->quad_block == kQuadTile ? h->quad_plain : h->quad_block;
     float4* dsep = h->params.solver == XPBD_SOLVER_GS_COLORED && h->variant == XPBD_VARIANT_CLUSTER_QUAD &&
                            quad_split(quad_block) && h->natt == 0 && iters > 0
                        ? h->d_dsep
