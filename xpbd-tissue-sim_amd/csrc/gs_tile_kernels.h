@@ -31,8 +31,6 @@ struct GsTileArgs {
                              // One lane a cluster, kLaneRow per row: see k_gs_tile_lane
     float2* lam;             // 16 (64) per row; with four lanes a block's first row: as home
     float2* dlam;            // solver order
-    const float2* kept;      // solver order, what an import reads: not dlam where this launch writes that and tiles
-                             // share clusters
     const float4* din;       // in-step motion, by slot of this group
     float4* dout;            // by slot of the next
     const float4* base;      // base displacement, inverse mass, by slot
@@ -40,6 +38,9 @@ struct GsTileArgs {
     int niter, nt;
     int lam_zero;            // the first iteration's multipliers are zero
     int lam_out;             // the last iteration also writes dlam
+    const float2* kept;      // solver order, what an import reads: not dlam where this launch writes that and tiles
+                             // share clusters.  Last: between the others it moved the kernel's loads of them, beam
+                             // 200x20x20 474 -> 477 us a step
 };
 
 struct GsTileFill {

@@ -18,8 +18,6 @@ struct JacobiTileArgs {
     const int2* out;
     float2* lam;              // per tile element
     float2* dlam;             // solver order
-    const float2* kept;       // solver order, what an import reads: not dlam where this launch writes that and tiles
-                              // share elements
     const float4* din;        // in-step motion by slot
     float4* dout;
     const float4* base;       // base displacement, inverse mass by slot
@@ -36,6 +34,8 @@ struct JacobiTileArgs {
     const double *rest, *cp, *cn, *cb;
     const float4* lo;
     double* clam;
+    const float2* kept;       // solver order, what an import reads: not dlam where this launch writes that and tiles
+                              // share elements
 };
 
 size_t jacobi_tile_smem(int verts, int slots);
