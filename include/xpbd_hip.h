@@ -354,7 +354,8 @@ int xpbd_get_variant(xpbd_handle* h, int32_t* variant, int32_t* block, int32_t* 
  * where the mesh's size suits them: a workgroup owns a set of vertices and
  * projects every element around them, so that one launch is an iteration and a
  * vertex's corrections are summed in one place (in the groups of the other patch
- * launches: the same results).  Deterministic mode without attachments; otherwise
+ * launches: the same results; with contacts those of the one, fused or not, that
+ * the untuned handle would run in its place).  Deterministic mode without attachments; otherwise
  * such a handle runs the other patch launches. */
 #define XPBD_PATCH_TILE 2
 /* Batch handles are also plain handles: xpbd_step, xpbd_destroy, ... apply. */

@@ -118,8 +118,9 @@ struct TileTry {
 // has a wave for each SIMD and no more (56^3 611, 2 colours 649; 66^3 805 and 739).
 // Two launches' phases hold up to 8 blocks of 64 clusters, a wave each.  Where they
 // fit they win (72^3 990, colour launches 1,085; 80^3 1,044 and 1,312; 96^3, tp = 432,
-// 1,562 and 2,156).  Where a tile's phases or vertices do not fit (88^3), and above
-// tp = 512, there is no plan.
+// 1,562 and 2,156).  Where a tile's phases or vertices do not fit (86^3 to 94^3, from
+// 98^3 on), and above tp = 512, there is no plan.  All of this is from boxes of one
+// object.
 void tile_tries(int tp, std::vector<TileTry>& t)
 {
     if (tp <= 11) t.push_back({ 4, 4, 16, 32 });
